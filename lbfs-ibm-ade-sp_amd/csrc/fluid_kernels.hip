@@ -124,6 +124,31 @@ struct TileGrad {
 // ---------------------------------------------------------------------------
 // face reconstruction and flux
 // ---------------------------------------------------------------------------
+// states and gradients extrapolated to an interior face from both sides, and
+// their mean
+template <class G>
+__device__ __forceinline__ void interior_sides(const float4 &d1, const float4 &d2, const float sov[4], const float4 sn,
+                                               const float go[12], float gn[12], const G &gsrc, int tf, int nb,
+                                               float po[4], float pn[4], float p0[4])
+{
+    gsrc.load_nbr(tf, nb, gn);
+    const float snv[4] = {sn.x, sn.y, sn.z, sn.w};
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        po[v] = sov[v] - (d1.x * go[3 * v] + d1.y * go[3 * v + 1] + d1.z * go[3 * v + 2]);
+        pn[v] = snv[v] - (d2.x * gn[3 * v] + d2.y * gn[3 * v + 1] + d2.z * gn[3 * v + 2]);
+        p0[v] = 0.5f * (po[v] + pn[v]);
+    }
+}
+
+// equilibrium deviation of the rest point, which takes the mean state
+template <class L>
+__device__ __forceinline__ float rest_point(const float p0[4], float rho0, float ig)
+{
+    const float uu = p0[1] * p0[1] + p0[2] * p0[2] + p0[3] * p0[3];
+    return L::w(0) * (p0[0] + (rho0 + p0[0]) * (-1.5f * uu * ig));
+}
+
 template <class L, bool BAND, class G>
 __device__ __forceinline__ float4 face_flux(const FluidArgs &a, const float4 *__restrict__ st, const G &gsrc, int tf)
 {
@@ -131,78 +156,73 @@ __device__ __forceinline__ float4 face_flux(const FluidArgs &a, const float4 *__
     const FaceRec fr = load_face(a, tf);
     const float4 fb = fr.d1, fcv = fr.d2;
     const int o = fr.o, nb = fr.nb;
-    const bool ghost = nb >= a.n_cells;
     const float nx = fr.nx, ny = fr.ny, nz = fr.nz, A = fr.A, dt = fr.dt;
+    const float rho0 = a.rho0, ig = a.inv_gamma;
     const float4 so = st[o];
     float go[12], gn[12];
     gsrc.load_owner(tf, o, go);
     const float sov[4] = {so.x, so.y, so.z, so.w};
     float po[4], pn[4], p0[4];
-    if (!ghost) {
-        const float4 sn = st[nb];
-        gsrc.load_nbr(tf, nb, gn);
-        const float snv[4] = {sn.x, sn.y, sn.z, sn.w};
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            po[v] = sov[v] - (fb.x * go[3 * v] + fb.y * go[3 * v + 1] + fb.z * go[3 * v + 2]);
-            pn[v] = snv[v] - (fcv.x * gn[3 * v] + fcv.y * gn[3 * v + 1] + fcv.z * gn[3 * v + 2]);
-            p0[v] = 0.5f * (po[v] + pn[v]);
-        }
-    } else {
-        // ghost gradient (gradients.cpp:393-505 / LBFS.cu:1933-2048) and face
-        // value from the boundary condition (Solver.cpp:855-900)
-        const int bc = nb - a.n_cells;
-        const int2 ty = a.bc_type[bc];
-        if (ty.y == LBFS_BC_EMPTY) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // Solver.cpp:308-310
-        const float4 bv = a.bc_val[bc];
-        const float bvv[4] = {bv.x, bv.y, bv.z, bv.w};
-        const float d1n = sqrtf(fb.x * fb.x + fb.y * fb.y + fb.z * fb.z);
-        const float inv_dmag = 2.0f / d1n;  // ghost centroid sits halfway to the face
-        float dir[3];
-        if (a.flags & LBFS_FLAG_GHOST_DIR_GPU) { dir[0] = -fb.x / d1n; dir[1] = -fb.y / d1n; dir[2] = -fb.z / d1n; }
-        else { dir[0] = nx; dir[1] = ny; dir[2] = nz; }
-        const float nv[3] = {nx, ny, nz};
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int type = v == 0 ? ty.x : ty.y;
-            if (type == 1 || type == 3) {
-                const float dphi = 2.0f * (bvv[v] - sov[v]) * inv_dmag;
-#pragma unroll
-                for (int c = 0; c < 3; c++) gn[3 * v + c] = dphi * dir[c];
-                // code 3 (parabolic/shear targets) extrapolates the face value
-                // with the ghost gradient (LBFS.cu:358-378)
-                p0[v] = type == 1 ? bvv[v] : sov[v] - (fb.x * gn[3 * v] + fb.y * gn[3 * v + 1] + fb.z * gn[3 * v + 2]);
-            } else {
-#pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    const float fac = (a.flags & LBFS_FLAG_NEUMANN_SIGNED) ? 1.0f - nv[c] : 1.0f - fabsf(nv[c]);
-                    gn[3 * v + c] = go[3 * v + c] * fac;
-                }
-                p0[v] = sov[v] - (fb.x * gn[3 * v] + fb.y * gn[3 * v + 1] + fb.z * gn[3 * v + 2]);
-            }
-            po[v] = p0[v];
-            pn[v] = p0[v];
-        }
-        // the GPU reconstruction hands the ghost gradient to the owner-side
-        // points too (grad_*_1 = grad_*_2, LBFS.cu:391-394)
-        if (a.flags & LBFS_FLAG_GHOST_FACE_GRAD) {
-#pragma unroll
-            for (int t = 0; t < 12; t++) go[t] = gn[t];
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < 12; t++) { go[t] *= dt; gn[t] *= dt; }
-    const float rho0 = a.rho0, ig = a.inv_gamma;
-    const float bw = 0.001f * dt;
     FaceSums f;
     f.S1x = f.S1y = f.S1z = f.Tx = f.Ty = f.Tz = 0.0f;
-    {
-        const float uu = p0[1] * p0[1] + p0[2] * p0[2] + p0[3] * p0[3];
-        const float P = -1.5f * uu * ig;
-        f.S0 = L::w(0) * (p0[0] + (rho0 + p0[0]) * P);
+    if (!fr.general) {
+        interior_sides(fb, fcv, sov, st[nb], go, gn, gsrc, tf, nb, po, pn, p0);
+        f.S0 = rest_point<L>(p0, rho0, ig);
+        const float ig15 = 1.5f * ig;
+        all_pairs_fast<L>(std::make_integer_sequence<int, (L::Q - 1) / 2>{}, f, po, pn, go, gn, nx, ny, nz, dt,
+                          rho0 * ig15, ig15, a.two_gamma);
+    } else {
+        const bool ghost = nb >= a.n_cells;
+        if (!ghost) {
+            interior_sides(fb, fcv, sov, st[nb], go, gn, gsrc, tf, nb, po, pn, p0);
+        } else {
+            // ghost gradient (gradients.cpp:393-505 / LBFS.cu:1933-2048) and face
+            // value from the boundary condition (Solver.cpp:855-900)
+            const int bc = nb - a.n_cells;
+            const int2 ty = a.bc_type[bc];
+            if (ty.y == LBFS_BC_EMPTY) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // Solver.cpp:308-310
+            const float4 bv = a.bc_val[bc];
+            const float bvv[4] = {bv.x, bv.y, bv.z, bv.w};
+            const float d1n = sqrtf(fb.x * fb.x + fb.y * fb.y + fb.z * fb.z);
+            const float inv_dmag = 2.0f / d1n;  // ghost centroid sits halfway to the face
+            float dir[3];
+            if (a.flags & LBFS_FLAG_GHOST_DIR_GPU) { dir[0] = -fb.x / d1n; dir[1] = -fb.y / d1n; dir[2] = -fb.z / d1n; }
+            else { dir[0] = nx; dir[1] = ny; dir[2] = nz; }
+            const float nv[3] = {nx, ny, nz};
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int type = v == 0 ? ty.x : ty.y;
+                if (type == 1 || type == 3) {
+                    const float dphi = 2.0f * (bvv[v] - sov[v]) * inv_dmag;
+#pragma unroll
+                    for (int c = 0; c < 3; c++) gn[3 * v + c] = dphi * dir[c];
+                    // code 3 (parabolic/shear targets) extrapolates the face value
+                    // with the ghost gradient (LBFS.cu:358-378)
+                    p0[v] = type == 1 ? bvv[v] : sov[v] - (fb.x * gn[3 * v] + fb.y * gn[3 * v + 1] + fb.z * gn[3 * v + 2]);
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        const float fac = (a.flags & LBFS_FLAG_NEUMANN_SIGNED) ? 1.0f - nv[c] : 1.0f - fabsf(nv[c]);
+                        gn[3 * v + c] = go[3 * v + c] * fac;
+                    }
+                    p0[v] = sov[v] - (fb.x * gn[3 * v] + fb.y * gn[3 * v + 1] + fb.z * gn[3 * v + 2]);
+                }
+                po[v] = p0[v];
+                pn[v] = p0[v];
+            }
+            // the GPU reconstruction hands the ghost gradient to the owner-side
+            // points too (grad_*_1 = grad_*_2, LBFS.cu:391-394)
+            if (a.flags & LBFS_FLAG_GHOST_FACE_GRAD) {
+#pragma unroll
+                for (int t = 0; t < 12; t++) go[t] = gn[t];
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 12; t++) { go[t] *= dt; gn[t] *= dt; }
+        f.S0 = rest_point<L>(p0, rho0, ig);
+        all_pairs<L, BAND>(std::make_integer_sequence<int, (L::Q - 1) / 2>{}, f, po, pn, p0, go, gn, nx, ny, nz,
+                           0.001f * dt, ghost, rho0, ig);
     }
-    all_pairs<L, BAND>(std::make_integer_sequence<int, (L::Q - 1) / 2>{}, f, po, pn, p0, go, gn, nx, ny, nz, bw, ghost,
-                       rho0, ig);
     const float S0 = f.S0, S1x = f.S1x, S1y = f.S1y, S1z = f.S1z, Tx = f.Tx, Ty = f.Ty, Tz = f.Tz;
     if (a.face_moments) a.face_moments[tf] = make_float4(S0, S1x, S1y, S1z);
     const float rho_f = rho0 + S0;

@@ -16,7 +16,7 @@ struct FluidArgs {
     const uint32_t *face_gslot;    // per tile-face: LDS gradient slots of owner | neighbour << 16
     int block_threads;             // workgroup size of the flux/update kernel (256 or 512)
     int lattice, flags;
-    float rho0, inv_gamma, visc3_over_gamma, dt;
+    float rho0, inv_gamma, two_gamma, visc3_over_gamma, dt;
     float body_force[3];
     // per cell (internal tile order)
     const int *stencil;            // [6 n] SoA
@@ -32,7 +32,7 @@ struct FluidArgs {
     const int *tile_cell_start, *tile_face_start;
     const int *tile_bface_start;   // first boundary face of each tile's list
     // tile faces
-    const float4 *fA, *fB, *fC;    // normal * area, dt | owner offset, owner | neighbour offset, neighbour
+    const float4 *fA, *fB, *fC;    // normal * area, dt (negative: general face) | owner offset, owner | neighbour offset, neighbour
     // boundary conditions
     const int2 *bc_type;           // (rho type, vel type)
     const float4 *bc_val;          // (rho - rho0, u, v, w)

@@ -82,8 +82,8 @@ static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params
         return ctx->fail(LBFS_E_INVALID_ARG, "block_threads must be 256, 512 or 576");
     rc = mesh_blocks(m, p.body_force, ctx->blocks, err);
     if (rc) return ctx->fail(rc, "mesh blocks: %s", err.c_str());
-    rc = build_layout(m, ctx->geo, lhs, rhs, p.rho0, p.body_force, p.lattice == LBFS_D2Q9 ? 2 : 3, tile, ctx->blocks,
-                      ctx->lay, err);
+    rc = build_layout(m, ctx->geo, lhs, rhs, p.rho0, p.body_force, p.lattice, (p.flags & LBFS_FLAG_UPWIND_BAND) != 0,
+                      tile, ctx->blocks, ctx->lay, err);
     if (rc) return ctx->fail(rc, "layout: %s", err.c_str());
     const DeviceLayout &d = ctx->lay;
     const int n = d.n_cells, nbc = d.n_bc;
@@ -117,6 +117,7 @@ static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params
     a.flags = p.flags;
     a.rho0 = (float)p.rho0;
     a.inv_gamma = (float)(1.0 / p.gamma);
+    a.two_gamma = (float)(2.0 * p.gamma);
     a.visc3_over_gamma = (float)(p.visc * 3.0 / p.gamma);
     a.dt = (float)p.dt;
     for (int t = 0; t < 3; t++) a.body_force[t] = (float)p.body_force[t];

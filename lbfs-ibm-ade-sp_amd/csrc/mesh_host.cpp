@@ -2,6 +2,8 @@
 // the tile-blocked device layout.
 #include "mesh_host.hpp"
 
+#include "lattice.hpp"
+
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -378,11 +380,26 @@ const double *cell_body_force(const std::vector<HostBlock> &blocks, int c, const
     return c < h.cell0 + h.n[0] * h.n[1] * h.n[2] ? h.force : dflt;
 }
 
+// smallest |e.n| over the moving directions of the lattice
+template <class L>
+static double min_component(const double n[3])
+{
+    double v = 4.0;
+    for (int k = 1; k < L::Q; k++) v = std::min(v, std::fabs(L::ex[k] * n[0] + L::ey[k] * n[1] + L::ez[k] * n[2]));
+    return v;
+}
+static double min_direction_component(int lattice, const double n[3])
+{
+    return lattice == LBFS_D3Q15 ? min_component<D3Q15>(n)
+                                 : (lattice == LBFS_D3Q19 ? min_component<D3Q19>(n) : min_component<D2Q9>(n));
+}
+
 int build_layout(const lbfs_mesh_desc &m, const Geometry &g, const std::vector<double> &lhs,
-                 const std::vector<double> &rhs, double rho0, const double body_force[3], int dims, const int tile[3],
-                 const std::vector<HostBlock> &blocks, DeviceLayout &d, std::string &err)
+                 const std::vector<double> &rhs, double rho0, const double body_force[3], int lattice, bool band,
+                 const int tile[3], const std::vector<HostBlock> &blocks, DeviceLayout &d, std::string &err)
 {
     const int nc = g.n_cells;
+    const int dims = lattice == LBFS_D2Q9 ? 2 : 3;
     d.n_cells = nc;
     d.n_bc = g.n_bc;
     d.perm.clear();
@@ -435,11 +452,22 @@ int build_layout(const lbfs_mesh_desc &m, const Geometry &g, const std::vector<d
             }
         }
     });
-    // Tile face lists: every face touching a cell of the tile, in caller face
-    // order; and the tile's halo, the cells across its border in the order
+    // Tile face lists: every face touching a cell of the tile, by class (below)
+    // and in caller face order; and the tile's halo, the cells across its border in the order
     // its faces first reach them.  Tiles are independent: first each tile's
     // lists (on worker threads), then their offsets, then the records.
     const int nt = d.n_tiles;
+    // 0: every lattice direction clearly on one side of the face; 1: one lies
+    // within rounding of the face's plane or of the tie band around it (normals
+    // are held in float: e.n is off by at most 3 ulps of 1); 2: boundary face
+    std::vector<unsigned char> fclass(g.n_faces);
+    parallel_for(g.n_faces, [&](int f0, int f1) {
+        for (int f = f0; f < f1; f++) {
+            const double tol = 1e-6 + (band ? 0.001 * g.fdt[f] * (1.0 + 1e-6) : 0.0);
+            fclass[f] = f >= g.n_int ? 2 : (min_direction_component(lattice, &g.normal[3 * (size_t)f]) > tol ? 0 : 1);
+        }
+    });
+    auto face_class = [&](int f) { return (int)fclass[f]; };
     std::vector<std::vector<int>> tfaces(nt), thalo(nt);
     std::string terr;
     std::mutex terr_lock;
@@ -462,6 +490,8 @@ int build_layout(const lbfs_mesh_desc &m, const Geometry &g, const std::vector<d
                 visit(d.inv[g.owner[f]]);
                 if (g.nbr[f] < nc) visit(d.inv[g.nbr[f]]);
             }
+            std::stable_partition(faces.begin(), faces.end(), [&](int f) { return face_class(f) == 0; });
+            std::stable_partition(faces.begin(), faces.end(), [&](int f) { return face_class(f) < 2; });
             if ((int)faces.size() > 32767 || ntc + (int)halo.size() >= 0xffff) {
                 std::lock_guard<std::mutex> lk(terr_lock);
                 if (terr.empty())
@@ -479,9 +509,10 @@ int build_layout(const lbfs_mesh_desc &m, const Geometry &g, const std::vector<d
         const int nft = (int)tfaces[t].size(), ntc = d.tile_cell_start[t + 1] - d.tile_cell_start[t];
         d.tile_face_start[t + 1] = d.tile_face_start[t] + nft;
         d.tile_halo_start[t + 1] = d.tile_halo_start[t] + (int)thalo[t].size();
-        // caller order puts internal faces (ids < n_int) before boundary faces
+        // boundary faces (ids from n_int) come last
         d.tile_bface_start[t] = d.tile_face_start[t] +
-            (int)(std::lower_bound(tfaces[t].begin(), tfaces[t].end(), g.n_int) - tfaces[t].begin());
+            (int)(std::partition_point(tfaces[t].begin(), tfaces[t].end(), [&](int f) { return f < g.n_int; }) -
+                  tfaces[t].begin());
         d.max_tile_faces = std::max(d.max_tile_faces, nft);
         d.max_grad_slots = std::max(d.max_grad_slots, ntc + (int)thalo[t].size());
     }
@@ -518,7 +549,8 @@ int build_layout(const lbfs_mesh_desc &m, const Geometry &g, const std::vector<d
                 std::memcpy(&ob, &on[0], 4);
                 std::memcpy(&nbb, &on[1], 4);
                 const float a4[4] = {(float)(g.normal[3 * (size_t)f] * A), (float)(g.normal[3 * (size_t)f + 1] * A),
-                                     (float)(g.normal[3 * (size_t)f + 2] * A), (float)g.fdt[f]};
+                                     (float)(g.normal[3 * (size_t)f + 2] * A),
+                                     std::copysign((float)g.fdt[f], face_class(f) ? -1.0f : 1.0f)};
                 const float b4[4] = {(float)d1.x, (float)d1.y, (float)d1.z, ob};
                 const float c4[4] = {(float)d2.x, (float)d2.y, (float)d2.z, nbb};
                 std::copy(a4, a4 + 4, d.fA.begin() + 4 * r);
@@ -526,11 +558,17 @@ int build_layout(const lbfs_mesh_desc &m, const Geometry &g, const std::vector<d
                 std::copy(c4, c4 + 4, d.fC.begin() + 4 * r);
                 d.face_ref[r] = f;
             }
+            // each class is in face order
+            size_t cut[4] = {0, 0, 0, faces.size()};
+            for (int c = 1; c < 3; c++)
+                cut[c] = std::partition_point(faces.begin(), faces.end(), [&](int f) { return face_class(f) < c; }) -
+                         faces.begin();
             for (int i = c0; i < c1; i++) {
                 const int c = d.perm[i];
                 for (int k = 0; k < 6; k++) {
-                    const int f = g.gface[6 * (size_t)c + k];
-                    const int sl = (int)(std::lower_bound(faces.begin(), faces.end(), f) - faces.begin());
+                    const int f = g.gface[6 * (size_t)c + k], q = face_class(f);
+                    const int sl = (int)(std::lower_bound(faces.begin() + cut[q], faces.begin() + cut[q + 1], f) -
+                                         faces.begin());
                     const int own = g.grole[6 * (size_t)c + k] == 0 ? 0x8000 : 0;
                     d.cell_slots[6 * (size_t)i + k] = (int16_t)(uint16_t)(sl | own);
                 }

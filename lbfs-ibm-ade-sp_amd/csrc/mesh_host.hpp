@@ -71,7 +71,8 @@ struct DeviceLayout {
     std::vector<int> perm;        // internal id -> caller id
     std::vector<int> inv;         // caller id -> internal id
     std::vector<int> tile_cell_start, tile_face_start;
-    std::vector<int> tile_bface_start;  // per tile: first boundary face (interior faces come first)
+    std::vector<int> tile_bface_start;  // per tile: first boundary face (interior faces come first, those of
+                                        // the general reconstruction last among them)
     // per cell (internal order)
     std::vector<int> stencil;     // 6 * n, SoA [k*n + i]; ghost entries encoded -1 - bc
     std::vector<float> gw;        // 18 * n, SoA [(k*3+c)*n + i], W_k = LHS^-1 RHS_k
@@ -82,7 +83,10 @@ struct DeviceLayout {
     // per tile-face (duplicated across tiles)
     // 48 B per face: the area-weighted normal (area = its length), the
     // centroid offsets, and the owner and neighbour ids as int bits
-    std::vector<float> fA;        // 4 per face: normal * area xyz, face dt
+    std::vector<float> fA;        // 4 per face: normal * area xyz, face dt with the sign bit set where the
+                                  // face takes the general reconstruction: boundary faces and faces
+                                  // with a lattice direction within rounding of their plane (or of
+                                  // the tie band), whose points may come from either side
     std::vector<float> fB;        // 4 per face: owner centroid - face centroid, owner id
     std::vector<float> fC;        // 4 per face: neighbour image centroid - face centroid, neighbour id
                                   // (ghost: n_cells + bc)
@@ -99,7 +103,7 @@ struct DeviceLayout {
     std::vector<int> bc_owner;    // internal owner id per bc
 };
 int build_layout(const lbfs_mesh_desc &m, const Geometry &g, const std::vector<double> &lhs,
-                 const std::vector<double> &rhs, double rho0, const double body_force[3], int dims, const int tile[3],
-                 const std::vector<HostBlock> &blocks, DeviceLayout &d, std::string &err);
+                 const std::vector<double> &rhs, double rho0, const double body_force[3], int lattice, bool band,
+                 const int tile[3], const std::vector<HostBlock> &blocks, DeviceLayout &d, std::string &err);
 
 }  // namespace lbfs
