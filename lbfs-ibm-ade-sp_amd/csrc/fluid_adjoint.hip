@@ -188,11 +188,10 @@ __device__ __forceinline__ void all_pair_vjps(std::integer_sequence<int, P...>, 
 template <class L, bool GHOST>
 __device__ __forceinline__ void face_vjp(const FluidArgs &a, const float4 *__restrict__ st,
                                          const float4 *__restrict__ grad, const float4 *__restrict__ mu, int tf,
-                                         float4 out[8])
+                                         int o, int nb, float4 out[8])
 {
-    const FaceRec fr = load_face(a, tf);
-    const float4 fb = fr.d1, fcv = fr.d2;
-    const int o = fr.o, nb = fr.nb;
+    const FaceRec fr = unpack_face(load_face_raw(a, tf));
+    const float3 fb = fr.d1, fcv = fr.d2;
     constexpr bool ghost = GHOST;  // boundary faces follow the interior faces in every tile list
     const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
@@ -377,10 +376,8 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_flux(FluidArgs a, AdjFluidA
                                                           const float4 *__restrict__ grad)
 {
     extern __shared__ float4 lds_adj[];
-    const int t = xcd_remap(blockIdx.x, gridDim.x);
-    const int f0 = a.tile_face_start[t], f1 = a.tile_face_start[t + 1];
-    const int c0 = a.tile_cell_start[t], c1 = a.tile_cell_start[t + 1];
-    const int fb = a.tile_bface_start[t];
+    const TileRec T = a.tiles[xcd_remap(blockIdx.x, gridDim.x)];
+    const int f0 = T.f0, f1 = T.f0 + T.nf, c0 = T.c0, c1 = T.c0 + T.nc, fb = T.f0 + T.nif;
     float acc[ADJ_CELLS][16];
     uint32_t slot[ADJ_CELLS][6];
 #pragma unroll
@@ -389,7 +386,7 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_flux(FluidArgs a, AdjFluidA
         for (int k = 0; k < 16; k++) acc[u][k] = 0.0f;
         const int i = c0 + (int)threadIdx.x + u * ADJ_THREADS;
         if (i < c1) {
-            const uint32_t *sl = reinterpret_cast<const uint32_t *>(a.cell_slots) + 3 * (size_t)i;
+            const uint32_t *sl = reinterpret_cast<const uint32_t *>(a.cell_slots) + 3 * (size_t)(T.pc + i - c0);
             const uint32_t s01 = sl[0], s23 = sl[1], s45 = sl[2];
             slot[u][0] = s01 & 0xffffu; slot[u][1] = s01 >> 16;
             slot[u][2] = s23 & 0xffffu; slot[u][3] = s23 >> 16;
@@ -403,8 +400,10 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_flux(FluidArgs a, AdjFluidA
         const int ce = cs + ADJ_CHUNK < f1 ? cs + ADJ_CHUNK : f1;
         for (int f = cs + threadIdx.x; f < ce; f += ADJ_THREADS) {
             float4 o[8];
-            if (f < fb) face_vjp<L, false>(a, st, grad, j.mu, f, o);
-            else face_vjp<L, true>(a, st, grad, j.mu, f, o);
+            const uint32_t gs = a.face_gslot[T.pf + f - f0];
+            const int oc = slot_cell(a, T, gs & 0xffffu), nb = face_neighbour(a, T, gs, f - f0);
+            if (f < fb) face_vjp<L, false>(a, st, grad, j.mu, f, oc, nb, o);
+            else face_vjp<L, true>(a, st, grad, j.mu, f, oc, nb, o);
 #pragma unroll
             for (int k = 0; k < 8; k++) lds_adj[k * ADJ_CHUNK + (f - cs)] = o[k];
         }

@@ -13,6 +13,17 @@
 
 namespace lbfs {
 
+// Multiply-adds are written out in the forward fluid path (this header up to
+// the reset at its end, and the kernels that use it): which products the
+// compiler fuses would otherwise depend on the kernel they are inlined into,
+// and the one-pass and two-pass steps give the same bits.
+#pragma clang fp contract(off)
+
+__device__ __forceinline__ float dot3(float ax, float ay, float az, float bx, float by, float bz)
+{
+    return fmaf(ax, bx, fmaf(ay, by, az * bz));
+}
+
 __device__ __forceinline__ void load_grad(const float4 *__restrict__ grad, int i, float g[12])
 {
     const float4 a = grad[3 * (size_t)i], b = grad[3 * (size_t)i + 1], c = grad[3 * (size_t)i + 2];
@@ -24,8 +35,7 @@ __device__ __forceinline__ void load_grad(const float4 *__restrict__ grad, int i
 // one tile-face record: unit normal and area from the area-weighted normal
 struct FaceRec {
     float nx, ny, nz, A, dt;
-    float4 d1, d2;  // owner and neighbour image centroid - face centroid (w: the ids' bits)
-    int o, nb;
+    float3 d1, d2;  // owner and neighbour image centroid - face centroid
     bool general;   // takes the general reconstruction (pair_step): boundary faces and faces with a
                     // lattice direction in their own plane (DeviceLayout::fA)
 };
@@ -46,22 +56,37 @@ __device__ __forceinline__ void length_and_inverse(float s, float &len, float &i
         inv = len > 0.0f ? 1.0f / len : 0.0f;
     }
 }
-__device__ __forceinline__ FaceRec load_face(const FluidArgs &a, int tf)
+// the record as stored
+struct FaceRaw {
+    float4 fa, fb;
+    float2 fc;
+};
+__device__ __forceinline__ FaceRaw load_face_raw(const FluidArgs &a, int tf) { return {a.fA[tf], a.fB[tf], a.fC[tf]}; }
+__device__ __forceinline__ FaceRec unpack_face(const FaceRaw &raw)
 {
-    const float4 fa = a.fA[tf];
+    const float4 fa = raw.fa;
     FaceRec r;
-    r.d1 = a.fB[tf];
-    r.d2 = a.fC[tf];
+    r.d1 = make_float3(raw.fb.x, raw.fb.y, raw.fb.z);
+    r.d2 = make_float3(raw.fb.w, raw.fc.x, raw.fc.y);
     float iA;
-    length_and_inverse(fa.x * fa.x + fa.y * fa.y + fa.z * fa.z, r.A, iA);
+    length_and_inverse(dot3(fa.x, fa.y, fa.z, fa.x, fa.y, fa.z), r.A, iA);
     r.nx = fa.x * iA;
     r.ny = fa.y * iA;
     r.nz = fa.z * iA;
     r.dt = fabsf(fa.w);
     r.general = __float_as_int(fa.w) < 0;
-    r.o = __float_as_int(r.d1.w);
-    r.nb = __float_as_int(r.d2.w);
     return r;
+}
+
+// cell id of a slot of tile T, and the neighbour of its face q: a cell id, or
+// n_cells + the boundary face's number
+__device__ __forceinline__ int slot_cell(const FluidArgs &a, const TileRec &T, int slot)
+{
+    return slot < T.nc ? T.c0 + slot : a.halo_ids[T.h0 + slot - T.nc];
+}
+__device__ __forceinline__ int face_neighbour(const FluidArgs &a, const TileRec &T, uint32_t gs, int q)
+{
+    return q < T.nif ? slot_cell(a, T, gs >> 16) : a.n_cells + a.tile_bc[T.b0 + q - T.nif];
 }
 
 template <class L>
@@ -100,20 +125,13 @@ __device__ __forceinline__ void efma(float &s, float a, float b)
 
 // equilibrium deviation g = w (drho + rho P) of one lattice point with state
 // ph = (drho, u, v, w): P = 3 e.u + 4.5 (e.u)^2 / gamma - 1.5 u.u / gamma
-__device__ __forceinline__ float eq_point_eu(const float ph[4], float eu, float w, float rho0, float ig)
-{
-    const float uu = ph[1] * ph[1] + ph[2] * ph[2] + ph[3] * ph[3];
-    const float P = eu * (3.0f + 4.5f * ig * eu) - 1.5f * ig * uu;
-    return w * (ph[0] + (rho0 + ph[0]) * P);
-}
-
 template <int EX, int EY, int EZ>
 __device__ __forceinline__ float eq_point(const float ph[4], float w, float rho0, float ig)
 {
     const float eu = edot<EX, EY, EZ>(ph[1], ph[2], ph[3]);
-    const float uu = ph[1] * ph[1] + ph[2] * ph[2] + ph[3] * ph[3];
-    const float P = eu * (3.0f + 4.5f * ig * eu) - 1.5f * ig * uu;
-    return w * (ph[0] + (rho0 + ph[0]) * P);
+    const float uu = dot3(ph[1], ph[2], ph[3], ph[1], ph[2], ph[3]);
+    const float P = fmaf(eu, fmaf(4.5f * ig, eu, 3.0f), -1.5f * ig * uu);
+    return w * fmaf(rho0 + ph[0], P, ph[0]);
 }
 
 struct FaceSums {
@@ -149,8 +167,7 @@ __device__ __forceinline__ void pair_step(FaceSums &f, const float po[4], const 
     const float gs = gk + gb, gd = gk - gb;
     f.S0 += gs;
     eacc<ex>(f.S1x, gd); eacc<ey>(f.S1y, gd); eacc<ez>(f.S1z, gd);
-    const float eng = en * gs;
-    eacc<ex>(f.Tx, eng); eacc<ey>(f.Ty, eng); eacc<ez>(f.Tz, eng);
+    efma<ex>(f.Tx, en, gs); efma<ey>(f.Ty, en, gs); efma<ez>(f.Tz, en, gs);
 }
 
 // The same pair on a face whose lattice directions all lie clearly on one side
@@ -209,5 +226,7 @@ __device__ __forceinline__ void all_pairs(std::integer_sequence<int, P...>, Face
 {
     (pair_step<L, BAND, 2 * P + 1>(f, po, pn, p0, go, gn, nx, ny, nz, bw, ghost, rho0, ig), ...);
 }
+
+#pragma clang fp contract(fast)
 
 }  // namespace lbfs

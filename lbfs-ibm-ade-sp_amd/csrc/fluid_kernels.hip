@@ -24,6 +24,8 @@
 
 namespace lbfs {
 
+#pragma clang fp contract(off)  // (fluid_device.hpp)
+
 // ---------------------------------------------------------------------------
 // gradients
 // ---------------------------------------------------------------------------
@@ -36,16 +38,20 @@ struct CellStencil {
     int jk[6];
     float wk[18];
 };
-__device__ __forceinline__ void load_stencil(const FluidArgs &a, const float4 *__restrict__ st, int i, CellStencil &c)
+__device__ __forceinline__ void load_stencil_ids(const FluidArgs &a, int i, CellStencil &c)
 {
-    const int n = a.n_cells;
-    c.si = st[i];
 #pragma unroll
-    for (int k = 0; k < 6; k++) c.jk[k] = a.stencil[(size_t)k * n + i];
+    for (int k = 0; k < 6; k++) c.jk[k] = a.stencil[(size_t)k * a.n_cells + i];
+}
+// (after the ids) cell i's weights are entry e of rows of length n
+__device__ __forceinline__ void load_stencil(const float4 *__restrict__ st, int i, const float *__restrict__ w, int n,
+                                             unsigned e, CellStencil &c)
+{
+    c.si = st[i];
 #pragma unroll
     for (int k = 0; k < 6; k++) c.sk[k] = st[c.jk[k] >= 0 ? c.jk[k] : i];
 #pragma unroll
-    for (int k = 0; k < 18; k++) c.wk[k] = a.gw[(size_t)k * n + i];
+    for (int k = 0; k < 18; k++) c.wk[k] = w[(size_t)k * n + e];
 }
 __device__ __forceinline__ void stencil_gradient(const FluidArgs &a, const CellStencil &c, float R[12])
 {
@@ -72,16 +78,20 @@ __device__ __forceinline__ void stencil_gradient(const FluidArgs &a, const CellS
             dw = mv ? 2.0f * (bv.w - si.w) : 0.0f;
         }
         const float wx = c.wk[3 * k], wy = c.wk[3 * k + 1], wz = c.wk[3 * k + 2];
-        R[0] += wx * dr; R[1] += wy * dr; R[2] += wz * dr;
-        R[3] += wx * du; R[4] += wy * du; R[5] += wz * du;
-        R[6] += wx * dv; R[7] += wy * dv; R[8] += wz * dv;
-        R[9] += wx * dw; R[10] += wy * dw; R[11] += wz * dw;
+        const float d[4] = {dr, du, dv, dw};
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            R[3 * v] = fmaf(wx, d[v], R[3 * v]);
+            R[3 * v + 1] = fmaf(wy, d[v], R[3 * v + 1]);
+            R[3 * v + 2] = fmaf(wz, d[v], R[3 * v + 2]);
+        }
     }
 }
 __device__ __forceinline__ void cell_gradient(const FluidArgs &a, const float4 *__restrict__ st, int i, float R[12])
 {
     CellStencil c;
-    load_stencil(a, st, i, c);
+    load_stencil_ids(a, i, c);
+    load_stencil(st, i, a.gw, a.n_cells, i, c);
     stencil_gradient(a, c, R);
 }
 
@@ -104,21 +114,15 @@ __global__ __launch_bounds__(256) void k_gradients(FluidArgs a, const float4 *__
 // and of the cells across its border in LDS, at the face's slots)
 struct GlobalGrad {
     const float4 *__restrict__ grad;
-    __device__ __forceinline__ void load_owner(int, int i, float g[12]) const { load_grad(grad, i, g); }
-    __device__ __forceinline__ void load_nbr(int, int i, float g[12]) const { load_grad(grad, i, g); }
+    int o, n;  // owner and neighbour ids
+    __device__ __forceinline__ void load_owner(float g[12]) const { load_grad(grad, o, g); }
+    __device__ __forceinline__ void load_nbr(float g[12]) const { load_grad(grad, n, g); }
 };
 struct TileGrad {
-    const float4 *lg;              // LDS: 3 float4 per gradient slot
-    const uint32_t *__restrict__ slots;  // per tile-face: owner slot | neighbour slot << 16
-    __device__ __forceinline__ void at(int q, float g[12]) const
-    {
-        const float4 x = lg[3 * q], y = lg[3 * q + 1], z = lg[3 * q + 2];
-        g[0] = x.x; g[1] = x.y; g[2] = x.z; g[3] = x.w;
-        g[4] = y.x; g[5] = y.y; g[6] = y.z; g[7] = y.w;
-        g[8] = z.x; g[9] = z.y; g[10] = z.z; g[11] = z.w;
-    }
-    __device__ __forceinline__ void load_owner(int tf, int, float g[12]) const { at(slots[tf] & 0xffffu, g); }
-    __device__ __forceinline__ void load_nbr(int tf, int, float g[12]) const { at(slots[tf] >> 16, g); }
+    const float4 *lg;  // LDS: 3 float4 per gradient slot
+    uint32_t slots;    // the face's owner slot | neighbour slot << 16
+    __device__ __forceinline__ void load_owner(float g[12]) const { load_grad(lg, slots & 0xffffu, g); }
+    __device__ __forceinline__ void load_nbr(float g[12]) const { load_grad(lg, slots >> 16, g); }
 };
 
 // ---------------------------------------------------------------------------
@@ -126,17 +130,15 @@ struct TileGrad {
 // ---------------------------------------------------------------------------
 // states and gradients extrapolated to an interior face from both sides, and
 // their mean
-template <class G>
-__device__ __forceinline__ void interior_sides(const float4 &d1, const float4 &d2, const float sov[4], const float4 sn,
-                                               const float go[12], float gn[12], const G &gsrc, int tf, int nb,
-                                               float po[4], float pn[4], float p0[4])
+__device__ __forceinline__ void interior_sides(const FaceRec &fr, const float4 &so, const float4 &sn,
+                                               const float go[12], const float gn[12], float po[4], float pn[4],
+                                               float p0[4])
 {
-    gsrc.load_nbr(tf, nb, gn);
-    const float snv[4] = {sn.x, sn.y, sn.z, sn.w};
+    const float sov[4] = {so.x, so.y, so.z, so.w}, snv[4] = {sn.x, sn.y, sn.z, sn.w};
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-        po[v] = sov[v] - (d1.x * go[3 * v] + d1.y * go[3 * v + 1] + d1.z * go[3 * v + 2]);
-        pn[v] = snv[v] - (d2.x * gn[3 * v] + d2.y * gn[3 * v + 1] + d2.z * gn[3 * v + 2]);
+        po[v] = sov[v] - dot3(fr.d1.x, fr.d1.y, fr.d1.z, go[3 * v], go[3 * v + 1], go[3 * v + 2]);
+        pn[v] = snv[v] - dot3(fr.d2.x, fr.d2.y, fr.d2.z, gn[3 * v], gn[3 * v + 1], gn[3 * v + 2]);
         p0[v] = 0.5f * (po[v] + pn[v]);
     }
 }
@@ -145,28 +147,30 @@ __device__ __forceinline__ void interior_sides(const float4 &d1, const float4 &d
 template <class L>
 __device__ __forceinline__ float rest_point(const float p0[4], float rho0, float ig)
 {
-    const float uu = p0[1] * p0[1] + p0[2] * p0[2] + p0[3] * p0[3];
-    return L::w(0) * (p0[0] + (rho0 + p0[0]) * (-1.5f * uu * ig));
+    const float uu = dot3(p0[1], p0[2], p0[3], p0[1], p0[2], p0[3]);
+    return L::w(0) * fmaf(rho0 + p0[0], -1.5f * ig * uu, p0[0]);
 }
 
+// The flux of tile-face tf from its record, the states of its owner (cell o)
+// and neighbour (nb: cell id, or n_cells + boundary face, whose sn is unused)
+// and their gradients
 template <class L, bool BAND, class G>
-__device__ __forceinline__ float4 face_flux(const FluidArgs &a, const float4 *__restrict__ st, const G &gsrc, int tf)
+__device__ __forceinline__ float4 face_flux(const FluidArgs &a, const G &gsrc, int tf, const FaceRaw &raw,
+                                            const float4 &so, const float4 &sn, int o, int nb)
 {
     static_assert(opposite_pairs<L>(), "lattice directions must come in opposite pairs after the rest point");
-    const FaceRec fr = load_face(a, tf);
-    const float4 fb = fr.d1, fcv = fr.d2;
-    const int o = fr.o, nb = fr.nb;
+    const FaceRec fr = unpack_face(raw);
+    const float3 fb = fr.d1;
     const float nx = fr.nx, ny = fr.ny, nz = fr.nz, A = fr.A, dt = fr.dt;
     const float rho0 = a.rho0, ig = a.inv_gamma;
-    const float4 so = st[o];
     float go[12], gn[12];
-    gsrc.load_owner(tf, o, go);
-    const float sov[4] = {so.x, so.y, so.z, so.w};
+    gsrc.load_owner(go);
     float po[4], pn[4], p0[4];
     FaceSums f;
     f.S1x = f.S1y = f.S1z = f.Tx = f.Ty = f.Tz = 0.0f;
     if (!fr.general) {
-        interior_sides(fb, fcv, sov, st[nb], go, gn, gsrc, tf, nb, po, pn, p0);
+        gsrc.load_nbr(gn);
+        interior_sides(fr, so, sn, go, gn, po, pn, p0);
         f.S0 = rest_point<L>(p0, rho0, ig);
         const float ig15 = 1.5f * ig;
         all_pairs_fast<L>(std::make_integer_sequence<int, (L::Q - 1) / 2>{}, f, po, pn, go, gn, nx, ny, nz, dt,
@@ -174,8 +178,10 @@ __device__ __forceinline__ float4 face_flux(const FluidArgs &a, const float4 *__
     } else {
         const bool ghost = nb >= a.n_cells;
         if (!ghost) {
-            interior_sides(fb, fcv, sov, st[nb], go, gn, gsrc, tf, nb, po, pn, p0);
+            gsrc.load_nbr(gn);
+            interior_sides(fr, so, sn, go, gn, po, pn, p0);
         } else {
+            const float sov[4] = {so.x, so.y, so.z, so.w};
             // ghost gradient (gradients.cpp:393-505 / LBFS.cu:1933-2048) and face
             // value from the boundary condition (Solver.cpp:855-900)
             const int bc = nb - a.n_cells;
@@ -183,7 +189,7 @@ __device__ __forceinline__ float4 face_flux(const FluidArgs &a, const float4 *__
             if (ty.y == LBFS_BC_EMPTY) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // Solver.cpp:308-310
             const float4 bv = a.bc_val[bc];
             const float bvv[4] = {bv.x, bv.y, bv.z, bv.w};
-            const float d1n = sqrtf(fb.x * fb.x + fb.y * fb.y + fb.z * fb.z);
+            const float d1n = sqrtf(dot3(fb.x, fb.y, fb.z, fb.x, fb.y, fb.z));
             const float inv_dmag = 2.0f / d1n;  // ghost centroid sits halfway to the face
             float dir[3];
             if (a.flags & LBFS_FLAG_GHOST_DIR_GPU) { dir[0] = -fb.x / d1n; dir[1] = -fb.y / d1n; dir[2] = -fb.z / d1n; }
@@ -198,14 +204,15 @@ __device__ __forceinline__ float4 face_flux(const FluidArgs &a, const float4 *__
                     for (int c = 0; c < 3; c++) gn[3 * v + c] = dphi * dir[c];
                     // code 3 (parabolic/shear targets) extrapolates the face value
                     // with the ghost gradient (LBFS.cu:358-378)
-                    p0[v] = type == 1 ? bvv[v] : sov[v] - (fb.x * gn[3 * v] + fb.y * gn[3 * v + 1] + fb.z * gn[3 * v + 2]);
+                    p0[v] = type == 1 ? bvv[v]
+                                      : sov[v] - dot3(fb.x, fb.y, fb.z, gn[3 * v], gn[3 * v + 1], gn[3 * v + 2]);
                 } else {
 #pragma unroll
                     for (int c = 0; c < 3; c++) {
                         const float fac = (a.flags & LBFS_FLAG_NEUMANN_SIGNED) ? 1.0f - nv[c] : 1.0f - fabsf(nv[c]);
                         gn[3 * v + c] = go[3 * v + c] * fac;
                     }
-                    p0[v] = sov[v] - (fb.x * gn[3 * v] + fb.y * gn[3 * v + 1] + fb.z * gn[3 * v + 2]);
+                    p0[v] = sov[v] - dot3(fb.x, fb.y, fb.z, gn[3 * v], gn[3 * v + 1], gn[3 * v + 2]);
                 }
                 po[v] = p0[v];
                 pn[v] = p0[v];
@@ -226,7 +233,7 @@ __device__ __forceinline__ float4 face_flux(const FluidArgs &a, const float4 *__
     const float S0 = f.S0, S1x = f.S1x, S1y = f.S1y, S1z = f.S1z, Tx = f.Tx, Ty = f.Ty, Tz = f.Tz;
     if (a.face_moments) a.face_moments[tf] = make_float4(S0, S1x, S1y, S1z);
     const float rho_f = rho0 + S0;
-    const float mn = S1x * nx + S1y * ny + S1z * nz;
+    const float mn = dot3(S1x, S1y, S1z, nx, ny, nz);
     const float vf = a.visc_factor ? a.visc_factor[o] : 1.0f;
     const float tau = a.visc3_over_gamma * vf * __builtin_amdgcn_rcpf(dt);
     const float c1 = 1.0f - tau;
@@ -234,10 +241,10 @@ __device__ __forceinline__ float4 face_flux(const FluidArgs &a, const float4 *__
     const float q = mn * __builtin_amdgcn_rcpf(rho_f) * ig;
     float4 r;
     r.x = mn * A;
-    r.y = A * (c1 * (third * nx + S1x * q) + tau * Tx);
-    r.z = A * (c1 * (third * ny + S1y * q) + tau * Ty);
+    r.y = A * fmaf(c1, fmaf(S1x, q, third * nx), tau * Tx);
+    r.z = A * fmaf(c1, fmaf(S1y, q, third * ny), tau * Ty);
     // a planar lattice carries no z momentum flux (its sum e_z e_z w is zero)
-    r.w = L::dims == 3 ? A * (c1 * (third * nz + S1z * q) + tau * Tz) : 0.0f;
+    r.w = L::dims == 3 ? A * fmaf(c1, fmaf(S1z, q, third * nz), tau * Tz) : 0.0f;
     return r;
 }
 
@@ -245,12 +252,13 @@ __device__ __forceinline__ float4 face_flux(const FluidArgs &a, const float4 *__
 // its six signed face slots in a fixed order (LBFS.cu:2242-2281), adds the
 // force density and advances (LBFS.cu:2089-2172)
 template <int NT>
-__device__ __forceinline__ void tile_update(const FluidArgs &a, const float4 *lds_flux, int c0, int c1,
+__device__ __forceinline__ void tile_update(const FluidArgs &a, const float4 *lds_flux, const TileRec &T,
                                             const float4 *__restrict__ st, float4 *__restrict__ st_out,
                                             float4 *__restrict__ res_out, int do_update)
 {
-    for (int i = c0 + threadIdx.x; i < c1; i += NT) {
-        const uint32_t *sl = reinterpret_cast<const uint32_t *>(a.cell_slots) + 3 * (size_t)i;
+    for (int q = threadIdx.x; q < T.nc; q += NT) {
+        const int i = T.c0 + q;
+        const uint32_t *sl = reinterpret_cast<const uint32_t *>(a.cell_slots) + 3 * (size_t)(T.pc + q);
         const uint32_t s01 = sl[0], s23 = sl[1], s45 = sl[2];
         // the cell's state and force loaded with its slots, not after the sums
         const float4 s0 = do_update ? st[i] : float4{};
@@ -265,7 +273,7 @@ __device__ __forceinline__ void tile_update(const FluidArgs &a, const float4 *ld
         for (int k = 0; k < 6; k++) {
             const float4 fl = lds_flux[s[k] & 0x7fffu];
             const float sg = (s[k] & 0x8000u) ? -1.0f : 1.0f;
-            r0 += sg * fl.x; r1 += sg * fl.y; r2 += sg * fl.z; r3 += sg * fl.w;
+            r0 = fmaf(sg, fl.x, r0); r1 = fmaf(sg, fl.y, r1); r2 = fmaf(sg, fl.z, r2); r3 = fmaf(sg, fl.w, r3);
         }
         const float iv = a.inv_vol[i];
         r0 *= iv; r1 *= iv; r2 *= iv; r3 *= iv;
@@ -283,16 +291,27 @@ __device__ __forceinline__ void tile_update(const FluidArgs &a, const float4 *ld
         } else if (a.ts_mode == LBFS_TS_MIN) {
             dt = __uint_as_float(*a.dt_min);
         }
-        const float drho = s0.x + dt * r0;
+        const float drho = fmaf(dt, r0, s0.x);
         const float rho = a.rho0 + drho;
         const float inv_rho = 1.0f / rho;
         float4 sn;
         sn.x = drho;
-        sn.y = s0.y + dt * (r1 - s0.y * r0) * inv_rho;
-        sn.z = s0.z + dt * (r2 - s0.z * r0) * inv_rho;
-        sn.w = s0.w + dt * (r3 - s0.w * r0) * inv_rho;
+        sn.y = fmaf(dt * fmaf(-s0.y, r0, r1), inv_rho, s0.y);
+        sn.z = fmaf(dt * fmaf(-s0.z, r0, r2), inv_rho, s0.z);
+        sn.w = fmaf(dt * fmaf(-s0.w, r0, r3), inv_rho, s0.w);
         st_out[i] = sn;
     }
+}
+
+// face q of tile T from the gradient array
+template <class L, bool BAND>
+__device__ __forceinline__ float4 tile_face_flux(const FluidArgs &a, const float4 *__restrict__ st,
+                                                 const float4 *__restrict__ grad, const TileRec &T, int q)
+{
+    const uint32_t gs = a.face_gslot[T.pf + q];
+    const int o = slot_cell(a, T, gs & 0xffffu), nb = face_neighbour(a, T, gs, q);
+    const int n = q < T.nif ? nb : o;  // (a boundary face loads its owner's, unused)
+    return face_flux<L, BAND>(a, GlobalGrad{grad, o, n}, T.f0 + q, load_face_raw(a, T.f0 + q), st[o], st[n], o, nb);
 }
 
 // two-pass step, second pass: the tile's faces from the gradient array
@@ -302,13 +321,11 @@ __global__ __launch_bounds__(NT) void k_flux_update(FluidArgs a, const float4 *_
                                                      float4 *__restrict__ res_out, int do_update)
 {
     extern __shared__ float4 lds_flux[];
-    const int t = xcd_remap(blockIdx.x, gridDim.x);
-    const int f0 = a.tile_face_start[t], f1 = a.tile_face_start[t + 1];
-    const GlobalGrad gsrc{grad};
-    for (int f = f0 + threadIdx.x; f < f1; f += blockDim.x)
-        lds_flux[f - f0] = face_flux<L, BAND>(a, st, gsrc, f);
+    const TileRec T = a.tiles[xcd_remap(blockIdx.x, gridDim.x)];
+    for (int q = threadIdx.x; q < T.nf; q += NT)
+        lds_flux[q] = tile_face_flux<L, BAND>(a, st, grad, T, q);
     __syncthreads();
-    tile_update<NT>(a, lds_flux, a.tile_cell_start[t], a.tile_cell_start[t + 1], st, st_out, res_out, do_update);
+    tile_update<NT>(a, lds_flux, T, st, st_out, res_out, do_update);
 }
 
 // Fused step, one workgroup per tile: the gradients of the tile's cells and
@@ -316,48 +333,88 @@ __global__ __launch_bounds__(NT) void k_flux_update(FluidArgs a, const float4 *_
 // arithmetic as the gradient pass), the tile's faces from them, then the cell
 // update.  Results equal the two-pass step bit for bit; the gradient array is
 // not read, and written (the tile's own cells) only when a.grad_out is set.
+//
+// Bound by memory: at 256x128x128 the same loads without the face arithmetic
+// take 0.97 of its time, 333 us for the 330 B a cell it moves (4.1 TB/s; a
+// device copy on the same card 5.1).  What it reads is laid out for it: cells
+// by slots of shared patterns rather than ids (faces 40 B, no stencil), the
+// weights of a tile and its halo as whole rows, each thread's next face on its
+// way while the present one is reconstructed.  D3Q19, 8x8x8 tiles, with face
+// ids, stencil ids and gathered weights before: 128x64x64 42.9 -> 38.3 us,
+// 256x128x128 428 -> 333 us.
 template <class L, bool BAND, int NT>
 __global__ __launch_bounds__(NT) void k_fluid_fused(FluidArgs a, const float4 *__restrict__ st,
                                                      float4 *__restrict__ st_out, float4 *__restrict__ res_out,
                                                      int do_update)
 {
     extern __shared__ float4 lds[];
-    float4 *lg = lds;                                   // 3 per gradient slot
-    float4 *lds_flux = lds + 3 * (size_t)a.max_grad_slots;
-    const int t = xcd_remap(blockIdx.x, gridDim.x);
-    const int c0 = a.tile_cell_start[t], c1 = a.tile_cell_start[t + 1], nc = c1 - c0;
-    const int h0 = a.tile_halo_start[t], nq = nc + a.tile_halo_start[t + 1] - h0;
-    for (int q = threadIdx.x; q < nq; q += NT) {
-        const int i = q < nc ? c0 + q : a.halo_ids[h0 + q - nc];
+    float4 *lg = lds;                                        // 3 per gradient slot
+    float4 *lds_flux = lg + 3 * (size_t)a.max_grad_slots;    // 1 per face
+    int *ids = reinterpret_cast<int *>(lds_flux + a.max_tile_faces);  // cell id of each slot
+    const TileRec T = a.tiles[xcd_remap(blockIdx.x, gridDim.x)];
+    const int ns = T.nc + T.nh;
+    for (int q = threadIdx.x; q < ns + T.n2; q += NT) ids[q] = q < T.nc ? T.c0 + q : a.halo_ids[T.h0 + q - T.nc];
+    // the first face's record and slots are on their way while the gradients
+    // are computed (here and below a thread past the end loads the last one's)
+    int q = threadIdx.x;
+    const int ql = T.nf - 1;
+    FaceRaw raw = load_face_raw(a, T.f0 + min(q, ql));
+    uint32_t gs = a.face_gslot[T.pf + min(q, ql)], gs1 = a.face_gslot[T.pf + min(q + NT, ql)];
+    __syncthreads();
+    for (int p = threadIdx.x; p < ns; p += NT) {
+        const int i = ids[p];
+        const uint32_t *nl = reinterpret_cast<const uint32_t *>(a.cell_nbrs) + 3 * (size_t)(T.pn + p);
+        const uint32_t n01 = nl[0], n23 = nl[1], n45 = nl[2];
+        const uint32_t nb[6] = {n01 & 0xffffu, n01 >> 16, n23 & 0xffffu, n23 >> 16, n45 & 0xffffu, n45 >> 16};
+        CellStencil c;
+#pragma unroll
+        for (int k = 0; k < 6; k++)
+            c.jk[k] = nb[k] & 0x8000u ? -1 - a.tile_bc[T.b0 + (nb[k] & 0x7fffu)] : ids[nb[k]];
         float R[12];
-        cell_gradient(a, st, i, R);
-        float4 *o = lg + 3 * q;
+        load_stencil(st, i, a.tile_w + 18 * (size_t)T.s0, ns, p, c);
+        stencil_gradient(a, c, R);
+        float4 *o = lg + 3 * p;
         o[0] = make_float4(R[0], R[1], R[2], R[3]);
         o[1] = make_float4(R[4], R[5], R[6], R[7]);
         o[2] = make_float4(R[8], R[9], R[10], R[11]);
-        if (a.grad_out && q < nc) {
+        if (a.grad_out && p < T.nc) {
             float4 *g = a.grad_out + 3 * (size_t)i;
             g[0] = o[0];
             g[1] = o[1];
             g[2] = o[2];
         }
     }
+    // a boundary face's neighbour slot is 0xffff: its state is the owner's, unused
+    const int last = ns - 1;
+    float4 so = st[ids[gs & 0xffffu]], sn = st[ids[min((int)(gs >> 16), last)]];
     __syncthreads();
-    const int f0 = a.tile_face_start[t], f1 = a.tile_face_start[t + 1];
-    const TileGrad gsrc{lg, a.face_gslot};
-    for (int f = f0 + threadIdx.x; f < f1; f += NT) lds_flux[f - f0] = face_flux<L, BAND>(a, st, gsrc, f);
+    while (q < T.nf) {
+        // the next face's record and states, and the slots of the one after,
+        // load while this one is reconstructed
+        const FaceRaw raw1 = load_face_raw(a, T.f0 + min(q + NT, ql));
+        const float4 so1 = st[ids[gs1 & 0xffffu]], sn1 = st[ids[min((int)(gs1 >> 16), last)]];
+        const uint32_t gs2 = a.face_gslot[T.pf + min(q + 2 * NT, ql)];
+        const int o = ids[gs & 0xffffu];
+        const int nb = q < T.nif ? 0 : a.n_cells + a.tile_bc[T.b0 + q - T.nif];
+        lds_flux[q] = face_flux<L, BAND>(a, TileGrad{lg, gs}, T.f0 + q, raw, so, sn, o, nb);
+        raw = raw1;
+        so = so1;
+        sn = sn1;
+        gs = gs1;
+        gs1 = gs2;
+        q += NT;
+    }
     __syncthreads();
-    tile_update<NT>(a, lds_flux, c0, c1, st, st_out, res_out, do_update);
+    tile_update<NT>(a, lds_flux, T, st, st_out, res_out, do_update);
 }
 
+// every tile-face's flux (one workgroup per tile)
 template <class L, bool BAND>
 __global__ __launch_bounds__(256) void k_face_flux_all(FluidArgs a, const float4 *__restrict__ st,
-                                                       const float4 *__restrict__ grad, float4 *__restrict__ out,
-                                                       int n_tile_faces)
+                                                       const float4 *__restrict__ grad, float4 *__restrict__ out)
 {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f < n_tile_faces)
-        out[f] = face_flux<L, BAND>(a, st, GlobalGrad{grad}, f);
+    const TileRec T = a.tiles[blockIdx.x];
+    for (int q = threadIdx.x; q < T.nf; q += 256) out[T.f0 + q] = tile_face_flux<L, BAND>(a, st, grad, T, q);
 }
 
 // ---------------------------------------------------------------------------
@@ -426,9 +483,27 @@ __global__ __launch_bounds__(256) void k_diag_partials(int n, float rho0, const 
     if (threadIdx.x < 6) part[6 * (size_t)blockIdx.x + threadIdx.x] = sh[threadIdx.x][0];
 }
 
+// the weight rows of each tile's gradient slots from the cells' (set-up)
+__global__ __launch_bounds__(256) void k_tile_weights(FluidArgs a, float *__restrict__ tw)
+{
+    const TileRec T = a.tiles[blockIdx.x];
+    const int ns = T.nc + T.nh;
+    float *w = tw + 18 * (size_t)T.s0;
+    for (int p = threadIdx.x; p < ns; p += 256) {
+        const int i = slot_cell(a, T, p);
+        for (int r = 0; r < 18; r++) w[(size_t)r * ns + p] = a.gw[(size_t)r * a.n_cells + i];
+    }
+}
+
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
+hipError_t launch_tile_weights(const FluidArgs &a, float *tile_w, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_tile_weights, dim3(a.n_tiles), dim3(256), 0, s, a, tile_w);
+    return hipGetLastError();
+}
+
 hipError_t launch_gradients(const FluidArgs &a, const float4 *st, float4 *grad, hipStream_t s)
 {
     const int blocks = (a.n_cells + 255) / 256;
@@ -470,9 +545,9 @@ struct FluxUpdate {
 template <class L, bool BAND>
 struct FaceFluxAll {
     static void launch(dim3 g, size_t lds, hipStream_t s, const FluidArgs &a, const float4 *st, const float4 *grad,
-                       float4 *out, int n)
+                       float4 *out)
     {
-        hipLaunchKernelGGL((k_face_flux_all<L, BAND>), g, dim3(256), lds, s, a, st, grad, out, n);
+        hipLaunchKernelGGL((k_face_flux_all<L, BAND>), g, dim3(256), lds, s, a, st, grad, out);
     }
 };
 
@@ -499,7 +574,7 @@ struct FluidFused {
 
 size_t fluid_fused_lds(const FluidArgs &a)
 {
-    return sizeof(float4) * (3 * (size_t)a.max_grad_slots + (size_t)a.max_tile_faces);
+    return sizeof(float4) * (3 * (size_t)a.max_grad_slots + (size_t)a.max_tile_faces) + sizeof(int) * a.max_slots;
 }
 
 hipError_t launch_fluid_fused(const FluidArgs &a, const float4 *st, float4 *st_out, float4 *res_out, int do_update,
@@ -508,11 +583,9 @@ hipError_t launch_fluid_fused(const FluidArgs &a, const float4 *st, float4 *st_o
     return dispatch<FluidFused>(a, dim3(a.n_tiles), fluid_fused_lds(a), s, st, st_out, res_out, do_update);
 }
 
-hipError_t launch_face_flux_all(const FluidArgs &a, const float4 *st, const float4 *grad, float4 *out, int n_tile_faces,
-                                hipStream_t s)
+hipError_t launch_face_flux_all(const FluidArgs &a, const float4 *st, const float4 *grad, float4 *out, hipStream_t s)
 {
-    const int blocks = (n_tile_faces + 255) / 256;
-    return dispatch<FaceFluxAll>(a, dim3(blocks), 0, s, st, grad, out, n_tile_faces);
+    return dispatch<FaceFluxAll>(a, dim3(a.n_tiles), 0, s, st, grad, out);
 }
 
 hipError_t launch_dt_min(const FluidArgs &a, const float4 *st, hipStream_t s)

@@ -71,17 +71,18 @@ static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params
                           lhs, rhs, err);
         if (rc) return ctx->fail(rc, "geometry: %s", err.c_str());
     }
-    int tile[3] = {8, 8, 4};
+    if (p.block_threads != 0 && p.block_threads != 256 && p.block_threads != 512 && p.block_threads != 576)
+        return ctx->fail(LBFS_E_INVALID_ARG, "block_threads must be 256, 512 or 576");
+    rc = mesh_blocks(m, p.body_force, ctx->blocks, err);
+    if (rc) return ctx->fail(rc, "mesh blocks: %s", err.c_str());
+    int tile[3] = {8, 8, 4}, threads = 256;
     if (p.tile[0] || p.tile[1] || p.tile[2]) {
         if (p.tile[0] < 1 || p.tile[1] < 1 || p.tile[2] < 1 || p.tile[0] * p.tile[1] * p.tile[2] > 2048)
             return ctx->fail(LBFS_E_INVALID_ARG, "tile %dx%dx%d: each side >= 1, at most 2048 cells", p.tile[0],
                              p.tile[1], p.tile[2]);
         for (int t = 0; t < 3; t++) tile[t] = p.tile[t];
     }
-    if (p.block_threads != 0 && p.block_threads != 256 && p.block_threads != 512 && p.block_threads != 576)
-        return ctx->fail(LBFS_E_INVALID_ARG, "block_threads must be 256, 512 or 576");
-    rc = mesh_blocks(m, p.body_force, ctx->blocks, err);
-    if (rc) return ctx->fail(rc, "mesh blocks: %s", err.c_str());
+    if (p.block_threads) threads = p.block_threads;
     rc = build_layout(m, ctx->geo, lhs, rhs, p.rho0, p.body_force, p.lattice, (p.flags & LBFS_FLAG_UPWIND_BAND) != 0,
                       tile, ctx->blocks, ctx->lay, err);
     if (rc) return ctx->fail(rc, "layout: %s", err.c_str());
@@ -93,25 +94,15 @@ static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params
     a.n_bc = nbc;
     a.n_tiles = d.n_tiles;
     a.max_tile_faces = d.max_tile_faces;
-    a.block_threads = p.block_threads == 512 || p.block_threads == 576 ? p.block_threads : 256;
+    a.block_threads = threads;
     if ((size_t)d.max_tile_faces * 16 > 96 * 1024)
         return ctx->fail(LBFS_E_INVALID_ARG, "tile too large: %d faces need more than 96 KiB of LDS", d.max_tile_faces);
     for (int t = 0; t < d.n_tiles; t++)
         a.max_tile_cells = std::max(a.max_tile_cells, d.tile_cell_start[t + 1] - d.tile_cell_start[t]);
     a.max_grad_slots = d.max_grad_slots;
-    {
-        int *ths, *hid;
-        uint32_t *fgs;
-        if ((rc = dev_upload(ctx, &ths, d.tile_halo_start.data(), d.tile_halo_start.size()))) return rc;
-        if ((rc = dev_upload(ctx, &hid, d.halo_ids.data(), d.halo_ids.size()))) return rc;
-        if ((rc = dev_upload(ctx, &fgs, d.face_gslot.data(), d.face_gslot.size()))) return rc;
-        a.tile_halo_start = ths;
-        a.halo_ids = hid;
-        a.face_gslot = fgs;
-    }
-    // the fused fluid pass keeps the tile's gradients in LDS beside its face
-    // fluxes; larger tiles run the two passes
-    ctx->fused_ok = fluid_fused_lds(a) <= 96 * 1024;
+    a.max_slots = d.max_slots;
+    // (larger tiles run the two passes)
+    ctx->fused_ok = d.fused_fits;
     ctx->fused = ctx->fused_ok;
     a.lattice = p.lattice;
     a.flags = p.flags;
@@ -121,21 +112,34 @@ static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params
     a.visc3_over_gamma = (float)(p.visc * 3.0 / p.gamma);
     a.dt = (float)p.dt;
     for (int t = 0; t < 3; t++) a.body_force[t] = (float)p.body_force[t];
-    int *stencil; float *gw, *inv_vol; int16_t *slots; int *tcs, *tfs;
-    float4 *fA, *fB, *fC; int2 *bct; float4 *bcv;
+    int *stencil; float *gw, *inv_vol; int *tcs;
+    float4 *fA, *fB; float2 *fC; int2 *bct; float4 *bcv;
     if ((rc = dev_upload(ctx, &stencil, d.stencil.data(), d.stencil.size()))) return rc;
     if ((rc = dev_upload(ctx, &gw, d.gw.data(), d.gw.size()))) return rc;
     if ((rc = dev_upload(ctx, &inv_vol, d.inv_vol.data(), d.inv_vol.size()))) return rc;
-    if ((rc = dev_upload(ctx, &slots, d.cell_slots.data(), d.cell_slots.size()))) return rc;
     if ((rc = dev_upload(ctx, &tcs, d.tile_cell_start.data(), d.tile_cell_start.size()))) return rc;
-    if ((rc = dev_upload(ctx, &tfs, d.tile_face_start.data(), d.tile_face_start.size()))) return rc;
-    int *tbs;
-    if ((rc = dev_upload(ctx, &tbs, d.tile_bface_start.data(), d.tile_bface_start.size()))) return rc;
-    a.tile_bface_start = tbs;
+    {
+        TileRec *tiles;
+        int *hid, *tbc;
+        uint32_t *fgs;
+        uint16_t *slots, *nbrs;
+        if ((rc = dev_upload(ctx, &tiles, d.tiles.data(), d.tiles.size()))) return rc;
+        if ((rc = dev_upload(ctx, &hid, d.halo_ids.data(), d.halo_ids.size()))) return rc;
+        if ((rc = dev_upload(ctx, &tbc, d.tile_bc.data(), d.tile_bc.size()))) return rc;
+        if ((rc = dev_upload(ctx, &fgs, d.face_gslot.data(), d.face_gslot.size()))) return rc;
+        if ((rc = dev_upload(ctx, &slots, d.cell_slots.data(), d.cell_slots.size()))) return rc;
+        if ((rc = dev_upload(ctx, &nbrs, d.cell_nbrs.data(), d.cell_nbrs.size()))) return rc;
+        a.tiles = tiles;
+        a.halo_ids = hid;
+        a.tile_bc = tbc;
+        a.face_gslot = fgs;
+        a.cell_slots = slots;
+        a.cell_nbrs = nbrs;
+    }
     const size_t ntf = d.face_ref.size();
     if ((rc = dev_upload(ctx, &fA, (const float4 *)d.fA.data(), ntf))) return rc;
     if ((rc = dev_upload(ctx, &fB, (const float4 *)d.fB.data(), ntf))) return rc;
-    if ((rc = dev_upload(ctx, &fC, (const float4 *)d.fC.data(), ntf))) return rc;
+    if ((rc = dev_upload(ctx, &fC, (const float2 *)d.fC.data(), ntf))) return rc;
     std::vector<int2> bt(nbc > 0 ? nbc : 1);
     ctx->bc_vel_type.assign(nbc, LBFS_BC_NEUMANN);
     std::vector<float4> bvals(nbc > 0 ? nbc : 1);
@@ -175,9 +179,15 @@ static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params
     }
     if ((rc = dev_upload(ctx, &bct, bt.data(), bt.size()))) return rc;
     if ((rc = dev_upload(ctx, &bcv, bvals.data(), bvals.size()))) return rc;
-    a.stencil = stencil; a.gw = gw; a.inv_vol = inv_vol; a.cell_slots = slots;
-    a.tile_cell_start = tcs; a.tile_face_start = tfs;
+    a.stencil = stencil; a.gw = gw; a.inv_vol = inv_vol;
+    a.tile_cell_start = tcs;
     a.fA = fA; a.fB = fB; a.fC = fC;
+    if (ctx->fused_ok) {
+        float *tw;
+        if ((rc = dev_upload<float>(ctx, &tw, nullptr, 18 * (size_t)d.n_slots))) return rc;
+        HIPCHK(launch_tile_weights(a, tw, ctx->stream));
+        a.tile_w = tw;
+    }
     a.bc_type = bct; a.bc_val = bcv;
     a.visc_factor = nullptr;
     // cell force density: body force + closure term, IBM forces are added on top
@@ -497,7 +507,7 @@ extern "C" int lbfs_stage_face_flux(lbfs_ctx *ctx, double *flux_out)
     if (!ctx || !flux_out) return LBFS_E_INVALID_ARG;
     const int ntf = (int)ctx->lay.face_ref.size();
     HIPCHK(launch_gradients(ctx->args, ctx->st[ctx->cur], ctx->grad, ctx->stream));
-    HIPCHK(launch_face_flux_all(ctx->args, ctx->st[ctx->cur], ctx->grad, ctx->face_scratch, ntf, ctx->stream));
+    HIPCHK(launch_face_flux_all(ctx->args, ctx->st[ctx->cur], ctx->grad, ctx->face_scratch, ctx->stream));
     std::vector<float4> h(ntf);
     HIPCHK(hipMemcpyAsync(h.data(), ctx->face_scratch, sizeof(float4) * ntf, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));

@@ -5,9 +5,11 @@
 #include "lattice.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <list>
 #include <mutex>
 #include <thread>
 #include <unordered_map>
@@ -39,6 +41,43 @@ void parallel_for(int n, F body, int grain = 1024)
     body(0, std::min(n, chunk));
     for (std::thread &th : pool) th.join();
 }
+
+// Slots of the cells a tile reaches: a small open-addressing table, cleared
+// per tile
+class SlotMap {
+    std::vector<int> key, val;
+    std::vector<unsigned> used;
+    unsigned mask;
+
+public:
+    SlotMap() : key(1024, -1), val(1024), mask(1023) {}
+    // makes room for n cells
+    void reset(size_t n)
+    {
+        for (unsigned h : used) key[h] = -1;
+        used.clear();
+        size_t cap = mask + 1;
+        while (cap < 4 * n) cap *= 2;
+        key.resize(cap, -1);
+        val.resize(cap);
+        mask = (unsigned)cap - 1;
+    }
+    // the slot of cell c, which is `next` if it has none yet (*added then)
+    int get(int c, int next, bool *added)
+    {
+        unsigned h = (unsigned)c * 2654435761u;
+        for (h = (h ^ (h >> 15)) & mask; key[h] != -1; h = (h + 1) & mask)
+            if (key[h] == c) {
+                *added = false;
+                return val[h];
+            }
+        *added = true;
+        used.push_back(h);
+        key[h] = c;
+        val[h] = next;
+        return next;
+    }
+};
 
 struct V3 {
     double x, y, z;
@@ -436,7 +475,6 @@ int build_layout(const lbfs_mesh_desc &m, const Geometry &g, const std::vector<d
     d.stencil.assign(6 * (size_t)nc, 0);
     d.gw.assign(18 * (size_t)nc, 0.0f);
     d.inv_vol.assign(nc, 0.0f);
-    d.cell_slots.assign(6 * (size_t)nc, 0);
     parallel_for(nc, [&](int i0, int i1) {
         for (int i = i0; i < i1; i++) {
             const int c = d.perm[i];
@@ -466,115 +504,216 @@ int build_layout(const lbfs_mesh_desc &m, const Geometry &g, const std::vector<d
             const double tol = 1e-6 + (band ? 0.001 * g.fdt[f] * (1.0 + 1e-6) : 0.0);
             fclass[f] = f >= g.n_int ? 2 : (min_direction_component(lattice, &g.normal[3 * (size_t)f]) > tol ? 0 : 1);
         }
-    });
-    auto face_class = [&](int f) { return (int)fclass[f]; };
-    std::vector<std::vector<int>> tfaces(nt), thalo(nt);
-    std::string terr;
-    std::mutex terr_lock;
+    }, 8192);
+    // What a tile's lists hold, in buffers of the worker that made them: its
+    // faces, halo and second-halo cells, the boundary faces of the halo's
+    // stencils, and its slot patterns
+    struct Lists {
+        std::vector<int> faces, halo, bc2;
+        std::vector<uint32_t> gslot;
+        std::vector<uint16_t> slots, nbrs;
+    };
+    struct Tile {
+        Lists *l;
+        size_t f, h, b, s, n;             // first entries: faces and gslot, halo, bc2, slots, nbrs
+        int nf, nif, nh, n2, nb, nn;      // faces, interior ones, halo, second halo, bc2, nbrs
+        uint64_t hash;
+    };
+    std::vector<Tile> tt(nt);
+    std::list<Lists> pool;
+    std::mutex pool_lock;
+    std::atomic<bool> fits{true};
     parallel_for(nt, [&](int t0, int t1) {
-        std::unordered_map<int, int> slot;
+        Lists *l;
+        {
+            std::lock_guard<std::mutex> lk(pool_lock);
+            pool.emplace_back();
+            l = &pool.back();
+        }
+        SlotMap slot;
+        std::vector<uint64_t> keys;
         for (int t = t0; t < t1; t++) {
-            std::vector<int> &faces = tfaces[t];
-            for (int i = d.tile_cell_start[t]; i < d.tile_cell_start[t + 1]; i++)
-                for (int k = 0; k < 6; k++) faces.push_back(g.gface[6 * (size_t)d.perm[i] + k]);
-            std::sort(faces.begin(), faces.end());
-            faces.erase(std::unique(faces.begin(), faces.end()), faces.end());
             const int c0 = d.tile_cell_start[t], c1 = d.tile_cell_start[t + 1], ntc = c1 - c0;
-            slot.clear();
-            std::vector<int> &halo = thalo[t];
-            auto visit = [&](int ic) {
-                if (ic >= c0 && ic < c1) return;
-                if (slot.emplace(ic, ntc + (int)halo.size()).second) halo.push_back(ic);
+            Tile &T = tt[t];
+            T.l = l;
+            T.f = l->faces.size(); T.h = l->halo.size(); T.b = l->bc2.size(); T.s = l->slots.size(); T.n = l->nbrs.size();
+            // each face once: from its owner, or its neighbour where the
+            // owner lies outside; by class, then in face order
+            keys.clear();
+            for (int i = c0; i < c1; i++)
+                for (int k = 0; k < 6; k++) {
+                    const size_t e = 6 * (size_t)d.perm[i] + k;
+                    const int f = g.gface[e];
+                    if (g.grole[e] != 0) {
+                        const int o = d.inv[g.owner[f]];
+                        if (o >= c0 && o < c1) continue;
+                    }
+                    keys.push_back((uint64_t)fclass[f] << 32 | (uint32_t)f);
+                }
+            std::sort(keys.begin(), keys.end());
+            T.nf = (int)keys.size();
+            for (uint64_t key : keys) l->faces.push_back((int)(uint32_t)key);
+            T.nif = (int)(std::lower_bound(keys.begin(), keys.end(), (uint64_t)2 << 32) - keys.begin());
+            auto face_index = [&](int f) {
+                return (int)(std::lower_bound(keys.begin(), keys.end(), (uint64_t)fclass[f] << 32 | (uint32_t)f) -
+                             keys.begin());
             };
-            for (int f : faces) {
-                visit(d.inv[g.owner[f]]);
-                if (g.nbr[f] < nc) visit(d.inv[g.nbr[f]]);
+            slot.reset(2 * keys.size());
+            auto visit = [&](int ic) {
+                if (ic >= c0 && ic < c1) return ic - c0;
+                bool added;
+                const int s = slot.get(ic, ntc + (int)(l->halo.size() - T.h), &added);
+                if (added) l->halo.push_back(ic);
+                return s;
+            };
+            for (uint64_t key : keys) {
+                const int f = (int)(uint32_t)key;
+                const uint32_t so = (uint32_t)visit(d.inv[g.owner[f]]);
+                l->gslot.push_back(so | (g.nbr[f] < nc ? (uint32_t)visit(d.inv[g.nbr[f]]) : 0xffffu) << 16);
             }
-            std::stable_partition(faces.begin(), faces.end(), [&](int f) { return face_class(f) == 0; });
-            std::stable_partition(faces.begin(), faces.end(), [&](int f) { return face_class(f) < 2; });
-            if ((int)faces.size() > 32767 || ntc + (int)halo.size() >= 0xffff) {
-                std::lock_guard<std::mutex> lk(terr_lock);
-                if (terr.empty())
-                    terr = (int)faces.size() > 32767 ? "tile has too many faces" : "tile and its halo exceed 65534 cells";
+            T.nh = (int)(l->halo.size() - T.h);
+            for (int i = c0; i < c1; i++)
+                for (int k = 0; k < 6; k++) {
+                    const size_t e = 6 * (size_t)d.perm[i] + k;
+                    l->slots.push_back((uint16_t)(face_index(g.gface[e]) | (g.grole[e] == 0 ? 0x8000 : 0)));
+                }
+            if (!fused_tile_fits(ntc + T.nh, T.nf)) fits = false;
+            for (int p = 0; p < ntc + T.nh && fits; p++) {
+                const int c = d.perm[p < ntc ? c0 + p : l->halo[T.h + p - ntc]];
+                for (int k = 0; k < 6; k++) {
+                    const int nb = g.gcell[6 * (size_t)c + k];
+                    int e;
+                    if (nb < nc) {
+                        e = visit(d.inv[nb]);
+                    } else {
+                        // the tile's own boundary faces end its list; those
+                        // of halo cells are appended
+                        const int f = g.gface[6 * (size_t)c + k], q = face_index(f);
+                        if (q < T.nf && (int)(uint32_t)keys[q] == f) {
+                            e = q - T.nif;
+                        } else {
+                            e = T.nf - T.nif + (int)(l->bc2.size() - T.b);
+                            l->bc2.push_back(nb - nc);
+                        }
+                        e |= 0x8000;
+                    }
+                    l->nbrs.push_back((uint16_t)e);
+                }
+            }
+            T.n2 = (int)(l->halo.size() - T.h) - T.nh;
+            T.nb = (int)(l->bc2.size() - T.b);
+            T.nn = (int)(l->nbrs.size() - T.n);
+            uint64_t h = (uint64_t)ntc << 32 | (uint32_t)T.nf;
+            auto mix = [&](const void *p, size_t bytes) {
+                const unsigned char *c = static_cast<const unsigned char *>(p);
+                for (; bytes >= 8; bytes -= 8, c += 8) {
+                    uint64_t v;
+                    std::memcpy(&v, c, 8);
+                    h = (h ^ v) * 0x9E3779B97F4A7C15ull;
+                    h ^= h >> 29;
+                }
+                for (; bytes > 0; bytes--) h = (h ^ *c++) * 0x9E3779B97F4A7C15ull;
+            };
+            mix(l->gslot.data() + T.f, 4 * (size_t)T.nf);
+            mix(l->slots.data() + T.s, 12 * (size_t)ntc);
+            mix(l->nbrs.data() + T.n, 2 * (size_t)T.nn);
+            T.hash = h;
+        }
+    }, 16);
+    // (the pass sizes its LDS for the largest tile's slots and faces)
+    d.max_tile_faces = d.max_grad_slots = d.max_slots = 0;
+    for (int t = 0; t < nt; t++) {
+        d.max_tile_faces = std::max(d.max_tile_faces, tt[t].nf);
+        d.max_grad_slots = std::max(d.max_grad_slots, d.tile_cell_start[t + 1] - d.tile_cell_start[t] + tt[t].nh);
+    }
+    d.fused_fits = fits && fused_tile_fits(d.max_grad_slots, d.max_tile_faces);
+    // tile records, and each pattern kept once (found by its hash, compared in
+    // full)
+    d.tile_face_start.assign(nt + 1, 0);
+    d.tiles.assign(nt, TileRec{});
+    d.face_gslot.clear();
+    d.cell_slots.clear();
+    d.cell_nbrs.clear();
+    std::unordered_multimap<uint64_t, int> seen;  // hash -> a tile holding the pattern
+    int n_halo = 0, n_tbc = 0;
+    d.n_slots = 0;
+    for (int t = 0; t < nt; t++) {
+        Tile &S = tt[t];
+        if (!d.fused_fits) S.n2 = S.nb = S.nn = 0;
+        TileRec &r = d.tiles[t];
+        r.c0 = d.tile_cell_start[t];
+        r.nc = d.tile_cell_start[t + 1] - r.c0;
+        r.f0 = d.tile_face_start[t];
+        r.nf = S.nf;
+        d.tile_face_start[t + 1] = r.f0 + r.nf;
+        r.h0 = n_halo;
+        r.nh = S.nh;
+        r.n2 = S.n2;
+        n_halo += r.nh + r.n2;
+        r.s0 = d.n_slots;
+        d.n_slots += r.nc + r.nh;
+        r.nif = S.nif;
+        r.b0 = n_tbc;
+        n_tbc += r.nf - r.nif + S.nb;
+        d.max_slots = std::max(d.max_slots, r.nc + r.nh + r.n2);
+        const uint32_t *gs = S.l->gslot.data() + S.f;
+        const uint16_t *sl = S.l->slots.data() + S.s, *nb = S.l->nbrs.data() + S.n;
+        bool found = false;
+        const auto range = seen.equal_range(S.hash);
+        for (auto it = range.first; it != range.second && !found; ++it) {
+            const TileRec &q = d.tiles[it->second];
+            found = q.nc == r.nc && q.nf == r.nf && q.nh == r.nh &&
+                    std::equal(gs, gs + r.nf, d.face_gslot.begin() + q.pf) &&
+                    std::equal(sl, sl + 6 * (size_t)r.nc, d.cell_slots.begin() + 6 * (size_t)q.pc) &&
+                    std::equal(nb, nb + S.nn, d.cell_nbrs.begin() + 6 * (size_t)q.pn);
+            if (found) {
+                r.pf = q.pf;
+                r.pc = q.pc;
+                r.pn = q.pn;
             }
         }
-    }, 4);
-    if (!terr.empty()) { err = terr; return LBFS_E_UNSUPPORTED; }
-    d.tile_face_start.assign(nt + 1, 0);
-    d.tile_halo_start.assign(nt + 1, 0);
-    d.tile_bface_start.assign(nt, 0);
-    d.max_tile_faces = 0;
-    d.max_grad_slots = 0;
-    for (int t = 0; t < nt; t++) {
-        const int nft = (int)tfaces[t].size(), ntc = d.tile_cell_start[t + 1] - d.tile_cell_start[t];
-        d.tile_face_start[t + 1] = d.tile_face_start[t] + nft;
-        d.tile_halo_start[t + 1] = d.tile_halo_start[t] + (int)thalo[t].size();
-        // boundary faces (ids from n_int) come last
-        d.tile_bface_start[t] = d.tile_face_start[t] +
-            (int)(std::partition_point(tfaces[t].begin(), tfaces[t].end(), [&](int f) { return f < g.n_int; }) -
-                  tfaces[t].begin());
-        d.max_tile_faces = std::max(d.max_tile_faces, nft);
-        d.max_grad_slots = std::max(d.max_grad_slots, ntc + (int)thalo[t].size());
+        if (found) continue;
+        r.pf = (int)d.face_gslot.size();
+        r.pc = (int)(d.cell_slots.size() / 6);
+        r.pn = (int)(d.cell_nbrs.size() / 6);
+        d.face_gslot.insert(d.face_gslot.end(), gs, gs + r.nf);
+        d.cell_slots.insert(d.cell_slots.end(), sl, sl + 6 * (size_t)r.nc);
+        d.cell_nbrs.insert(d.cell_nbrs.end(), nb, nb + S.nn);
+        seen.emplace(S.hash, t);
     }
     const size_t ntf = (size_t)d.tile_face_start[nt];
-    d.face_gslot.assign(ntf, 0u);
-    d.halo_ids.assign((size_t)d.tile_halo_start[nt], 0);
-    d.fA.assign(4 * ntf, 0.0f); d.fB.assign(4 * ntf, 0.0f); d.fC.assign(4 * ntf, 0.0f);
+    d.halo_ids.assign((size_t)n_halo, 0);
+    d.tile_bc.assign((size_t)n_tbc, 0);
+    d.fA.assign(4 * ntf, 0.0f); d.fB.assign(4 * ntf, 0.0f); d.fC.assign(2 * ntf, 0.0f);
     d.face_ref.assign(ntf, 0);
     parallel_for(nt, [&](int t0, int t1) {
-        std::unordered_map<int, int> slot;
         for (int t = t0; t < t1; t++) {
-            const std::vector<int> &faces = tfaces[t], &halo = thalo[t];
-            const int base = d.tile_face_start[t], c0 = d.tile_cell_start[t], c1 = d.tile_cell_start[t + 1];
-            const int ntc = c1 - c0;
-            slot.clear();
-            for (size_t h = 0; h < halo.size(); h++) slot.emplace(halo[h], ntc + (int)h);
-            std::copy(halo.begin(), halo.end(), d.halo_ids.begin() + d.tile_halo_start[t]);
-            auto gslot = [&](int ic) -> uint32_t {
-                if (ic >= c0 && ic < c1) return (uint32_t)(ic - c0);
-                return (uint32_t)slot.at(ic);
-            };
-            for (size_t q = 0; q < faces.size(); q++) {
+            const Tile &S = tt[t];
+            const TileRec &T = d.tiles[t];
+            const int *faces = S.l->faces.data() + S.f, *halo = S.l->halo.data() + S.h, *bc2 = S.l->bc2.data() + S.b;
+            std::copy(halo, halo + T.nh + T.n2, d.halo_ids.begin() + T.h0);
+            for (int q = T.nif; q < T.nf; q++) d.tile_bc[(size_t)T.b0 + q - T.nif] = faces[q] - g.n_int;
+            std::copy(bc2, bc2 + S.nb, d.tile_bc.begin() + T.b0 + T.nf - T.nif);
+            for (int q = 0; q < T.nf; q++) {
                 const int f = faces[q];
                 const int o = g.owner[f], n = g.nbr[f];
-                const uint32_t so = gslot(d.inv[o]), sn = n < nc ? gslot(d.inv[n]) : 0xffffu;
-                const size_t r = (size_t)base + q;
-                d.face_gslot[r] = so | (sn << 16);
+                const size_t r = (size_t)T.f0 + q;
                 const V3 xf = load3(&g.fc[3 * (size_t)f]);
                 const V3 d1 = load3(&g.cc[3 * (size_t)o]) - xf;
                 const V3 d2 = load3(&g.cc[3 * (size_t)n]) + load3(&g.shift[3 * (size_t)f]) - xf;
                 const double A = g.area[f];
-                const int on[2] = {d.inv[o], n < nc ? d.inv[n] : n};
-                float ob, nbb;
-                std::memcpy(&ob, &on[0], 4);
-                std::memcpy(&nbb, &on[1], 4);
                 const float a4[4] = {(float)(g.normal[3 * (size_t)f] * A), (float)(g.normal[3 * (size_t)f + 1] * A),
                                      (float)(g.normal[3 * (size_t)f + 2] * A),
-                                     std::copysign((float)g.fdt[f], face_class(f) ? -1.0f : 1.0f)};
-                const float b4[4] = {(float)d1.x, (float)d1.y, (float)d1.z, ob};
-                const float c4[4] = {(float)d2.x, (float)d2.y, (float)d2.z, nbb};
+                                     std::copysign((float)g.fdt[f], fclass[f] ? -1.0f : 1.0f)};
+                const float b4[4] = {(float)d1.x, (float)d1.y, (float)d1.z, (float)d2.x};
+                const float c2[2] = {(float)d2.y, (float)d2.z};
                 std::copy(a4, a4 + 4, d.fA.begin() + 4 * r);
                 std::copy(b4, b4 + 4, d.fB.begin() + 4 * r);
-                std::copy(c4, c4 + 4, d.fC.begin() + 4 * r);
+                std::copy(c2, c2 + 2, d.fC.begin() + 2 * r);
                 d.face_ref[r] = f;
             }
-            // each class is in face order
-            size_t cut[4] = {0, 0, 0, faces.size()};
-            for (int c = 1; c < 3; c++)
-                cut[c] = std::partition_point(faces.begin(), faces.end(), [&](int f) { return face_class(f) < c; }) -
-                         faces.begin();
-            for (int i = c0; i < c1; i++) {
-                const int c = d.perm[i];
-                for (int k = 0; k < 6; k++) {
-                    const int f = g.gface[6 * (size_t)c + k], q = face_class(f);
-                    const int sl = (int)(std::lower_bound(faces.begin() + cut[q], faces.begin() + cut[q + 1], f) -
-                                         faces.begin());
-                    const int own = g.grole[6 * (size_t)c + k] == 0 ? 0x8000 : 0;
-                    d.cell_slots[6 * (size_t)i + k] = (int16_t)(uint16_t)(sl | own);
-                }
-            }
         }
-    }, 4);
+    }, 16);
     d.face_first.assign(g.n_faces, -1);
     for (size_t r = 0; r < ntf; r++)
         if (d.face_first[d.face_ref[r]] < 0) d.face_first[d.face_ref[r]] = (int)r;

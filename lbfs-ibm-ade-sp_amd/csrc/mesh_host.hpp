@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "lbfs_abi.h"
+#include "tile_rec.hpp"
 
 namespace lbfs {
 
@@ -71,32 +72,38 @@ struct DeviceLayout {
     std::vector<int> perm;        // internal id -> caller id
     std::vector<int> inv;         // caller id -> internal id
     std::vector<int> tile_cell_start, tile_face_start;
-    std::vector<int> tile_bface_start;  // per tile: first boundary face (interior faces come first, those of
-                                        // the general reconstruction last among them)
+    std::vector<TileRec> tiles;   // interior faces come first in a tile's list, those of the general
+                                  // reconstruction last among them
     // per cell (internal order)
     std::vector<int> stencil;     // 6 * n, SoA [k*n + i]; ghost entries encoded -1 - bc
     std::vector<float> gw;        // 18 * n, SoA [(k*3+c)*n + i], W_k = LHS^-1 RHS_k
     std::vector<float> inv_vol;   // n
     std::vector<float> static_force; // 3 * n: body force + pressure closure defect of the cell
     std::vector<double> closure;  // 3 * n, caller order: sum of n A over the faces that carry flux
-    std::vector<int16_t> cell_slots; // 6 * n, AoS [i*6+k]: tile-local face slot, sign in bit 15 (1 = owner)
-    // per tile-face (duplicated across tiles)
-    // 48 B per face: the area-weighted normal (area = its length), the
-    // centroid offsets, and the owner and neighbour ids as int bits
+    // per tile-face (duplicated across tiles), 40 B per face
     std::vector<float> fA;        // 4 per face: normal * area xyz, face dt with the sign bit set where the
                                   // face takes the general reconstruction: boundary faces and faces
                                   // with a lattice direction within rounding of their plane (or of
                                   // the tie band), whose points may come from either side
-    std::vector<float> fB;        // 4 per face: owner centroid - face centroid, owner id
-    std::vector<float> fC;        // 4 per face: neighbour image centroid - face centroid, neighbour id
-                                  // (ghost: n_cells + bc)
-    // fused fluid pass: per tile the cells across its border that its faces
-    // reach (their gradients are computed into the tile's LDS after its own),
-    // and per tile-face the LDS gradient slots of owner and neighbour
-    // (tile cells first, then that halo; 0xffff for a ghost)
-    std::vector<int> tile_halo_start, halo_ids;
-    std::vector<uint32_t> face_gslot;
-    int max_grad_slots = 0;
+    std::vector<float> fB;        // 4 per face: owner centroid - face centroid xyz, neighbour image
+                                  // centroid - face centroid x
+    std::vector<float> fC;        // 2 per face: neighbour image centroid - face centroid yz
+    // Cells are addressed within a tile by slots: its own cells in order, the
+    // halo its faces reach, and the second halo the halo's gradients reach.
+    // The slot lists of a tile (its patterns) depend only on how its cells and
+    // faces join, so tiles alike share one copy and read it from cache: 60 B
+    // a cell of indices the tiles would otherwise stream.
+    std::vector<uint32_t> face_gslot;  // per pattern face: owner slot | neighbour slot << 16 (0xffff: the
+                                       // face is a boundary face)
+    std::vector<uint16_t> cell_slots;  // 6 per pattern cell: tile-local face index, bit 15: the cell owns it
+    std::vector<uint16_t> cell_nbrs;   // 6 per pattern gradient slot (tile and halo): slot of the gradient
+                                       // stencil's cell, or bit 15 and an entry of the tile's boundary ids
+    std::vector<int> halo_ids;         // per tile the ids of its halo and second-halo cells
+    std::vector<int> tile_bc;          // per tile the ids of its boundary faces, then of its halo cells'
+    int n_slots = 0;                   // gradient slots of all tiles
+    bool fused_fits = true;            // every tile fits the fused fluid pass (else no tile has a second
+                                       // halo or a gradient pattern, which only that pass reads)
+    int max_grad_slots = 0, max_slots = 0;  // largest tile and halo, and with the second halo
     std::vector<int> face_ref;    // caller face id of each tile-face
     std::vector<int> face_first;  // caller face id -> one tile-face holding it
     // boundary faces
