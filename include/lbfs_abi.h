@@ -127,9 +127,10 @@ typedef struct {
     int time_stepping;  /* LBFS_TS_*; 0 = constant dt */
     double max_velocity;/* U of the CFL estimate (LBFS_TS_LOCAL / LBFS_TS_MIN) */
     int tile[3];        /* cells per tile along x, y, z of the logical grid (no counterpart in the
-                           reference); 0 0 0 = 8 8 4.  Results do not depend on it. */
-    int block_threads;  /* workgroup size of the fluid kernels: 0 (= 256), 256, 512 or 576 (three faces per
-                           thread on 8x8x8 tiles: 1728 faces) */
+                           reference); 0 0 0 = by the mesh's size (8x8x8 to 4x4x4).  Results do not
+                           depend on it. */
+    int block_threads;  /* workgroup size of the fluid kernels: 0 (= 256, or the size that goes with tile 0 0 0),
+                           256, 512 or 576 */
 } lbfs_params;
 
 /* time stepping (gpu_time_stepping, Solver_gpu.cu:767-790; get_cfl_device

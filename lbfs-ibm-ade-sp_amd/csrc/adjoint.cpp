@@ -332,7 +332,7 @@ hipError_t replay_fluid(const lbfs_ctx *ctx, FluidArgs a, StepRec &r, const floa
                         hipStream_t s)
 {
     a.face_moments = r.mom;
-    if (ctx->fused && ctx->fused_ok && a.ts_mode != LBFS_TS_MIN) {
+    if (ctx->fused && ctx->fused_ok) {
         a.grad_out = r.grad;
         return launch_fluid_fused(a, st, st_next, r.res, 1, s);
     }

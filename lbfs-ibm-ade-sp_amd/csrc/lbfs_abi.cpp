@@ -54,6 +54,35 @@ extern "C" const char *lbfs_last_error(const lbfs_ctx *ctx)
     return ctx->err.c_str();
 }
 
+// The tile and workgroup size a caller leaves open.  A tile costs its halo's
+// gradients and its border faces again (8x8x8: 1.75 gradients and 3.4 faces a
+// cell, 8x4x4: 2.25 and 3.6, 4x4x4: 2.5 and 3.75), a small mesh the time of one
+// workgroup, so 8x8x8 tiles of 512 threads (two workgroups a compute unit) are
+// taken from 1000 tiles on, about two rounds of the chip: measured per plain
+// D3Q19 step 128x64x64 (1024 tiles) 38.3 us against 43.1 with 8x4x4, 192x96x96
+// 147 against 165, but 96x64x48 (576) 29.5 against 28.9 and 45x22x22 (54) 12.5
+// against 8.7.  Below 200 tiles of 8x4x4 the 4x4x4 ones are as fast or faster:
+// 24x16x16 (48) 7.4 against 9.5 us, 45x22x22 (216) 8.6 against 8.7, 70x33x29
+// (648) 14.1 against 11.7.  One layer of cells keeps 8x8 tiles of 256 threads
+// (64x64: 5.3 us, 16x16 9.5), and meshes without a logical structure runs of
+// 256 cells.
+static void default_tile(const std::vector<HostBlock> &blocks, int tile[3], int &threads)
+{
+    if (blocks.empty()) return;
+    auto tiles = [&](int tx, int ty, int tz) {
+        long long n = 0;
+        for (const HostBlock &b : blocks)
+            n += (long long)((b.n[0] + tx - 1) / tx) * ((b.n[1] + ty - 1) / ty) * ((b.n[2] + tz - 1) / tz);
+        return n;
+    };
+    for (const HostBlock &b : blocks)
+        if (b.n[0] == 1 || b.n[1] == 1 || b.n[2] == 1) return;
+    const bool large = tiles(8, 8, 8) >= 1000;
+    tile[0] = large || tiles(8, 4, 4) >= 200 ? 8 : 4;
+    tile[1] = tile[2] = large ? 8 : 4;
+    threads = large ? 512 : 256;
+}
+
 static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params &p)
 {
     std::string err;
@@ -81,6 +110,8 @@ static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params
             return ctx->fail(LBFS_E_INVALID_ARG, "tile %dx%dx%d: each side >= 1, at most 2048 cells", p.tile[0],
                              p.tile[1], p.tile[2]);
         for (int t = 0; t < 3; t++) tile[t] = p.tile[t];
+    } else {
+        default_tile(ctx->blocks, tile, threads);
     }
     if (p.block_threads) threads = p.block_threads;
     rc = build_layout(m, ctx->geo, lhs, rhs, p.rho0, p.body_force, p.lattice, (p.flags & LBFS_FLAG_UPWIND_BAND) != 0,

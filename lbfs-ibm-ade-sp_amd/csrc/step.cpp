@@ -77,7 +77,7 @@ std::vector<lbfs_ctx::Stage> lbfs_ctx::step_stages(bool with_visc, bool fused_fl
                      },
                      288.0 * nn + cell_bytes * touched + (gather_forces ? node_force_bytes : 0.0)});
     }
-    const bool fused = fused_fluid && fused_ok && args.ts_mode != LBFS_TS_MIN;
+    const bool fused = fused_fluid && fused_ok;
     if (args.ts_mode == LBFS_TS_MIN)
         s.push_back({"dt_min", [ctx]() -> int {
                          HIPCHK(launch_dt_min(ctx->args, ctx->st[ctx->cur], ctx->stream));
@@ -150,7 +150,7 @@ std::vector<lbfs_ctx::Stage> lbfs_ctx::step_stages(bool with_visc, bool fused_fl
 int lbfs_ctx::run_stages(bool with_visc)
 {
     lbfs_ctx *ctx = this;
-    const bool fz = fused && fused_ok && args.ts_mode != LBFS_TS_MIN;
+    const bool fz = fused && fused_ok;
     if (!have_membranes || !side || with_visc) {
         // (the internal viscosity field feeds the face pass: in the steps
         // that rebuild it, everything runs in order on one stream)
