@@ -555,14 +555,11 @@ extern "C" int lbfs_adjoint_backward(lbfs_ctx *ctx, const double *lam_nodes, con
     // seeds: adjoints of the final state and node positions, cleared sums;
     // all on the context's stream (it does not wait for the null stream)
     {
-        std::vector<float4> h(n, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
-        if (lam_state)
-            for (int i = 0; i < n; i++) {
-                const int c = ctx->lay.perm[i];
-                h[i] = make_float4((float)lam_state[4 * (size_t)c], (float)lam_state[4 * (size_t)c + 1],
-                                   (float)lam_state[4 * (size_t)c + 2], (float)lam_state[4 * (size_t)c + 3]);
-            }
-        HIPCHK(hipMemcpyAsync(A.lam_st[0], h.data(), sizeof(float4) * n, hipMemcpyHostToDevice, ctx->stream));
+        if (lam_state) {
+            if ((rc = write_cells(ctx, lam_state, A.lam_st[0]))) return rc;
+        } else {
+            HIPCHK(hipMemsetAsync(A.lam_st[0], 0, sizeof(float4) * n, ctx->stream));
+        }
         HIPCHK(hipMemsetAsync(A.gforce, 0, 3 * sizeof(double), ctx->stream));
         HIPCHK(hipMemsetAsync(A.fpart, 0, 3 * sizeof(double) * A.n_fpart, ctx->stream));
         HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -646,15 +643,8 @@ extern "C" int lbfs_adjoint_backward(lbfs_ctx *ctx, const double *lam_nodes, con
         }
     }
     if (lam_state0) {
-        std::vector<float4> h(n);
-        HIPCHK(hipMemcpy(h.data(), A.lam_st[cur_l], sizeof(float4) * n, hipMemcpyDeviceToHost));
-        for (int i = 0; i < n; i++) {
-            const int c = ctx->lay.perm[i];
-            lam_state0[4 * (size_t)c] = h[i].x;
-            lam_state0[4 * (size_t)c + 1] = h[i].y;
-            lam_state0[4 * (size_t)c + 2] = h[i].z;
-            lam_state0[4 * (size_t)c + 3] = h[i].w;
-        }
+        CellArrays out{{nullptr, nullptr, nullptr, nullptr}, lam_state0};
+        if ((rc = read_cells(ctx, A.lam_st[cur_l], 0.0, out))) return rc;
     }
     if (lam_nodes0) {
         const int nn = ctx->mem.n_nodes;

@@ -12,6 +12,7 @@
 #include "fluid_kernels.hpp"
 #include "lbfs_abi.h"
 #include "mesh_host.hpp"
+#include "transfer.hpp"
 
 namespace lbfs {
 struct AdjointState;  // adjoint.cpp
@@ -41,6 +42,8 @@ struct lbfs_ctx {
                                     // the next lbfs_add_membranes
     float *static_force = nullptr;  // [3 n] body force + closure term
     float *cell_force = nullptr;    // [3 n] static force + spread IBM force
+    int *cell_inv = nullptr;        // [n] internal id of each caller cell
+    lbfs::Staging staging;          // pinned buffers of the host transfers
     std::vector<void *> allocs;
 
     // membranes and IBM coupling (lbfs_add_membranes)
@@ -51,7 +54,6 @@ struct lbfs_ctx {
     double *mem_energy = nullptr;   // [7 n_mem] output of lbfs_get_membrane_energies
     double *energy_scratch = nullptr; // this device's static staging of lbfs_get_membrane_energies_noalloc
     int ibm_binned_option = -1;     // LBFS_OPT_IBM_BINNED: -1 by node density, else IBM_SPREAD_*
-    std::vector<double> mem_origin;
     // host copies behind lbfs_set_membrane_moduli: per-membrane parameters,
     // per-edge spring constant per unit shear modulus (FP64), edge ranges
     std::vector<lbfs::MemParamDev> mem_params;

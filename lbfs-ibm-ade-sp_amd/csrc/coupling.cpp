@@ -191,12 +191,6 @@ extern "C" int lbfs_add_membranes(lbfs_ctx *ctx, const lbfs_membrane_desc *mem, 
             ctx->mem_ks_unit[mem_edge_start[i] + e] =
                 mem[i].shear_modulus != 0.0 ? ms[i].spring_constant[e] / mem[i].shear_modulus : 0.0;
     }
-    ctx->mem_origin.assign(3 * (size_t)count, 0.0);
-    for (int i = 0; i < count; i++) {
-        ctx->mem_origin[3 * (size_t)i] = origin[i].x;
-        ctx->mem_origin[3 * (size_t)i + 1] = origin[i].y;
-        ctx->mem_origin[3 * (size_t)i + 2] = origin[i].z;
-    }
     // IBM grids: one per logical box, bins (= spreading tiles) numbered box after box
     IbmArgs &g = ctx->ibm;
     memset(&g, 0, sizeof(g));
@@ -351,7 +345,7 @@ extern "C" int lbfs_add_membranes(lbfs_ctx *ctx, const lbfs_membrane_desc *mem, 
     float *dssc;
     if ((rc = cp_alloc(ctx, &dssc, ssc.data(), ssc.size()))) return rc;
     g.spread_sc = dssc;
-    int *dinv, *tcount, *slots, *ov, *nov;
+    int *tcount, *slots, *ov, *nov;
     float4 *dcen;
     float *wn, *sf;
     int4 *nbs;
@@ -364,7 +358,6 @@ extern "C" int lbfs_add_membranes(lbfs_ctx *ctx, const lbfs_membrane_desc *mem, 
     if ((rc = cp_alloc<int>(ctx, &nblist, nullptr, 1))) return rc;
     g.bin_list = blist;
     g.n_bin_list = nblist;
-    if ((rc = cp_alloc(ctx, &dinv, ctx->lay.inv.data(), nc))) return rc;
     if ((rc = cp_alloc(ctx, &dcen, cen.data(), nc))) return rc;
     if ((rc = cp_alloc<int>(ctx, &tcount, nullptr, g.n_tiles))) return rc;
     if ((rc = cp_alloc<int>(ctx, &slots, nullptr, (size_t)g.tile_cap * g.n_tiles))) return rc;
@@ -377,7 +370,7 @@ extern "C" int lbfs_add_membranes(lbfs_ctx *ctx, const lbfs_membrane_desc *mem, 
     g.spread_f = sf;
     if ((rc = cp_alloc<float>(ctx, &wn, nullptr, 64 * (size_t)nn))) return rc;
     if ((rc = cp_alloc<int4>(ctx, &nbs, nullptr, nn))) return rc;
-    g.inv = dinv; g.cen = dcen; g.tile_count = tcount; g.tile_slots = slots; g.overflow = ov; g.n_overflow = nov;
+    g.inv = ctx->cell_inv; g.cen = dcen; g.tile_count = tcount; g.tile_slots = slots; g.overflow = ov; g.n_overflow = nov;
     g.wnode = wn; g.nbase = nbs;
     g.static_force = ctx->static_force;
     g.cell_force = ctx->cell_force;
@@ -437,22 +430,7 @@ extern "C" int lbfs_get_membrane_nodes(lbfs_ctx *ctx, double *X, double *U, doub
     if (!ctx->have_membranes) return ctx->fail(LBFS_E_STATE, "no membranes attached");
     int rc = ctx->check_device_error();
     if (rc) return rc;
-    const int nn = ctx->mem.n_nodes;
-    std::vector<float4> hx(nn), hu(nn), hf(nn);
-    std::vector<int> nm(nn);
-    HIPCHK(hipMemcpyAsync(hx.data(), ctx->mem.X, sizeof(float4) * nn, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipMemcpyAsync(hu.data(), ctx->mem.U, sizeof(float4) * nn, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipMemcpyAsync(hf.data(), ctx->mem.F, sizeof(float4) * nn, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    int mi = 0;
-    for (int n = 0; n < nn; n++) {
-        while (n >= ctx->mem_node_start[mi + 1]) mi++;
-        const double *o = &ctx->mem_origin[3 * (size_t)mi];
-        if (X) { X[3 * (size_t)n] = o[0] + hx[n].x; X[3 * (size_t)n + 1] = o[1] + hx[n].y; X[3 * (size_t)n + 2] = o[2] + hx[n].z; }
-        if (U) { U[3 * (size_t)n] = hu[n].x; U[3 * (size_t)n + 1] = hu[n].y; U[3 * (size_t)n + 2] = hu[n].z; }
-        if (F) { F[3 * (size_t)n] = hf[n].x; F[3 * (size_t)n + 1] = hf[n].y; F[3 * (size_t)n + 2] = hf[n].z; }
-    }
-    return LBFS_OK;
+    return read_nodes(ctx, X, U, F);
 }
 
 extern "C" int lbfs_get_membrane_globals(lbfs_ctx *ctx, double *out6)

@@ -148,6 +148,7 @@ static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params
     if ((rc = dev_upload(ctx, &stencil, d.stencil.data(), d.stencil.size()))) return rc;
     if ((rc = dev_upload(ctx, &gw, d.gw.data(), d.gw.size()))) return rc;
     if ((rc = dev_upload(ctx, &inv_vol, d.inv_vol.data(), d.inv_vol.size()))) return rc;
+    if ((rc = dev_upload(ctx, &ctx->cell_inv, d.inv.data(), d.inv.size()))) return rc;
     if ((rc = dev_upload(ctx, &tcs, d.tile_cell_start.data(), d.tile_cell_start.size()))) return rc;
     {
         TileRec *tiles;
@@ -338,6 +339,7 @@ extern "C" int lbfs_destroy(lbfs_ctx *ctx)
     ctx->release_extensions();
     for (void *p : ctx->allocs) hipFree(p);
     ctx->allocs.clear();
+    ctx->staging.release();
     if (ctx->side) (void)hipStreamSynchronize(ctx->side);
     if (ctx->side2) (void)hipStreamSynchronize(ctx->side2);
     if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
@@ -393,16 +395,8 @@ extern "C" int lbfs_set_state(lbfs_ctx *ctx, const double *rho, const double *u,
 extern "C" int lbfs_get_state(lbfs_ctx *ctx, double *rho, double *u, double *v, double *w)
 {
     if (!ctx || !rho || !u || !v || !w) return LBFS_E_INVALID_ARG;
-    const int n = ctx->lay.n_cells;
-    std::vector<float4> h(n);
-    HIPCHK(hipMemcpyAsync(h.data(), ctx->st[ctx->cur], sizeof(float4) * n, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    for (int i = 0; i < n; i++) {
-        const int c = ctx->lay.perm[i];
-        rho[c] = ctx->params.rho0 + (double)h[i].x;
-        u[c] = h[i].y; v[c] = h[i].z; w[c] = h[i].w;
-    }
-    return LBFS_OK;
+    CellArrays out{{rho, u, v, w}, nullptr};
+    return read_cells(ctx, ctx->st[ctx->cur], ctx->params.rho0, out);
 }
 
 void lbfs_ctx::drop_graph()
