@@ -495,10 +495,13 @@ extern "C" int lbfs_adjoint_forward(lbfs_ctx *ctx, int n_steps, int checkpoint_e
     if ((rc = save(ctx, A.ckpt[0]))) return rc;
     // the steps before the last segment, checkpointed every K steps
     const int n_seg = (n_steps + every - 1) / every, s_last = (n_seg - 1) * every;
-    for (int t = 0; t < s_last; t++) {
-        if ((rc = ctx->enqueue_step())) return rc;
-        if ((t + 1) % every == 0)
-            if ((rc = save(ctx, A.ckpt[(t + 1) / every]))) return rc;
+    // (a short run does not make up for capturing a graph)
+    const bool graphs = s_last >= 32;
+    for (int t = 0; t < s_last; t += every) {
+        for (int q = 0; !graphs && q < every; q++)
+            if ((rc = ctx->enqueue_step())) return rc;
+        if (graphs && (rc = ctx->enqueue_steps(every))) return rc;
+        if ((rc = save(ctx, A.ckpt[t / every + 1]))) return rc;
     }
     // the last segment straight into the step records (the same kernels on
     // the same inputs), so the backward pass starts without replaying it;

@@ -71,12 +71,19 @@ struct lbfs_ctx {
     // checkpoints and buffers of the discrete adjoint (lbfs_adjoint_*)
     lbfs::AdjointState *adj = nullptr;
 
-    // hipGraph of two consecutive steps starting from cur == 0
+    // hipGraphs of graph_steps(k) consecutive steps (even numbers) starting from
+    // cur == 0, captured when a run first has that many (8 coupled steps hold
+    // some 60 launches, whose capture a first run pays for).  A graph launch costs the
+    // host 16 us and the device a gap of 3-5 us however many steps it holds: per
+    // step of 64x64 cells 8.0 us in graphs of two, 5.7 of 8, 5.2 of 32, and 5.9
+    // launched one by one; of 128x64x64 40.6, 39.1 and 38.9, with its cell (six
+    // launches on two streams) 62.6, 61.8 and 61.8.
+    int graph_steps(int k) const { return k == 1 ? 2 : (have_membranes ? 8 : 32); }
     int schedule_option = 0;        // LBFS_OPT_STEP_SCHEDULE
     bool fused_ok = false;          // the tiles fit the fused fluid pass's LDS
     bool fused = false;             // LBFS_OPT_FUSED_FLUID: whole steps run the fused fluid pass
     bool use_graph = true;
-    hipGraphExec_t graph_exec = nullptr;
+    hipGraphExec_t graph_exec[2] = {nullptr, nullptr};
     void drop_graph();
     // arguments of the apply pass that ends a coupled step
     lbfs::ApplyArgs apply_args(float4 *st_new, float *cell_force_out, int all) const

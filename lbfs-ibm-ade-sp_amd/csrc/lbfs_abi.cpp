@@ -401,27 +401,29 @@ extern "C" int lbfs_get_state(lbfs_ctx *ctx, double *rho, double *u, double *v, 
 
 void lbfs_ctx::drop_graph()
 {
-    if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
-    graph_exec = nullptr;
+    for (hipGraphExec_t &g : graph_exec) {
+        if (g) (void)hipGraphExecDestroy(g);
+        g = nullptr;
+    }
 }
 
-// capture two consecutive steps (state ping-pong back to buffer 0) into a graph
-static int capture_graph(lbfs_ctx *ctx)
+// capture graph k: its steps, an even number (state ping-pong back to buffer 0)
+static int capture_graph(lbfs_ctx *ctx, int k)
 {
     hipGraph_t g = nullptr;
     HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-    int rc = ctx->run_stages(false);
-    if (!rc) rc = ctx->run_stages(false);
+    int rc = LBFS_OK;
+    for (int q = 0; q < ctx->graph_steps(k) && !rc; q++) rc = ctx->run_stages(false);
     hipError_t e = hipStreamEndCapture(ctx->stream, &g);
     if (rc) {
         if (g) (void)hipGraphDestroy(g);
         return rc;
     }
     if (e != hipSuccess) return ctx->fail(LBFS_E_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
-    e = hipGraphInstantiate(&ctx->graph_exec, g, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(&ctx->graph_exec[k], g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     if (e != hipSuccess) {
-        ctx->graph_exec = nullptr;
+        ctx->graph_exec[k] = nullptr;
         return ctx->fail(LBFS_E_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e));
     }
     return LBFS_OK;
@@ -437,29 +439,37 @@ int lbfs_ctx::enqueue_steps(int nsteps)
             if (rc) return rc;
             s++;
         }
-        if (!graph_exec) {
-            const int saved = cur;
-            int rc = capture_graph(this);
-            cur = saved;  // capture only recorded the launches
-            if (rc) return rc;
-        }
-        // graph pairs, falling back to single eager steps where the internal
-        // viscosity field is due
-        while (s + 2 <= nsteps) {
-            if (visc_due(t_step) || visc_due(t_step + 1)) {
-                int rc = enqueue_step();
-                if (rc) return rc;
-                s++;
-                if (cur != 0) {
-                    rc = enqueue_step();
+        for (int k = 0; k < 2; k++) {
+            // graphs of this many steps, falling back to single eager steps
+            // where the internal viscosity field is due
+            const int gs = graph_steps(k);
+            while (s + gs <= nsteps) {
+                bool due = false;
+                for (int q = 0; q < gs; q++) due |= visc_due(t_step + q);
+                if (due) {
+                    int rc = enqueue_step();
                     if (rc) return rc;
                     s++;
+                    if (cur != 0) {
+                        rc = enqueue_step();
+                        if (rc) return rc;
+                        s++;
+                    }
+                    continue;
                 }
-                continue;
+                if (!graph_exec[k]) {
+                    const int saved = cur;
+                    int rc = capture_graph(this, k);
+                    cur = saved;  // capture only recorded the launches
+                    if (rc) return rc;
+                }
+                HIPCHK(hipGraphLaunch(graph_exec[k], stream));
+                t_step += gs;
+                s += gs;
             }
-            HIPCHK(hipGraphLaunch(graph_exec, stream));
-            t_step += 2;
-            s += 2;
+            // (one launch a step: the rest of a run is as fast launched one by
+            // one as in pairs)
+            if (!have_membranes && args.ts_mode != LBFS_TS_MIN) break;
         }
     }
     for (; s < nsteps; s++) {
