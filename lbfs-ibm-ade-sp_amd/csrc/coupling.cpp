@@ -208,7 +208,7 @@ extern "C" int lbfs_add_membranes(lbfs_ctx *ctx, const lbfs_membrane_desc *mem, 
     const int nc0 = ctx->lay.n_cells;
     if (ctx->ibm_binned_option >= 0) g.binned = ctx->ibm_binned_option;
     else g.binned = (double)nn >= 0.01 * nc0 ? IBM_SPREAD_GATHER : IBM_SPREAD_BINS;
-    if (g.binned == IBM_SPREAD_GATHER && spread_tile_lds(ctx->args.max_tile_cells) > 150 * 1024)
+    if (g.binned == IBM_SPREAD_GATHER && spread_tile_lds(512, ctx->args.max_tile_cells) > 150 * 1024)
         g.binned = IBM_SPREAD_BINS;  // tiles beyond the LDS budget
     const int nblk = (int)ctx->blocks.size();
     std::vector<IbmBlock> blk(nblk);
@@ -261,6 +261,11 @@ extern "C" int lbfs_add_membranes(lbfs_ctx *ctx, const lbfs_membrane_desc *mem, 
                 B.per[a] = 1;
                 B.L[a] = (float)std::fabs(ctx->geo.shift[3 * (size_t)f + a]);
             }
+    bool one_image = true;
+    for (const IbmBlock &B : blk)
+        for (int a = 0; a < 3; a++)
+            one_image &= !B.per[a] || B.n[a] >= std::min(B.tw[a], B.n[a]) + 3;  // stencils of up to 4 cells
+    g.spread_nt = spread_threads((int)tile_lo.size(), one_image);
     for (IbmBlock &B : blk)
         for (int a = 0; a < 3; a++) B.period_step[a] = B.L[a] / (float)B.n[a];
     // 4-point Lagrange kernel: per box and axis the vertex planes along the

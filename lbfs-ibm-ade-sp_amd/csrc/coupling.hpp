@@ -86,6 +86,7 @@ struct IbmArgs {
     const int *tile_cell_start;  // [n_tiles + 1] internal cell ids of each tile (tile gathering: the
                               // node-list tiles are the fluid tiles)
     int max_tile_cells;
+    int spread_nt;            // threads of the tile spreading
     int *bin_list, *n_bin_list;  // bin scattering: the tiles holding nodes this step (the count is
                               // cleared by the apply pass)
     const int *node_block;    // [n_nodes] box of each node
@@ -139,11 +140,19 @@ struct ApplyArgs {
     int n_mem;
 };
 
-// threads of the tile spreading, also the candidate nodes it tests at a time
-constexpr int SPREAD_NT = 512;
-// LDS of the tile spreading: the staged candidate nodes (base 16 B, force
-// 16 B, id 4 B), then three 64-bit sums per tile cell
-inline size_t spread_tile_lds(int max_tile_cells) { return (size_t)SPREAD_NT * 36 + (size_t)max_tile_cells * 24; }
+// Threads of the tile spreading, also the candidate nodes it tests at a time.
+// Many tiles keep every compute unit at its limit of workgroups, where smaller
+// ones wait less for their slowest wavefront: 8192 tiles (380k nodes) 142 us with
+// 256 threads, 172 with 512; 1024 tiles (48k nodes) 36 and 33, the densest tile
+// alone setting the time.  The smaller ones take boxes where a tile sees a node
+// once (the code for more images costs them 10 us by its registers).
+inline int spread_threads(int n_tiles, bool one_image) { return n_tiles >= 4096 && one_image ? 256 : 512; }
+// its LDS: the staged candidate nodes (base 16 B, force 16 B, id 4 B), then
+// three 64-bit sums per tile cell
+inline size_t spread_tile_lds(int threads, int max_tile_cells)
+{
+    return (size_t)threads * 36 + (size_t)max_tile_cells * 24;
+}
 
 hipError_t launch_ibm_interp(const MemArgs &m, const IbmArgs &g, const float4 *st, hipStream_t s);
 // weights and tiles of the current node positions (after attaching membranes

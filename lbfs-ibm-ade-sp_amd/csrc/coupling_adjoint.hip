@@ -71,6 +71,7 @@ __device__ __forceinline__ void weight_term(float wh, const float dw[3], float i
 // ---------------------------------------------------------------------------
 // spreading: f_c = static_c + (1 / V_c) sum_n w_nc F_n
 // ---------------------------------------------------------------------------
+template <bool ONE>
 __global__ __launch_bounds__(256) void k_adj_spread(MemArgs m, IbmArgs g, AdjMemArgs j)
 {
     const int lane = threadIdx.x & 63;
@@ -79,7 +80,7 @@ __global__ __launch_bounds__(256) void k_adj_spread(MemArgs m, IbmArgs g, AdjMem
     // previous step's readers ran before this kernel on the same stream)
     if (blockIdx.x == 0 && threadIdx.x == 0) *j.umax = 0u;
     if (nd >= m.n_nodes) return;
-    const IbmBlock B = node_block(g, nd);
+    const IbmBlock B = node_block<ONE>(g, nd);
     const float4 o = m.origin[m.node_mem[nd]], xl = m.X[nd];
     const float P[3] = {o.x + xl.x, o.y + xl.y, o.z + xl.z};
     float wh, dw[3];
@@ -351,12 +352,13 @@ __global__ __launch_bounds__(256) void k_adj_mem_nodes(MemArgs m, IbmArgs g, Adj
 // ---------------------------------------------------------------------------
 // interpolation: U_n = sum_c w_nc(X^n) u_c
 // ---------------------------------------------------------------------------
+template <bool ONE>
 __global__ __launch_bounds__(256) void k_adj_interp(MemArgs m, IbmArgs g, AdjMemArgs j)
 {
     const int lane = threadIdx.x & 63;
     const int nd = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (nd >= m.n_nodes) return;
-    const IbmBlock B = node_block(g, nd);
+    const IbmBlock B = node_block<ONE>(g, nd);
     const float4 o = m.origin[m.node_mem[nd]], xl = j.Xn[nd];
     const float P[3] = {o.x + xl.x, o.y + xl.y, o.z + xl.z};
     float wh, dw[3];
@@ -388,13 +390,15 @@ __global__ __launch_bounds__(256) void k_adj_interp(MemArgs m, IbmArgs g, AdjMem
 hipError_t launch_adj_coupling(const MemArgs &m, const IbmArgs &g, const AdjMemArgs &j, hipStream_t s)
 {
     const int nb4 = (m.n_nodes + 3) / 4;
-    hipLaunchKernelGGL(k_adj_spread, dim3(nb4), dim3(256), 0, s, m, g, j);
+    if (g.n_blocks == 1) hipLaunchKernelGGL(k_adj_spread<true>, dim3(nb4), dim3(256), 0, s, m, g, j);
+    else hipLaunchKernelGGL(k_adj_spread<false>, dim3(nb4), dim3(256), 0, s, m, g, j);
     hipLaunchKernelGGL(k_adj_mem_edges, dim3((24 * m.n_edges + 255) / 256), dim3(256), 0, s, m, j);
     hipLaunchKernelGGL(k_adj_mem_partials, dim3(j.n_echunks), dim3(256), 0, s, m, j);
     hipLaunchKernelGGL(k_adj_mem_coef, dim3((ADJ_COEF_LANES * m.n_edges + ADJ_COEF_NT - 1) / ADJ_COEF_NT),
                        dim3(ADJ_COEF_NT), 0, s, m, j);
     hipLaunchKernelGGL(k_adj_mem_nodes, dim3((8 * m.n_nodes + 255) / 256), dim3(256), 0, s, m, g, j);
-    hipLaunchKernelGGL(k_adj_interp, dim3(nb4), dim3(256), 0, s, m, g, j);
+    if (g.n_blocks == 1) hipLaunchKernelGGL(k_adj_interp<true>, dim3(nb4), dim3(256), 0, s, m, g, j);
+    else hipLaunchKernelGGL(k_adj_interp<false>, dim3(nb4), dim3(256), 0, s, m, g, j);
     return hipGetLastError();
 }
 

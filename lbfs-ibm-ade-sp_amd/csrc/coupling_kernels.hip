@@ -135,54 +135,60 @@ __device__ __forceinline__ float group_sum(float v)
     return v;
 }
 
-// Per node, S x S lanes, lane (j, k) taking the S cells of stencil row (j, k).
+// Per node, S x S lanes, lane (i, j) taking the S cells of stencil column
+// (i, j): with x fastest in the tile order, a load of the wavefront then touches
+// the S cells of a row in one cache line (rows by lane instead, each lane its own
+// line: 173 -> 128 us for the 380k nodes of a 256x128x128 suspension; the
+// latency of these scattered loads bounds it, its bytes take 50 us).
 // INTERP: the fluid velocity at the node from its kept weights
 // (immersed_boundary_method.cu:14-97, or the 4-point kernels) and the
 // advection X += U dt (immersed_boundary_method.cu:234-264).  Always: the
 // weights of the (new) position, normalised for the cosine kernel, kept with
 // the stencil base and its fluid tile; INTERP also lists the node in that
 // tile for the spreading.
-template <int K, bool INTERP>
+template <int K, bool ONE, bool INTERP>
 __global__ __launch_bounds__(256) void k_ibm_interp(MemArgs m, IbmArgs g, const float4 *__restrict__ st)
 {
     constexpr int S = Stencil<K>::S, L = S * S;
     // consecutive nodes (neighbours on a membrane) on one XCD share its L2
     const int gid = xcd_remap(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    const int r = gid % L, j = r % S, k = r / S;
+    const int r = gid % L, i = r % S, j = r / S;
     const bool live = gid / L < m.n_nodes;
     const int nd = live ? gid / L : m.n_nodes - 1;  // dead lanes shadow a live node for the group sums
-    const IbmBlock B = node_block(g, nd);
+    const IbmBlock B = node_block<ONE>(g, nd);
     const float4 o = m.node_origin[nd];
     float4 xl = m.X[nd];
-    float *row = g.wnode + 64 * (size_t)nd + S * r;  // this lane's S weights
+    float *col = g.wnode + 64 * (size_t)nd + r;  // this lane's S weights, L apart
     if constexpr (INTERP) {
         const int4 nb = g.nbase[nd];
         float ux = 0.0f, uy = 0.0f, uz = 0.0f;
-        int w[3] = {0, 0, 0};
-        const bool rowok = wrap_index(B, 1, nb.y + j, w[1]) && wrap_index(B, 2, nb.z + k, w[2]);
-        // the row's cell indices first, then its states and kept weights (a
+        int wx = 0, wy = 0;
+        const bool colok = wrap_index(B, 0, nb.x + i, wx) && wrap_index(B, 1, nb.y + j, wy);
+        const int xy = cell_xy(B, wx, wy);
+        // the column's cell indices first, then its states and kept weights (a
         // cell off a wall loads cell 0, unused), so the loads are in flight
         // together rather than one cell at a time
         bool ok[S];
         int ci[S];
 #pragma unroll
-        for (int i = 0; i < S; i++) {
-            ok[i] = rowok && wrap_index(B, 0, nb.x + i, w[0]);
-            ci[i] = ok[i] ? cell_internal(g, B, w) : 0;
+        for (int k = 0; k < S; k++) {
+            int wz = 0;
+            ok[k] = colok && wrap_index(B, 2, nb.z + k, wz);
+            ci[k] = ok[k] ? cell_id(g, B, xy, cell_z(B, wz)) : 0;
         }
         float4 sv[S];
         float rw[S];
 #pragma unroll
-        for (int i = 0; i < S; i++) {
-            sv[i] = st[ci[i]];
-            rw[i] = row[i];
+        for (int k = 0; k < S; k++) {
+            sv[k] = st[ci[k]];
+            rw[k] = col[L * k];
         }
 #pragma unroll
-        for (int i = 0; i < S; i++) {
-            if (!ok[i]) continue;
-            ux = fmaf(rw[i], sv[i].y, ux);
-            uy = fmaf(rw[i], sv[i].z, uy);
-            uz = fmaf(rw[i], sv[i].w, uz);
+        for (int k = 0; k < S; k++) {
+            if (!ok[k]) continue;
+            ux = fmaf(rw[k], sv[k].y, ux);
+            uy = fmaf(rw[k], sv[k].z, uy);
+            uz = fmaf(rw[k], sv[k].w, uz);
         }
         ux = group_sum<L>(ux);
         uy = group_sum<L>(uy);
@@ -202,47 +208,42 @@ __global__ __launch_bounds__(256) void k_ibm_interp(MemArgs m, IbmArgs g, const 
     float wt[S];
     float ws = 0.0f;
     {
-        int w[3] = {0, 0, 0};
-        const bool rowok = wrap_index(B, 1, base[1] + j, w[1]) && wrap_index(B, 2, base[2] + k, w[2]);
-        // the row's wrapped indices, then (cosine kernel) every centroid at
+        int wx = 0, wy = 0;
+        const bool colok = wrap_index(B, 0, base[0] + i, wx) && wrap_index(B, 1, base[1] + j, wy);
+        const int xy = cell_xy(B, wx, wy);
+        // the column's wrapped indices, then (cosine kernel) every centroid at
         // once, then the weights
         bool ok[S];
-        int wx[S];
+        int wz[S];
 #pragma unroll
-        for (int i = 0; i < S; i++) {
-            wx[i] = 0;
-            ok[i] = rowok && wrap_index(B, 0, base[0] + i, wx[i]);
+        for (int k = 0; k < S; k++) {
+            wz[k] = 0;
+            ok[k] = colok && wrap_index(B, 2, base[2] + k, wz[k]);
         }
         float4 c[S];
 #pragma unroll
-        for (int i = 0; i < S; i++) {
-            c[i] = float4{};
-            if constexpr (K == LBFS_IBM_COS4) {
-                const int wi[3] = {wx[i], w[1], w[2]};
-                c[i] = g.cen[ok[i] ? cell_internal(g, B, wi) : 0];
-            }
+        for (int k = 0; k < S; k++) {
+            c[k] = float4{};
+            if constexpr (K == LBFS_IBM_COS4) c[k] = g.cen[ok[k] ? cell_id(g, B, xy, cell_z(B, wz[k])) : 0];
         }
 #pragma unroll
-        for (int i = 0; i < S; i++) {
-            wt[i] = 0.0f;
-            if (!ok[i]) continue;
-            const int wi[3] = {wx[i], w[1], w[2]};
-            wt[i] = stencil_weight<K>(g, B, P, xr, base, i, j, k, wi, c[i]);
-            ws += wt[i];
+        for (int k = 0; k < S; k++) {
+            wt[k] = 0.0f;
+            if (!ok[k]) continue;
+            const int wi[3] = {wx, wy, wz[k]};
+            wt[k] = stencil_weight<K>(g, B, P, xr, base, i, j, k, wi, c[k]);
+            ws += wt[k];
         }
     }
     if constexpr (K == LBFS_IBM_COS4) {
         ws = group_sum<L>(ws);
         const float inv = ws > 0.0f ? 1.0f / ws : 0.0f;
 #pragma unroll
-        for (int i = 0; i < S; i++) wt[i] *= inv;
+        for (int k = 0; k < S; k++) wt[k] *= inv;
     }
     if (live) {
-        if constexpr (S == 4) {
-            *reinterpret_cast<float4 *>(row) = make_float4(wt[0], wt[1], wt[2], wt[3]);
-        } else {
-            *reinterpret_cast<float2 *>(row) = make_float2(wt[0], wt[1]);
-        }
+#pragma unroll
+        for (int k = 0; k < S; k++) col[L * k] = wt[k];
     }
     const int key = node_tile(B, base);
     if (live && r == 0) g.nbase[nd] = make_int4(base[0], base[1], base[2], key);
@@ -318,14 +319,14 @@ __device__ __forceinline__ float4 node_force8(const MemArgs &m, int nd, int sub)
 }
 
 // one node by one wavefront (lane = stencil cell) into the global accumulators
-template <int K>
+template <int K, bool ONE>
 __device__ __forceinline__ void spread_node_global(const MemArgs &m, const IbmArgs &g, int nd, int lane, float4 F)
 {
     constexpr int S = Stencil<K>::S;
     if (lane >= S * S * S) return;
     const float wt = g.wnode[64 * (size_t)nd + lane];
     if (wt == 0.0f) return;
-    const IbmBlock B = node_block(g, nd);
+    const IbmBlock B = node_block<ONE>(g, nd);
     const int4 nb = g.nbase[nd];
     int off[3], w[3];
     lane_offset(S, lane, off);
@@ -340,23 +341,32 @@ __device__ __forceinline__ void spread_node_global(const MemArgs &m, const IbmAr
     g.tile_acc[g.cell_tile[ic]] = 1;
 }
 
-// offsets along one axis whose (wrapped) cell lies in [lo, lo + dim), and
-// their local index
+// Where a stencil's S cells from `base` lie along one axis of a tile of `dim`
+// cells from lo: r0, local index of the first with base wrapped into the axis.
+// The stencil reaches the tile there, or one period before (the next images,
+// periods further back, in a box shorter than the stencil); the return value
+// says whether it does.
 template <int S>
-__device__ __forceinline__ unsigned axis_in(const IbmBlock &B, int a, int base, int lo, int dim, int loc[S])
+__device__ __forceinline__ bool axis_reach(const IbmBlock &B, int a, int base, int lo, int dim, int &r0)
 {
-    unsigned in = 0u;
-#pragma unroll
-    for (int o = 0; o < S; o++) {
-        int w = 0;
-        const bool ok = wrap_index(B, a, base + o, w);
-        loc[o] = w - lo;
-        if (ok && loc[o] >= 0 && loc[o] < dim) in |= 1u << o;
+    const int n = B.n[a];
+    int w = base;
+    if (B.per[a] && (w < 0 || w >= n)) {
+        w = w < 0 ? w + n : w - n;
+        if (__builtin_expect(w < 0 || w >= n, 0)) w = ((base % n) + n) % n;
     }
-    return in;
+    r0 = w - lo;
+    return (r0 > -S && r0 < dim) || (B.per[a] && r0 - n > -S);
 }
 
-template <int K>
+// What bounds this kernel: the candidates' loads, a chain of list, base and
+// force reads per chunk, then the weight rows; one LDS atomic a cell instead of
+// three gains 7 %.  So a lane decides once per candidate where its stencil lies,
+// and a wavefront spreads eight nodes' rows loaded together; what each cell of
+// each node decided before (its wrapped index, its box by flat loads, the range
+// test of a term) took most of the time: 261 -> 142 us for the 380k nodes of a
+// 256x128x128 suspension, 49 -> 34 us for 48k in 96x96x64.
+template <int K, bool ONE, int SPREAD_NT>
 __global__ __launch_bounds__(SPREAD_NT) void k_ibm_spread_tiles(MemArgs m, IbmArgs g)
 {
     constexpr int S = Stencil<K>::S, C = S * S * S, NPW = 64 / C, NW = SPREAD_NT / 64, NS = S * S * S;
@@ -365,27 +375,36 @@ __global__ __launch_bounds__(SPREAD_NT) void k_ibm_spread_tiles(MemArgs m, IbmAr
     const int T = xcd_remap(blockIdx.x, gridDim.x);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int4 tl = g.tile_lo[T];
-    const IbmBlock B = box(g, tl.w);
+    const IbmBlock B = box<ONE>(g, tl.w);
     const int lo[3] = {tl.x, tl.y, tl.z};
     const int dim[3] = {min(B.tw[0], B.n[0] - lo[0]), min(B.tw[1], B.n[1] - lo[1]), min(B.tw[2], B.n[2] - lo[2])};
-    if (tid == 0) {
+    if (wave == 0) {
         // tiles holding the bases of nodes that can reach this tile: per axis
         // those of the cells lo - (S - 1) ... lo (wrapped, or clamped at a wall
-        // as the node tiles are); constant axis indices keep the box in registers
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-            int n = 0;
-#pragma unroll
-            for (int o = S - 1; o >= 0; o--) {
-                int w = lo[a] - o;
-                if (w < 0) w = B.per[a] ? ((w % B.n[a]) + B.n[a]) % B.n[a] : 0;
-                const int t = w / B.tw[a];
-                bool seen = false;
-                for (int q = 0; q < n; q++) seen |= s_tc[a][q] == t;
-                if (!seen) s_tc[a][n++] = t;
+        // as the node tiles are), a lane per cell
+        const int a = lane / S, o = S - 1 - lane % S;
+        int t = 0;
+        bool is_new = false;
+        if (lane < 3 * S) {
+            const int n = a == 0 ? B.n[0] : a == 1 ? B.n[1] : B.n[2];
+            const int tw = a == 0 ? B.tw[0] : a == 1 ? B.tw[1] : B.tw[2];
+            const int per = a == 0 ? B.per[0] : a == 1 ? B.per[1] : B.per[2];
+            int w = (a == 0 ? lo[0] : a == 1 ? lo[1] : lo[2]) - o;
+            if (w < 0) {
+                w = per ? w + n : 0;
+                if (__builtin_expect(w < 0, 0)) w = ((w % n) + n) % n;
             }
-            s_ntc[a] = n;
+            t = w / tw;
+            is_new = true;
         }
+#pragma unroll
+        for (int q = 1; q < S; q++) {
+            const int before = __shfl_up(t, q, 64);
+            if (lane % S >= q && before == t) is_new = false;
+        }
+        const unsigned long long news = __ballot(is_new) >> (a < 3 ? a * S : 0) & ((1ull << S) - 1ull);
+        if (is_new) s_tc[a][__popcll(news & ((1ull << (lane % S)) - 1ull))] = t;
+        if (lane < 3 * S && o == 0) s_ntc[a] = __popcll(news);
     }
     __syncthreads();
     if (wave == 0) {
@@ -427,40 +446,73 @@ __global__ __launch_bounds__(SPREAD_NT) void k_ibm_spread_tiles(MemArgs m, IbmAr
     int *cand = reinterpret_cast<int *>(cF + SPREAD_NT);                 // [SPREAD_NT] node ids
     unsigned long long *tacc = reinterpret_cast<unsigned long long *>(cand + SPREAD_NT);  // 3 x cap sums
     for (int i = tid; i < nct; i += SPREAD_NT) tacc[i] = tacc[cap + i] = tacc[2 * cap + i] = 0ull;
-    for (int q0 = 0; q0 < tot + nov; q0 += SPREAD_NT) {
+    // images of a node to look at along each axis, and how many of them the tile
+    // can keep (one, unless it spans most of a periodic box)
+    int img[3], keeps = 1;
+    if constexpr (SPREAD_NT == 512) {  // (fewer threads: boxes of one image)
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            img[a] = !B.per[a] ? 1 : B.n[a] >= S - 1 ? 2 : (B.n[a] + S - 2) / B.n[a] + 1;
+            if (B.n[a] < dim[a] + S - 1) keeps *= img[a];
+        }
+    }
+    const int chunk = keeps == 1 ? SPREAD_NT : SPREAD_NT / keeps;
+    for (int q0 = 0; q0 < tot + nov; q0 += chunk) {
         if (tid == 0) s_nk = 0;
         __syncthreads();  // the previous chunk is spread
         const int q = q0 + tid;
-        if (q < tot + nov) {
-            int nd;
+        int nd = -1, rx = 0, ry = 0, rz = 0;
+        bool keep = false;
+        if (tid < chunk && q < tot + nov) {
             if (q < tot) {
                 int k = 0;
                 while (q >= s_pre[k + 1]) k++;
                 nd = g.tile_slots[(size_t)s_tile[k] * g.tile_cap + (q - s_pre[k])];
             } else {
                 nd = g.overflow[q - tot];
+                if (!ONE && g.node_block[nd] != tl.w) nd = -1;
             }
-            if (q < tot || g.node_block[nd] == tl.w) {
+            if (nd >= 0) {
                 const int4 nb = g.nbase[nd];
-                int loc[S];
-                const unsigned ix = axis_in<S>(B, 0, nb.x, lo[0], dim[0], loc);
-                const unsigned iy = axis_in<S>(B, 1, nb.y, lo[1], dim[1], loc);
-                const unsigned iz = axis_in<S>(B, 2, nb.z, lo[2], dim[2], loc);
-                if (ix && iy && iz) {
-                    // keep it: the spreading pass below reads it from LDS
-                    const int e = atomicAdd(&s_nk, 1);
-                    cand[e] = nd;
-                    cbase[e] = nb;
-                    cF[e] = m.F[nd];
-                }
+                keep = axis_reach<S>(B, 0, nb.x, lo[0], dim[0], rx) & axis_reach<S>(B, 1, nb.y, lo[1], dim[1], ry) &
+                       axis_reach<S>(B, 2, nb.z, lo[2], dim[2], rz);
             }
+        }
+        // the nodes that reach the tile are kept: the spreading pass below
+        // reads them from LDS
+        float4 F{};
+        if (keep) {
+            F = m.F[nd];
+            F.w = fix_fast_weight(F);
+        }
+        auto put = [&](int e, int x, int y, int z) {
+            cand[e] = nd;
+            cbase[e] = make_int4(x, y, z, x + dim[0] * (y + dim[1] * z));
+            cF[e] = F;
+        };
+        if (keeps == 1) {
+            // one image each: slots by wavefront
+            const unsigned long long kept = __ballot(keep);
+            int e0 = 0;
+            if (lane == 0 && kept) e0 = atomicAdd(&s_nk, __popcll(kept));
+            e0 = __shfl(e0, 0, 64);
+            if (keep)
+                put(e0 + __popcll(kept & ((1ull << lane) - 1ull)), rx < dim[0] ? rx : rx - B.n[0],
+                    ry < dim[1] ? ry : ry - B.n[1], rz < dim[2] ? rz : rz - B.n[2]);
+        } else if (keep) {
+            for (int kz = 0, z = rz; kz < img[2]; kz++, z -= B.n[2])
+                for (int ky = 0, y = ry; ky < img[1]; ky++, y -= B.n[1])
+                    for (int kx = 0, x = rx; kx < img[0]; kx++, x -= B.n[0])
+                        if (x > -S && x < dim[0] && y > -S && y < dim[1] && z > -S && z < dim[2])
+                            put(atomicAdd(&s_nk, 1), x, y, z);
         }
         __syncthreads();
         const int nk = s_nk;
         int off[3];
         lane_offset(S, lane % C, off);
+        const int loff = off[0] + dim[0] * (off[1] + dim[1] * off[2]);
         // UN nodes per wavefront and pass: their weight loads in flight together
-        constexpr int UN = 4;
+        constexpr int UN = 8;
         for (int e0 = wave * NPW * UN; e0 < nk; e0 += NW * NPW * UN) {
             float wt[UN];
 #pragma unroll
@@ -470,20 +522,24 @@ __global__ __launch_bounds__(SPREAD_NT) void k_ibm_spread_tiles(MemArgs m, IbmAr
             }
 #pragma unroll
             for (int u = 0; u < UN; u++) {
-                if (wt[u] == 0.0f) continue;
                 const int e = e0 + u * NPW + lane / C;
-                const int4 nb = cbase[e];
-                int w[3];
-                if (!(wrap_index(B, 0, nb.x + off[0], w[0]) && wrap_index(B, 1, nb.y + off[1], w[1]) &&
-                      wrap_index(B, 2, nb.z + off[2], w[2])))
+                if (wt[u] == 0.0f) continue;
+                const int4 rb = cbase[e];
+                if ((unsigned)(rb.x + off[0]) >= (unsigned)dim[0] || (unsigned)(rb.y + off[1]) >= (unsigned)dim[1] ||
+                    (unsigned)(rb.z + off[2]) >= (unsigned)dim[2])
                     continue;
-                const int l0 = w[0] - lo[0], l1 = w[1] - lo[1], l2 = w[2] - lo[2];
-                if (l0 < 0 || l0 >= dim[0] || l1 < 0 || l1 >= dim[1] || l2 < 0 || l2 >= dim[2]) continue;
-                const int li = l0 + dim[0] * (l1 + dim[1] * l2);
+                const int li = rb.w + loff;
                 const float4 F = cF[e];
-                atomicAdd(tacc + li, fix_term_f(F.x * wt[u], g.err, ERR_FIX_IBM));
-                atomicAdd(tacc + cap + li, fix_term_f(F.y * wt[u], g.err, ERR_FIX_IBM));
-                atomicAdd(tacc + 2 * cap + li, fix_term_f(F.z * wt[u], g.err, ERR_FIX_IBM));
+                const float vx = F.x * wt[u], vy = F.y * wt[u], vz = F.z * wt[u];
+                if (__builtin_expect(fabsf(wt[u]) <= F.w, 1)) {
+                    atomicAdd(tacc + li, fix_term_fast(vx));
+                    atomicAdd(tacc + cap + li, fix_term_fast(vy));
+                    atomicAdd(tacc + 2 * cap + li, fix_term_fast(vz));
+                } else {
+                    atomicAdd(tacc + li, fix_term_f(vx, g.err, ERR_FIX_IBM));
+                    atomicAdd(tacc + cap + li, fix_term_f(vy, g.err, ERR_FIX_IBM));
+                    atomicAdd(tacc + 2 * cap + li, fix_term_f(vz, g.err, ERR_FIX_IBM));
+                }
             }
         }
     }
@@ -513,7 +569,7 @@ __global__ __launch_bounds__(SPREAD_NT) void k_ibm_spread_tiles(MemArgs m, IbmAr
 // window's nonzero sums to the per-cell accumulators.
 constexpr int BIN_NT = 512, BIN_CH = 32;
 
-template <int K>
+template <int K, bool ONE>
 __global__ __launch_bounds__(BIN_NT) void k_ibm_spread_bins(MemArgs m, IbmArgs g)
 {
     constexpr int S = Stencil<K>::S, C = S * S * S, NPW = 64 / C, NW = BIN_NT / 64;
@@ -534,7 +590,7 @@ __global__ __launch_bounds__(BIN_NT) void k_ibm_spread_bins(MemArgs m, IbmArgs g
         const int c_begin = (it % NCH) * BIN_CH, cnt = min(cnt_all, c_begin + BIN_CH) - c_begin;
         if (cnt <= 0) continue;  // uniform over the workgroup
         const int4 tl = g.tile_lo[b];
-        const IbmBlock B = box(g, tl.w);
+        const IbmBlock B = box<ONE>(g, tl.w);
         const int bo[3] = {tl.x, tl.y, tl.z};
         __syncthreads();  // the previous item's window is flushed
         for (int q = tid; q < 3 * NWIN; q += BIN_NT) racc[q / NWIN][q % NWIN] = 0ull;
@@ -557,8 +613,8 @@ __global__ __launch_bounds__(BIN_NT) void k_ibm_spread_bins(MemArgs m, IbmArgs g
             const bool ok = jn < cnt;
             const float4 F = node_force8(m, ok ? cnd[jn] : 0, ok ? (tid & 7) : 8);
             if (ok && (tid & 7) == 0) {
-                cF[jn] = F;
                 m.F[cnd[jn]] = F;
+                cF[jn] = make_float4(F.x, F.y, F.z, fix_fast_weight(F));
             }
         }
 #pragma unroll
@@ -592,9 +648,16 @@ __global__ __launch_bounds__(BIN_NT) void k_ibm_spread_bins(MemArgs m, IbmArgs g
             }
             if (!in) continue;
             const float4 F = cF[jn];
-            atomicAdd(&racc[0][loc], fix_term_f(F.x * wt, g.err, ERR_FIX_IBM));
-            atomicAdd(&racc[1][loc], fix_term_f(F.y * wt, g.err, ERR_FIX_IBM));
-            atomicAdd(&racc[2][loc], fix_term_f(F.z * wt, g.err, ERR_FIX_IBM));
+            const float vx = F.x * wt, vy = F.y * wt, vz = F.z * wt;
+            if (__builtin_expect(fabsf(wt) <= F.w, 1)) {
+                atomicAdd(&racc[0][loc], fix_term_fast(vx));
+                atomicAdd(&racc[1][loc], fix_term_fast(vy));
+                atomicAdd(&racc[2][loc], fix_term_fast(vz));
+            } else {
+                atomicAdd(&racc[0][loc], fix_term_f(vx, g.err, ERR_FIX_IBM));
+                atomicAdd(&racc[1][loc], fix_term_f(vy, g.err, ERR_FIX_IBM));
+                atomicAdd(&racc[2][loc], fix_term_f(vz, g.err, ERR_FIX_IBM));
+            }
         }
         __syncthreads();
         for (int q = tid; q < NWIN; q += BIN_NT) {
@@ -630,17 +693,17 @@ __global__ __launch_bounds__(BIN_NT) void k_ibm_spread_bins(MemArgs m, IbmArgs g
         float4 F = node_force8(m, nd, lane < 8 ? lane : 8);
         F = make_float4(__shfl(F.x, 0, 64), __shfl(F.y, 0, 64), __shfl(F.z, 0, 64), 0.0f);
         if (lane == 0) m.F[nd] = F;
-        spread_node_global<K>(m, g, nd, lane, F);
+        spread_node_global<K, ONE>(m, g, nd, lane, F);
     }
 }
 
 // per-node spreading of every node: one wavefront each
-template <int K>
+template <int K, bool ONE>
 __global__ __launch_bounds__(256) void k_ibm_spread_nodes(MemArgs m, IbmArgs g)
 {
     const int nd = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (nd >= m.n_nodes) return;
-    spread_node_global<K>(m, g, nd, threadIdx.x & 63, m.F[nd]);
+    spread_node_global<K, ONE>(m, g, nd, threadIdx.x & 63, m.F[nd]);
 }
 
 // One workgroup per fluid tile: the tile's spread force densities (written
@@ -798,27 +861,43 @@ __global__ __launch_bounds__(256) void k_mem_nodes(MemArgs m)
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-template <bool INTERP>
-static hipError_t launch_interp_kernel(const MemArgs &m, const IbmArgs &g, const float4 *st, hipStream_t s)
+// a kernel template for the context's stencil and for one box or several
+#define IBM_LAUNCH(KERNEL, grid, blk, lds, s, ...)                                                              \
+    do {                                                                                                      \
+        const bool one_ = g.n_blocks == 1;                                                                    \
+        if (g.kernel == LBFS_IBM_LINEAR2) {                                                                   \
+            if (one_) hipLaunchKernelGGL((KERNEL(LBFS_IBM_LINEAR2, true)), grid, blk, lds, s, __VA_ARGS__);      \
+            else hipLaunchKernelGGL((KERNEL(LBFS_IBM_LINEAR2, false)), grid, blk, lds, s, __VA_ARGS__);          \
+        } else if (g.kernel == LBFS_IBM_LAGRANGE4) {                                                          \
+            if (one_) hipLaunchKernelGGL((KERNEL(LBFS_IBM_LAGRANGE4, true)), grid, blk, lds, s, __VA_ARGS__);    \
+            else hipLaunchKernelGGL((KERNEL(LBFS_IBM_LAGRANGE4, false)), grid, blk, lds, s, __VA_ARGS__);        \
+        } else {                                                                                              \
+            if (one_) hipLaunchKernelGGL((KERNEL(LBFS_IBM_COS4, true)), grid, blk, lds, s, __VA_ARGS__);         \
+            else hipLaunchKernelGGL((KERNEL(LBFS_IBM_COS4, false)), grid, blk, lds, s, __VA_ARGS__);             \
+        }                                                                                                     \
+    } while (0)
+#define K_INTERP(K, ONE) k_ibm_interp<K, ONE, true>
+#define K_WEIGHTS(K, ONE) k_ibm_interp<K, ONE, false>
+#define K_SPREAD_BINS(K, ONE) k_ibm_spread_bins<K, ONE>
+#define K_SPREAD_TILES256(K, ONE) k_ibm_spread_tiles<K, ONE, 256>
+#define K_SPREAD_TILES512(K, ONE) k_ibm_spread_tiles<K, ONE, 512>
+#define K_SPREAD_NODES(K, ONE) k_ibm_spread_nodes<K, ONE>
+
+// S x S lanes per node
+static dim3 interp_grid(const MemArgs &m, const IbmArgs &g)
 {
-    // S x S lanes per node
     const int lanes = g.kernel == LBFS_IBM_LINEAR2 ? 4 : 16;
-    const dim3 grid((unsigned)(((size_t)m.n_nodes * lanes + 255) / 256)), blk(256);
-    if (g.kernel == LBFS_IBM_LINEAR2)
-        hipLaunchKernelGGL((k_ibm_interp<LBFS_IBM_LINEAR2, INTERP>), grid, blk, 0, s, m, g, st);
-    else if (g.kernel == LBFS_IBM_LAGRANGE4)
-        hipLaunchKernelGGL((k_ibm_interp<LBFS_IBM_LAGRANGE4, INTERP>), grid, blk, 0, s, m, g, st);
-    else
-        hipLaunchKernelGGL((k_ibm_interp<LBFS_IBM_COS4, INTERP>), grid, blk, 0, s, m, g, st);
-    return hipGetLastError();
+    return dim3((unsigned)(((size_t)m.n_nodes * lanes + 255) / 256));
 }
 hipError_t launch_ibm_interp(const MemArgs &m, const IbmArgs &g, const float4 *st, hipStream_t s)
 {
-    return launch_interp_kernel<true>(m, g, st, s);
+    IBM_LAUNCH(K_INTERP, interp_grid(m, g), dim3(256), 0, s, m, g, st);
+    return hipGetLastError();
 }
 hipError_t launch_ibm_weights(const MemArgs &m, const IbmArgs &g, hipStream_t s)
 {
-    return launch_interp_kernel<false>(m, g, nullptr, s);
+    IBM_LAUNCH(K_WEIGHTS, interp_grid(m, g), dim3(256), 0, s, m, g, (const float4 *)nullptr);
+    return hipGetLastError();
 }
 hipError_t launch_mem_edges(const MemArgs &m, hipStream_t s)
 {
@@ -842,30 +921,14 @@ hipError_t launch_mem_nodes(const MemArgs &m, hipStream_t s)
 }
 hipError_t launch_ibm_spread(const MemArgs &m, const IbmArgs &g, hipStream_t s)
 {
-    if (g.binned == IBM_SPREAD_BINS) {
-        const dim3 grid(std::min(g.n_tiles * (IBM_BIN_CAP / BIN_CH), 1024)), blk(BIN_NT);
-        if (g.kernel == LBFS_IBM_LINEAR2)
-            hipLaunchKernelGGL(k_ibm_spread_bins<LBFS_IBM_LINEAR2>, grid, blk, 0, s, m, g);
-        else if (g.kernel == LBFS_IBM_LAGRANGE4)
-            hipLaunchKernelGGL(k_ibm_spread_bins<LBFS_IBM_LAGRANGE4>, grid, blk, 0, s, m, g);
-        else
-            hipLaunchKernelGGL(k_ibm_spread_bins<LBFS_IBM_COS4>, grid, blk, 0, s, m, g);
-    } else if (g.binned == IBM_SPREAD_GATHER) {
-        const size_t lds = spread_tile_lds(g.max_tile_cells);
-        const dim3 grid(g.n_tiles), blk(SPREAD_NT);
-        if (g.kernel == LBFS_IBM_LINEAR2)
-            hipLaunchKernelGGL(k_ibm_spread_tiles<LBFS_IBM_LINEAR2>, grid, blk, lds, s, m, g);
-        else if (g.kernel == LBFS_IBM_LAGRANGE4)
-            hipLaunchKernelGGL(k_ibm_spread_tiles<LBFS_IBM_LAGRANGE4>, grid, blk, lds, s, m, g);
-        else
-            hipLaunchKernelGGL(k_ibm_spread_tiles<LBFS_IBM_COS4>, grid, blk, lds, s, m, g);
-    } else {
-        const dim3 grid((m.n_nodes + 3) / 4), blk(256);
-        if (g.kernel == LBFS_IBM_LINEAR2) hipLaunchKernelGGL(k_ibm_spread_nodes<LBFS_IBM_LINEAR2>, grid, blk, 0, s, m, g);
-        else if (g.kernel == LBFS_IBM_LAGRANGE4)
-            hipLaunchKernelGGL(k_ibm_spread_nodes<LBFS_IBM_LAGRANGE4>, grid, blk, 0, s, m, g);
-        else hipLaunchKernelGGL(k_ibm_spread_nodes<LBFS_IBM_COS4>, grid, blk, 0, s, m, g);
-    }
+    if (g.binned == IBM_SPREAD_BINS)
+        IBM_LAUNCH(K_SPREAD_BINS, dim3(std::min(g.n_tiles * (IBM_BIN_CAP / BIN_CH), 1024)), dim3(BIN_NT), 0, s, m, g);
+    else if (g.binned == IBM_SPREAD_GATHER && g.spread_nt == 256)
+        IBM_LAUNCH(K_SPREAD_TILES256, dim3(g.n_tiles), dim3(256), spread_tile_lds(256, g.max_tile_cells), s, m, g);
+    else if (g.binned == IBM_SPREAD_GATHER)
+        IBM_LAUNCH(K_SPREAD_TILES512, dim3(g.n_tiles), dim3(512), spread_tile_lds(512, g.max_tile_cells), s, m, g);
+    else
+        IBM_LAUNCH(K_SPREAD_NODES, dim3((m.n_nodes + 3) / 4), dim3(256), 0, s, m, g);
     return hipGetLastError();
 }
 

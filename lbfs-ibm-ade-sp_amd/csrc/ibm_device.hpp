@@ -37,6 +37,23 @@ __device__ __forceinline__ unsigned long long fix_term_f(float v, int *err, int 
     return 0ull;
 }
 
+// The same term where |v| < 2^11 is known: added to 1.5 2^52, the
+// double's low mantissa bits are v 2^40 rounded to nearest, the very integer
+// fix_term_f converts to, in three instructions instead of fourteen.
+__device__ __forceinline__ unsigned long long fix_term_fast(float v)
+{
+    const unsigned long long b = (unsigned long long)__double_as_longlong(__fma_rn((double)v, FIX_SCALE, 6755399441055744.0));
+    const unsigned hi = (unsigned)(b >> 32) - 0x43380000u;
+    return ((unsigned long long)hi << 32) | (unsigned)b;
+}
+// largest weight whose terms of force F stay below 2^11 (negative if none does:
+// no weight, and no NaN, is then within it)
+__device__ __forceinline__ float fix_fast_weight(float4 F)
+{
+    const float s = fabsf(F.x) + fabsf(F.y) + fabsf(F.z);
+    return s < 1e30f ? fminf(1024.0f / s, 1e30f) : -1.0f;
+}
+
 struct f3 {
     float x, y, z;
 };
@@ -218,12 +235,22 @@ __device__ __forceinline__ float cos4_weight_grad(const IbmBlock &B, const float
 // internal id of the cell with (wrapped) index w: from the tile layout in a
 // box of whole tiles (tiles x fastest, cells x fastest within a tile), else
 // through the id map
-// the box of node nd, and box b (a single box comes by value with the arguments)
+// The box of node nd, and box b of a whole workgroup.  ONE: the mesh is a single
+// box, which comes by value with the arguments and stays in scalar registers (a
+// kernel that chose between the two at run time read it through flat loads,
+// lane by lane).
+template <bool ONE>
 __device__ __forceinline__ IbmBlock node_block(const IbmArgs &g, int nd)
 {
-    return g.n_blocks == 1 ? g.blk0 : g.blk[g.node_block[nd]];
+    if constexpr (ONE) return g.blk0;
+    else return g.blk[g.node_block[nd]];
 }
-__device__ __forceinline__ IbmBlock box(const IbmArgs &g, int b) { return g.n_blocks == 1 ? g.blk0 : g.blk[b]; }
+template <bool ONE>
+__device__ __forceinline__ IbmBlock box(const IbmArgs &g, int b)
+{
+    if constexpr (ONE) return g.blk0;
+    else return g.blk[__builtin_amdgcn_readfirstlane(b)];
+}
 
 __device__ __forceinline__ int cell_internal(const IbmArgs &g, const IbmBlock &B, const int w[3])
 {
@@ -234,6 +261,27 @@ __device__ __forceinline__ int cell_internal(const IbmArgs &g, const IbmBlock &B
         return B.icell0 + ((t0 + B.fnt[0] * (t1 + B.fnt[1] * t2)) << (B.fsh[0] + B.fsh[1] + B.fsh[2])) + l;
     }
     return g.inv[B.cell0 + w[0] + B.n[0] * (w[1] + B.n[1] * w[2])];
+}
+
+// the same id in two parts, of the indices along x and y and of the index
+// along z, for cells that share their x and y; cell_id joins them
+__device__ __forceinline__ int cell_xy(const IbmBlock &B, int wx, int wy)
+{
+    if (B.regular)
+        return (((wx >> B.fsh[0]) + B.fnt[0] * (wy >> B.fsh[1])) << (B.fsh[0] + B.fsh[1] + B.fsh[2])) +
+               (wx & (B.ftw[0] - 1)) + ((wy & (B.ftw[1] - 1)) << B.fsh[0]);
+    return wx + B.n[0] * wy;
+}
+__device__ __forceinline__ int cell_z(const IbmBlock &B, int wz)
+{
+    if (B.regular)
+        return ((B.fnt[0] * B.fnt[1] * (wz >> B.fsh[2])) << (B.fsh[0] + B.fsh[1] + B.fsh[2])) +
+               ((wz & (B.ftw[2] - 1)) << (B.fsh[0] + B.fsh[1]));
+    return B.n[0] * B.n[1] * wz;
+}
+__device__ __forceinline__ int cell_id(const IbmArgs &g, const IbmBlock &B, int xy, int z)
+{
+    return B.regular ? B.icell0 + xy + z : g.inv[B.cell0 + xy + z];
 }
 
 // fluid tile coordinate along axis a of a node whose stencil base index is
