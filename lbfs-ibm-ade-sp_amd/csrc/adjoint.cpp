@@ -366,12 +366,10 @@ int replay_step(lbfs_ctx *ctx, StepRec &r, const float4 *st, float4 *st_next, co
     HIPCHK(replay_fluid(ctx, ctx->args, r, st, st_next, q.side));
     HIPCHK(hipEventRecord(q.join, q.side));
     HIPCHK(hipStreamWaitEvent(q.side2, q.fork, 0));
-    HIPCHK(launch_mem_volume(m, q.side2));
-    HIPCHK(launch_mem_edges(m, q.side2));
-    if (!spread_gathers_forces(ctx->ibm)) HIPCHK(launch_mem_nodes(m, q.side2));
+    HIPCHK(launch_mem_forces(m, !spread_gathers_forces(ctx->ibm), q.side2));
     HIPCHK(hipEventRecord(q.join2, q.side2));
     HIPCHK(hipStreamWaitEvent(q.main, q.join2, 0));
-    HIPCHK(launch_ibm_spread(m, ctx->ibm, q.main));
+    HIPCHK(launch_ibm_spread(m, ctx->ibm, m.n_force_wg > 0, q.main));
     HIPCHK(hipStreamWaitEvent(q.main, q.join, 0));
     // the step's cell force goes straight into the record (every cell)
     lbfs::ApplyArgs p = ctx->apply_args(st_next, r.cf, 1);

@@ -178,6 +178,24 @@ extern "C" int lbfs_add_membranes(lbfs_ctx *ctx, const lbfs_membrane_desc *mem, 
     m.X = dX; m.U = dU; m.F = dF; m.node_mem = dnm; m.origin = dorig; m.node_origin = dnorig; m.tri = dtri;
     m.mem_tri_start = dts; m.mem_edge_start = des0; m.edges = dedg; m.edge_mem = dem;
     m.edge_const = dec; m.edge_area0 = dea; m.edge_state = des; m.edge_force = def;
+    std::vector<int2> force_wg;
+    int most_tri = 0;
+    for (int i = 0; i < count; i++) {
+        most_tri = std::max(most_tri, ms[i].n_tri);
+        for (int n = mem_node_start[i]; n < mem_node_start[i + 1]; n += FORCE_NODES) force_wg.push_back(make_int2(i, n));
+    }
+    // Small membranes take the one-launch force pass: three launches of some 3 us
+    // and the gaps between them become one of 6 (a step beside 8 cells of 642
+    // nodes 60 -> 55 us, 27 of 162 nodes 54 -> 48, one of 642 in tile-gathered
+    // 32k cells 46 -> 42).  Each workgroup sums its membrane's volume and area and
+    // each spring is evaluated four times, so larger ones lose: one of 1442 nodes
+    // 51.4 -> 50.7, of 1962 53.8 -> 55.5, of 2562 55.7 -> 58.4, 27 of 1482 118 -> 142.
+    if (most_tri <= 2560 && nn <= 8192) {
+        int2 *dwg;
+        if ((rc = cp_alloc(ctx, &dwg, force_wg.data(), force_wg.size()))) return rc;
+        m.force_wg = dwg;
+        m.n_force_wg = (int)force_wg.size();
+    }
     m.inc_start = dis; m.inc = dinc; m.params = dpar; m.glob = dgl; m.mem_acc = dmacc;
     ctx->mem_node_start = mem_node_start;
     ctx->mem_params = params;

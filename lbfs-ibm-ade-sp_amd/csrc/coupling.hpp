@@ -52,6 +52,8 @@ struct MemArgs {
                               // A_prev, MAD of the next force call
     unsigned long long *mem_acc;  // 4 per membrane: running sums of V, A and the MAD numerator
                               // (fixed point, MEM_SUM_SCALE), closed out by the cell update
+    const int2 *force_wg;     // [n_force_wg] workgroups of the one-launch force pass: membrane, first node
+    int n_force_wg;           // 0: the forces in separate passes
     float4 *bbox;             // 2 per membrane: lower and upper corner of the nodes
     const int *mem_block;     // box of each membrane
     int *err;                 // the context's device error word (ERR_FIX_* bits, fixed_point.hpp)
@@ -161,9 +163,15 @@ hipError_t launch_ibm_weights(const MemArgs &m, const IbmArgs &g, hipStream_t s)
 hipError_t launch_mem_volume(const MemArgs &m, hipStream_t s);
 hipError_t launch_mem_edges(const MemArgs &m, hipStream_t s);
 hipError_t launch_mem_nodes(const MemArgs &m, hipStream_t s);
+// A step's membrane forces (the same bits either way): node forces in one
+// launch, or the passes above; the bin scattering then gathers the node forces
+// itself, so node_forces says whether F is wanted.
+constexpr int FORCE_NT = 512, FORCE_NODES = FORCE_NT / 16;
+hipError_t launch_mem_forces(const MemArgs &m, bool node_forces, hipStream_t s);
 // spreading: per fluid tile into spread_f, or per node into the fixed-point
 // cell accumulators; launch_ibm_apply adds the force densities to the state
-hipError_t launch_ibm_spread(const MemArgs &m, const IbmArgs &g, hipStream_t s);
+// (have_F: the node forces are in F; if not, the bin scattering gathers them)
+hipError_t launch_ibm_spread(const MemArgs &m, const IbmArgs &g, bool have_F, hipStream_t s);
 hipError_t launch_ibm_apply(const IbmArgs &g, const ApplyArgs &p, hipStream_t s);
 // Binned search structure of the internal-viscosity field, rebuilt with it:
 // per membrane its triangles by the y-z bins their projections overlap (a ray

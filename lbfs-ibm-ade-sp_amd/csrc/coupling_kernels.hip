@@ -9,8 +9,8 @@
 //   k_mem_edges    per spring: all membrane force terms (spring_network.cu:613-971),
 //                  written per edge and slot (no atomics); the MAD sum of the next
 //                  force call (spring_network.cu:1186-1238)
-//   k_mem_nodes    per node: sum of its edge slots in a fixed order, combined
-//                  with the membrane's global coefficients
+//   k_mem_nodes    per node: sum of its edge slots in a fixed order
+//   k_mem_forces   the three above in one launch, for small membranes
 //   k_ibm_spread_tiles
 //                  per fluid tile: the forces of the nodes listed around the tile
 //                  spread onto its cells (immersed_boundary_method.cu:947-1024) in
@@ -56,29 +56,22 @@ __device__ __forceinline__ long long mem_fx(double x, int *err)
     return (long long)fix_term(x, MEM_SUM_SCALE, err, ERR_FIX_MEM);
 }
 
-// volume and area of triangle t (thread t) added to its membrane's sums
-__device__ __forceinline__ void triangle_sums(const MemArgs &m, int t)
+// volume and area of triangle qq
+__device__ __forceinline__ void triangle_terms(const MemArgs &m, const int4 qq, long long v[2])
 {
-    int tm = -1;
-    long long v[2] = {0, 0};
-    if (t < m.n_tri) {
-        const int4 qq = m.tri[t];
-        const f3 a = ld3(m.X[qq.x]), b = ld3(m.X[qq.y]), c = ld3(m.X[qq.z]);
-        const f3 N = cross(b - a, c - a);
-        v[0] = mem_fx((double)dot(N, (a + b + c) * (1.0f / 3.0f)) / 6.0, m.err);
-        v[1] = mem_fx(0.5 * (double)sqrtf(dot(N, N)), m.err);
-        tm = qq.w;
-    }
-    mem_sum_add(m.mem_acc, tm, v, 2);
+    const f3 a = ld3(m.X[qq.x]), b = ld3(m.X[qq.y]), c = ld3(m.X[qq.z]);
+    const f3 N = cross(b - a, c - a);
+    v[0] = mem_fx((double)dot(N, (a + b + c) * (1.0f / 3.0f)) / 6.0, m.err);
+    v[1] = mem_fx(0.5 * (double)sqrtf(dot(N, N)), m.err);
 }
 
-// the membrane's global coefficients in FP64 from the running volume and area
-// sums and the MAD of this force call, rounded once to the working precision
-__device__ __forceinline__ void mem_coefs(const MemArgs &m, int mem, float &vol, float &area, float &mad)
+// the membrane's global coefficients in FP64 from its volume and area sums and
+// the MAD of this force call, rounded once to the working precision
+__device__ __forceinline__ void mem_coefs(const MemArgs &m, int mem, long long v, long long a, float &vol, float &area,
+                                          float &mad)
 {
     const double *gl = m.glob + 8 * (size_t)mem;
-    const unsigned long long *acc = m.mem_acc + 4 * (size_t)mem;
-    const double V = (double)(long long)acc[0] * (1.0 / MEM_SUM_SCALE), A = (double)(long long)acc[1] * (1.0 / MEM_SUM_SCALE);
+    const double V = (double)v * (1.0 / MEM_SUM_SCALE), A = (double)a * (1.0 / MEM_SUM_SCALE);
     const MemParamDev &p = m.params[mem];
     vol = (float)(-(double)p.volume_modulus * (V / gl[3] - 1.0) / 6.0);
     area = (float)(-(double)p.global_area_modulus * (A / gl[4] - 1.0));
@@ -570,7 +563,7 @@ __global__ __launch_bounds__(SPREAD_NT) void k_ibm_spread_tiles(MemArgs m, IbmAr
 constexpr int BIN_NT = 512, BIN_CH = 32;
 
 template <int K, bool ONE>
-__global__ __launch_bounds__(BIN_NT) void k_ibm_spread_bins(MemArgs m, IbmArgs g)
+__global__ __launch_bounds__(BIN_NT) void k_ibm_spread_bins(MemArgs m, IbmArgs g, bool have_F)
 {
     constexpr int S = Stencil<K>::S, C = S * S * S, NPW = 64 / C, NW = BIN_NT / 64;
     constexpr int NCH = IBM_BIN_CAP / BIN_CH, WD = 4 + S - 1, NWIN = WD * WD * WD;
@@ -611,9 +604,11 @@ __global__ __launch_bounds__(BIN_NT) void k_ibm_spread_bins(MemArgs m, IbmArgs g
         if (tid < 8 * BIN_CH) {  // whole wavefronts: the eight-lane sums shuffle
             const int jn = tid >> 3;
             const bool ok = jn < cnt;
-            const float4 F = node_force8(m, ok ? cnd[jn] : 0, ok ? (tid & 7) : 8);
+            float4 F{};
+            if (!have_F) F = node_force8(m, ok ? cnd[jn] : 0, ok ? (tid & 7) : 8);
             if (ok && (tid & 7) == 0) {
-                m.F[cnd[jn]] = F;
+                if (have_F) F = m.F[cnd[jn]];
+                else m.F[cnd[jn]] = F;
                 cF[jn] = make_float4(F.x, F.y, F.z, fix_fast_weight(F));
             }
         }
@@ -690,9 +685,14 @@ __global__ __launch_bounds__(BIN_NT) void k_ibm_spread_bins(MemArgs m, IbmArgs g
     const int nov = min(*g.n_overflow, m.n_nodes);
     for (int e = blockIdx.x * NW + wave; e < nov; e += gridDim.x * NW) {
         const int nd = g.overflow[e];
-        float4 F = node_force8(m, nd, lane < 8 ? lane : 8);
-        F = make_float4(__shfl(F.x, 0, 64), __shfl(F.y, 0, 64), __shfl(F.z, 0, 64), 0.0f);
-        if (lane == 0) m.F[nd] = F;
+        float4 F;
+        if (have_F) {
+            F = m.F[nd];
+        } else {
+            F = node_force8(m, nd, lane < 8 ? lane : 8);
+            F = make_float4(__shfl(F.x, 0, 64), __shfl(F.y, 0, 64), __shfl(F.z, 0, 64), 0.0f);
+            if (lane == 0) m.F[nd] = F;
+        }
         spread_node_global<K, ONE>(m, g, nd, lane, F);
     }
 }
@@ -805,7 +805,40 @@ __device__ __forceinline__ memf::EdgeConst edge_const(const MemArgs &m, const Me
 // per triangle: volume and area sums
 __global__ __launch_bounds__(256) void k_mem_volume(MemArgs m)
 {
-    triangle_sums(m, blockIdx.x * blockDim.x + threadIdx.x);
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    int tm = -1;
+    long long v[2] = {0, 0};
+    if (t < m.n_tri) {
+        const int4 qq = m.tri[t];
+        triangle_terms(m, qq, v);
+        tm = qq.w;
+    }
+    mem_sum_add(m.mem_acc, tm, v, 2);
+}
+
+// edge e's nodes' positions and velocities and its moduli, all but the
+// membrane's global coefficients
+__device__ __forceinline__ void edge_inputs(const MemArgs &m, const MemParamDev &p, int e, memf::EdgeIn<float> &in)
+{
+    const int4 q = m.edges[e];
+    const float4 xa = m.X[q.x], xb = m.X[q.y], xc = m.X[q.z], xd = m.X[q.w], va = m.U[q.x], vc = m.U[q.z];
+    in.A = {xa.x, xa.y, xa.z};
+    in.B = {xb.x, xb.y, xb.z};
+    in.C = {xc.x, xc.y, xc.z};
+    in.D = {xd.x, xd.y, xd.z};
+    in.Ua = {va.x, va.y, va.z};
+    in.Uc = {vc.x, vc.y, vc.z};
+    in.ks = m.edge_const[e].y;
+    in.lb = p.local_bending;
+    in.gb = p.global_bending;
+}
+
+// the edge's state for the next force call: kept, and its MAD term
+__device__ __forceinline__ long long edge_keep(const MemArgs &m, const MemParamDev &p, int e, int first_edge,
+                                               const memf::EdgeOut<float> &out)
+{
+    m.edge_state[e] = make_float4(out.kappa, out.n1, out.n2, 0.0f);
+    return e - first_edge < p.n_mad ? mem_fx((double)out.kappa * ((double)out.n1 + (double)out.n2) / 3.0, m.err) : 0;
 }
 
 // Per spring: the force on its four nodes with the membrane's global
@@ -820,32 +853,111 @@ __global__ __launch_bounds__(128) void k_mem_edges(MemArgs m)
     if (e < m.n_edges) {
         const int mem = m.edge_mem[e];
         const MemParamDev p = m.params[mem];
+        const unsigned long long *acc = m.mem_acc + 4 * (size_t)mem;
         memf::EdgeIn<float> in;
-        mem_coefs(m, mem, in.vol_coef, in.area_coef, in.mad_coef);
-        const int4 q = m.edges[e];
-        const float4 xa = m.X[q.x], xb = m.X[q.y], xc = m.X[q.z], xd = m.X[q.w], va = m.U[q.x], vc = m.U[q.z];
-        in.A = {xa.x, xa.y, xa.z};
-        in.B = {xb.x, xb.y, xb.z};
-        in.C = {xc.x, xc.y, xc.z};
-        in.D = {xd.x, xd.y, xd.z};
-        in.Ua = {va.x, va.y, va.z};
-        in.Uc = {vc.x, vc.y, vc.z};
-        in.ks = m.edge_const[e].y;
-        in.lb = p.local_bending;
-        in.gb = p.global_bending;
+        mem_coefs(m, mem, (long long)acc[0], (long long)acc[1], in.vol_coef, in.area_coef, in.mad_coef);
+        edge_inputs(m, p, e, in);
         memf::EdgeOut<float> out;
         memf::edge_force(in, edge_const(m, p, e), out);
-        m.edge_state[e] = make_float4(out.kappa, out.n1, out.n2, 0.0f);
 #pragma unroll
         for (int j = 0; j < 4; j++)
             m.edge_force[4 * (size_t)e + j] = make_float4(out.F[j].x, out.F[j].y, out.F[j].z, 0.0f);
-        if (e - m.mem_edge_start[mem] < p.n_mad) {
-            em = mem;
-            mv[0] = mem_fx((double)out.kappa * ((double)out.n1 + (double)out.n2) / 3.0, m.err);
-        }
+        em = mem;
+        mv[0] = edge_keep(m, p, e, m.mem_edge_start[mem], out);
     }
     // the MAD sum goes to the third slot
     mem_sum_add(m.mem_acc + 2, em, mv, 1);
+}
+
+// sums of up to two values over the workgroup, in every thread
+template <int NT>
+__device__ __forceinline__ void wg_sum(long long v[2], long long lds[2][NT / 64])
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < 2; k++) v[k] += __shfl_xor(v[k], off, 64);
+    if ((threadIdx.x & 63) == 0)
+        for (int k = 0; k < 2; k++) lds[k][threadIdx.x >> 6] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        v[k] = 0;
+#pragma unroll
+        for (int w = 0; w < NT / 64; w++) v[k] += lds[k][w];
+    }
+}
+
+// The three passes in one launch: a workgroup sums its membrane's volume
+// and area itself, then sixteen lanes per node evaluate the springs
+// around it and add their shares in the order of node_force8 (so the bits are
+// those of the separate passes; a spring is evaluated once for each of its four
+// nodes, and the one at slot 0 keeps its state).  Latency bounds it: the chains
+// of index, position and arithmetic of one triangle and one spring per lane.
+__global__ __launch_bounds__(FORCE_NT) void k_mem_forces(MemArgs m)
+{
+    __shared__ long long s_sum[2][FORCE_NT / 64], s_mad[2][FORCE_NT / 64];
+    __shared__ float s_coef[3];
+    const int2 wg = m.force_wg[xcd_remap(blockIdx.x, gridDim.x)];
+    const int mem = __builtin_amdgcn_readfirstlane(wg.x), n0 = __builtin_amdgcn_readfirstlane(wg.y);
+    const int tid = threadIdx.x, lane = tid & 15;
+    const int nd = n0 + (tid >> 4);
+    const bool live = nd < m.mem_node_start[mem + 1];
+    int j = 0, j1 = 0;
+    if (live) {
+        j = m.inc_start[nd] + lane;
+        j1 = m.inc_start[nd + 1];
+    }
+    long long v[2] = {0, 0};
+    for (int t = m.mem_tri_start[mem] + tid; t < m.mem_tri_start[mem + 1]; t += FORCE_NT) {
+        long long w[2];
+        triangle_terms(m, m.tri[t], w);
+        v[0] += w[0];
+        v[1] += w[1];
+    }
+    wg_sum<FORCE_NT>(v, s_sum);
+    if (tid == 0) {
+        if (n0 == m.mem_node_start[mem]) {
+            m.mem_acc[4 * (size_t)mem] = (unsigned long long)v[0];
+            m.mem_acc[4 * (size_t)mem + 1] = (unsigned long long)v[1];
+        }
+        mem_coefs(m, mem, v[0], v[1], s_coef[0], s_coef[1], s_coef[2]);
+    }
+    __syncthreads();
+    const MemParamDev p = m.params[mem];
+    const int first_edge = m.mem_edge_start[mem];
+    long long mad[2] = {0, 0};
+    float fx = 0.0f, fy = 0.0f, fz = 0.0f;
+    for (; __any(j < j1); j += 16) {
+        float x = 0.0f, y = 0.0f, z = 0.0f;
+        if (j < j1) {
+            const int es = m.inc[j], e = es >> 2, slot = es & 3;
+            memf::EdgeIn<float> in;
+            in.vol_coef = s_coef[0];
+            in.area_coef = s_coef[1];
+            in.mad_coef = s_coef[2];
+            edge_inputs(m, p, e, in);
+            memf::EdgeOut<float> out;
+            memf::edge_force(in, edge_const(m, p, e), out);
+            const memf::V3<float> a = slot & 1 ? out.F[1] : out.F[0], b = slot & 1 ? out.F[3] : out.F[2];
+            x = slot & 2 ? b.x : a.x;
+            y = slot & 2 ? b.y : a.y;
+            z = slot & 2 ? b.z : a.z;
+            if (slot == 0) mad[0] += edge_keep(m, p, e, first_edge, out);
+        }
+        // lane s < 8: the shares s, s + 8, s + 16, ... in this order
+        fx += x; fy += y; fz += z;
+        fx += __shfl_xor(x, 8, 64); fy += __shfl_xor(y, 8, 64); fz += __shfl_xor(z, 8, 64);
+    }
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1) {
+        fx += __shfl_xor(fx, off, 64);
+        fy += __shfl_xor(fy, off, 64);
+        fz += __shfl_xor(fz, off, 64);
+    }
+    if (live && lane == 0) m.F[nd] = make_float4(fx, fy, fz, 0.0f);
+    wg_sum<FORCE_NT>(mad, s_mad);
+    if (tid == 0 && mad[0]) atomicAdd(m.mem_acc + 4 * (size_t)mem + 2, (unsigned long long)mad[0]);
 }
 
 // eight lanes per node, each summing every eighth incidence
@@ -919,10 +1031,21 @@ hipError_t launch_mem_nodes(const MemArgs &m, hipStream_t s)
     hipLaunchKernelGGL(k_mem_nodes, dim3((8 * m.n_nodes + 255) / 256), dim3(256), 0, s, m);
     return hipGetLastError();
 }
-hipError_t launch_ibm_spread(const MemArgs &m, const IbmArgs &g, hipStream_t s)
+hipError_t launch_mem_forces(const MemArgs &m, bool node_forces, hipStream_t s)
+{
+    if (m.n_force_wg) {
+        hipLaunchKernelGGL(k_mem_forces, dim3(m.n_force_wg), dim3(FORCE_NT), 0, s, m);
+        return hipGetLastError();
+    }
+    hipError_t e = launch_mem_volume(m, s);
+    if (e == hipSuccess) e = launch_mem_edges(m, s);
+    if (e == hipSuccess && node_forces) e = launch_mem_nodes(m, s);
+    return e;
+}
+hipError_t launch_ibm_spread(const MemArgs &m, const IbmArgs &g, bool have_F, hipStream_t s)
 {
     if (g.binned == IBM_SPREAD_BINS)
-        IBM_LAUNCH(K_SPREAD_BINS, dim3(std::min(g.n_tiles * (IBM_BIN_CAP / BIN_CH), 1024)), dim3(BIN_NT), 0, s, m, g);
+        IBM_LAUNCH(K_SPREAD_BINS, dim3(std::min(g.n_tiles * (IBM_BIN_CAP / BIN_CH), 1024)), dim3(BIN_NT), 0, s, m, g, have_F);
     else if (g.binned == IBM_SPREAD_GATHER && g.spread_nt == 256)
         IBM_LAUNCH(K_SPREAD_TILES256, dim3(g.n_tiles), dim3(256), spread_tile_lds(256, g.max_tile_cells), s, m, g);
     else if (g.binned == IBM_SPREAD_GATHER)

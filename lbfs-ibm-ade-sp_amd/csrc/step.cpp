@@ -72,7 +72,7 @@ std::vector<lbfs_ctx::Stage> lbfs_ctx::step_stages(bool with_visc, bool fused_fl
         // fixed-point sums read and written 48 (per-node and bin scattering)
         const double cell_bytes = ibm.binned == IBM_SPREAD_GATHER ? 12.0 : 48.0;
         s.push_back({"ibm_spread", [ctx]() -> int {
-                         HIPCHK(launch_ibm_spread(ctx->mem, ctx->ibm, ctx->stream));
+                         HIPCHK(launch_ibm_spread(ctx->mem, ctx->ibm, false, ctx->stream));
                          return LBFS_OK;
                      },
                      288.0 * nn + cell_bytes * touched + (gather_forces ? node_force_bytes : 0.0)});
@@ -187,10 +187,8 @@ int lbfs_ctx::run_stages(bool with_visc)
         }
         HIPCHK(hipStreamWaitEvent(side, ev_fork, 0));
         if (!interp_first) HIPCHK(launch_ibm_interp(mem, ibm, st[cur], side));
-        HIPCHK(launch_mem_volume(mem, side));
-        HIPCHK(launch_mem_edges(mem, side));
-        if (!spread_gathers_forces(ibm)) HIPCHK(launch_mem_nodes(mem, side));
-        HIPCHK(launch_ibm_spread(mem, ibm, side));
+        HIPCHK(launch_mem_forces(mem, !spread_gathers_forces(ibm), side));
+        HIPCHK(launch_ibm_spread(mem, ibm, mem.n_force_wg > 0, side));
         HIPCHK(hipEventRecord(ev_join, side));
         HIPCHK(hipStreamWaitEvent(stream, ev_join, 0));
         HIPCHK(launch_ibm_apply(ibm, apply_args(st[cur ^ 1], cell_force, 0), stream));
@@ -209,12 +207,10 @@ int lbfs_ctx::run_stages(bool with_visc)
     HIPCHK(launch_ibm_interp(mem, ibm, st[cur], stream));
     HIPCHK(hipEventRecord(ev_fork2, stream));
     HIPCHK(hipStreamWaitEvent(side2, ev_fork2, 0));
-    HIPCHK(launch_mem_volume(mem, side2));
-    HIPCHK(launch_mem_edges(mem, side2));
-    if (!spread_gathers_forces(ibm)) HIPCHK(launch_mem_nodes(mem, side2));
+    HIPCHK(launch_mem_forces(mem, !spread_gathers_forces(ibm), side2));
     HIPCHK(hipEventRecord(ev_join2, side2));
     HIPCHK(hipStreamWaitEvent(stream, ev_join2, 0));
-    HIPCHK(launch_ibm_spread(mem, ibm, stream));
+    HIPCHK(launch_ibm_spread(mem, ibm, mem.n_force_wg > 0, stream));
     HIPCHK(hipStreamWaitEvent(stream, ev_join, 0));
     HIPCHK(launch_ibm_apply(ibm, apply_args(st[cur ^ 1], cell_force, 0), stream));
     cur ^= 1;
