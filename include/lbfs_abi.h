@@ -170,7 +170,8 @@ int lbfs_step(lbfs_ctx *ctx, int nsteps);
                                  bit for bit */
 #define LBFS_OPT_STEP_SCHEDULE 3 /* coupled step schedule (the result is the same bit for bit):
                                     0 (default) the fluid passes on the main stream from the start
-                                    of the step, the whole coupling chain on a second; 1 the
+                                    of the step, the whole coupling chain on a second (up to 128 k
+                                    cells after them on the same stream); 1 the
                                     interpolation alone, then the fluid passes on the main stream
                                     and the membrane forces and spreading on a second; 2 the fluid
                                     passes on a second stream from the start, the membrane forces

@@ -19,6 +19,14 @@ struct AdjointState;  // adjoint.cpp
 void adjoint_release(lbfs_ctx *ctx);
 }  // namespace lbfs
 
+// Coupled meshes up to this many cells run a step's kernels in order on one
+// stream: the waits across streams cost a step 17 us in a graph, more than the
+// overlap gains there.  One stream against two, a cell of 642 nodes: 9600 cells
+// 38.6 and 47.4 us a step, 41k 38.9 and 44.7, 77k 40.1 and 43.7, 147k 47.5 and
+// 46.4, 251k 55.5 and 50.2; of 2562 nodes 73 and 83, 58 and 65, 53 and 58, 59 and
+// 60, 71 and 66.
+constexpr int ONE_STREAM_CELLS = 128 * 1024;
+
 struct lbfs_ctx {
     std::string err;
     int device = 0;

@@ -166,7 +166,8 @@ int lbfs_ctx::run_stages(bool with_visc)
     // face pass and for spreading.  Same kernels, same inputs: the results are
     // those of the sequential order.
     // Schedule 0 (the default): the fluid passes on the main stream from the
-    // start of the step, the whole coupling chain on a second.  Schedule 1:
+    // start of the step, the whole coupling chain on a second (on small meshes
+    // after them on the main stream).  Schedule 1:
     // the interpolation first and alone on the main stream (beside the fluid
     // passes it runs several times slower), then the fluid passes on the main
     // stream and the membrane forces and spreading on a second.  Schedule 2:
@@ -175,6 +176,20 @@ int lbfs_ctx::run_stages(bool with_visc)
     // first: a captured graph launches its branches in that order.)  In a
     // graph each wait across streams costs 10-20 us; schedules 0 and 2 measure
     // the same, schedule 1 some 2 us more per step.
+    if (schedule_option == 0 && lay.n_cells <= ONE_STREAM_CELLS) {
+        if (fz) {
+            HIPCHK(launch_fluid_fused(args, st[cur], st[cur ^ 1], res_out(), 1, stream));
+        } else {
+            HIPCHK(launch_gradients(args, st[cur], grad, stream));
+            HIPCHK(launch_flux_update(args, st[cur], grad, st[cur ^ 1], res_out(), 1, stream));
+        }
+        HIPCHK(launch_ibm_interp(mem, ibm, st[cur], stream));
+        HIPCHK(launch_mem_forces(mem, !spread_gathers_forces(ibm), stream));
+        HIPCHK(launch_ibm_spread(mem, ibm, mem.n_force_wg > 0, stream));
+        HIPCHK(launch_ibm_apply(ibm, apply_args(st[cur ^ 1], cell_force, 0), stream));
+        cur ^= 1;
+        return LBFS_OK;
+    }
     if (schedule_option == 0 || schedule_option == 1) {
         const bool interp_first = schedule_option == 1;
         if (interp_first) HIPCHK(launch_ibm_interp(mem, ibm, st[cur], stream));

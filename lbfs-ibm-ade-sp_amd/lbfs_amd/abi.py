@@ -699,7 +699,7 @@ class Solver:
 
     def set_step_schedule(self, mode):
         """Coupled step schedule: 0 (default) fluid on the main stream from the start, the whole
-        coupling chain on a side stream; 1 interpolation alone, then fluid on the main stream and
+        coupling chain on a side stream (small meshes: all on one stream); 1 interpolation alone, then fluid on the main stream and
         membrane forces + spreading on a side stream; 2 fluid on a side stream, forces on a third."""
         check(load().lbfs_set_option(self.ctx, OPT_STEP_SCHEDULE, int(mode)), self.ctx)
 
