@@ -180,36 +180,218 @@ __device__ __forceinline__ void all_pair_vjps(std::integer_sequence<int, P...>, 
     (pair_vjp<L, 2 * P + 1>(fa, po, pn, Go, Gn, nx, ny, nz, rho0, ig, lpo, lpn, lGo, lGn), ...);
 }
 
+// What one tile-face's adjoint reads: its record, its moments S0 and S1 as the
+// forward pass computed them, and the state, gradient and residual adjoint of
+// both sides (a boundary face's neighbour is unused)
+struct FaceLoads {
+    FaceRaw raw;
+    float4 mom, so, sn, mo, mn, go[3], gn[3];
+};
+__device__ __forceinline__ FaceLoads load_face(const FluidArgs &a, const float4 *__restrict__ st,
+                                               const float4 *__restrict__ grad, const float4 *__restrict__ mu, int tf,
+                                               int o, int n)
+{
+    FaceLoads l;
+    l.raw = load_face_raw(a, tf);
+    l.mom = a.face_moments[tf];
+    l.so = st[o]; l.sn = st[n];
+    l.mo = mu[o]; l.mn = mu[n];
+#pragma unroll
+    for (int k = 0; k < 3; k++) { l.go[k] = grad[3 * (size_t)o + k]; l.gn[k] = grad[3 * (size_t)n + k]; }
+    return l;
+}
+__device__ __forceinline__ void grad_array(const float4 v[3], float g[12])
+{
+#pragma unroll
+    for (int k = 0; k < 3; k++) { g[4 * k] = v[k].x; g[4 * k + 1] = v[k].y; g[4 * k + 2] = v[k].z; g[4 * k + 3] = v[k].w; }
+}
+
+// reverse of the flux from the moments to the moments' adjoints; lam: the flux
+// adjoint (neighbour's residual adjoint less the owner's)
+template <class L>
+__device__ __forceinline__ FaceAdj flux_vjp(const FluidArgs &a, const FaceRec &fr, float4 fm, float4 lam, int o)
+{
+    const float nx = fr.nx, ny = fr.ny, nz = fr.nz, A = fr.A, ig = a.inv_gamma;
+    const float rho_f = a.rho0 + fm.x;
+    const float mnrm = fm.y * nx + fm.z * ny + fm.w * nz;
+    const float vf = a.visc_factor ? a.visc_factor[o] : 1.0f;
+    const float tau = a.visc3_over_gamma * vf / fr.dt;
+    const float c1 = 1.0f - tau;
+    const float irf = 1.0f / rho_f;
+    const float q = mnrm * irf * ig;
+    const float Lx = lam.y, Ly = lam.z, Lz = L::dims == 3 ? lam.w : 0.0f;
+    const float lq = A * c1 * (Lx * fm.y + Ly * fm.z + Lz * fm.w);
+    const float lmn = lam.x * A + lq * ig * irf;
+    const float lrf = -lq * mnrm * ig * irf * irf;
+    FaceAdj fj;
+    fj.lS0 = A * c1 * (Lx * nx + Ly * ny + Lz * nz) * (1.0f / 3.0f) + lrf;
+    fj.lS1x = Lx * A * c1 * q + lmn * nx;
+    fj.lS1y = Ly * A * c1 * q + lmn * ny;
+    fj.lS1z = Lz * A * c1 * q + lmn * nz;
+    fj.lTx = Lx * A * tau;
+    fj.lTy = Ly * A * tau;
+    fj.lTz = Lz * A * tau;
+    return fj;
+}
+
+// adjoint of the rest point (the mean state of both sides)
+template <class L>
+__device__ __forceinline__ void rest_vjp(const FluidArgs &a, const FaceAdj &fj, const float p0[4], float lp0[4])
+{
+    const float ig = a.inv_gamma, w0 = L::w(0);
+    const float P0 = -1.5f * (p0[1] * p0[1] + p0[2] * p0[2] + p0[3] * p0[3]) * ig;
+    lp0[0] = fj.lS0 * w0 * (1.0f + P0);
+    const float c = fj.lS0 * w0 * (a.rho0 + p0[0]) * (-3.0f * ig);
+    lp0[1] = c * p0[1];
+    lp0[2] = c * p0[2];
+    lp0[3] = c * p0[3];
+}
+
+// One side of a face whose lattice directions all lie clearly on one side
+// (FaceRec::general unset): the points along s e (s the direction's sign on
+// this side) come from this side alone, q = p - s dt (e.grad).  With R the
+// adjoint factor of a point's velocity terms and h that of its e.u, the point
+// adjoint of velocity u_t is -3/gamma R u_t + e_t h, linear in the side's p and
+// grad: only the moments of R, h and the density adjoint over the directions
+// are summed here, 14 sums a point in place of the 4 + 12 components' own
+// (with their selections on a tie): about 970 instructions a face for the 1350
+// of face_vjp, which faces with a tie keep.
+struct SideMoments {
+    float z0, z[3];         // density adjoint l: sum l, sum s e l
+    float m0, m[3], mm[6];  // sum R, sum s e R, sum e e R (xx, yy, zz, xy, xz, yz)
+    float h[3], hh[6];      // sum e h, sum s e e h
+};
+template <int EX, int EY, int EZ>
+__device__ __forceinline__ void point_vjp(SideMoments &m, const float p[4], const float g[12], float sdt, float s,
+                                          float s3, float lg, float rho0, float ig45, float ig15)
+{
+    float q[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) q[v] = fmaf(-sdt, edot<EX, EY, EZ>(g[3 * v], g[3 * v + 1], g[3 * v + 2]), p[v]);
+    const float x = edot<EX, EY, EZ>(q[1], q[2], q[3]);
+    const float uu = dot3(q[1], q[2], q[3], q[1], q[2], q[3]);
+    const float t = fmaf(ig45, x, s3);
+    const float P = fmaf(x, t, -ig15 * uu);
+    const float l = fmaf(lg, P, lg), R = lg * (rho0 + q[0]), h = R * fmaf(ig45, x, t);
+    m.z0 += l;
+    efma<EX>(m.z[0], s, l); efma<EY>(m.z[1], s, l); efma<EZ>(m.z[2], s, l);
+    m.m0 += R;
+    efma<EX>(m.m[0], s, R); efma<EY>(m.m[1], s, R); efma<EZ>(m.m[2], s, R);
+    eacc<EX * EX>(m.mm[0], R); eacc<EY * EY>(m.mm[1], R); eacc<EZ * EZ>(m.mm[2], R);
+    eacc<EX * EY>(m.mm[3], R); eacc<EX * EZ>(m.mm[4], R); eacc<EY * EZ>(m.mm[5], R);
+    eacc<EX>(m.h[0], h); eacc<EY>(m.h[1], h); eacc<EZ>(m.h[2], h);
+    efma<EX * EX>(m.hh[0], s, h); efma<EY * EY>(m.hh[1], s, h); efma<EZ * EZ>(m.hh[2], s, h);
+    efma<EX * EY>(m.hh[3], s, h); efma<EX * EZ>(m.hh[4], s, h); efma<EY * EZ>(m.hh[5], s, h);
+}
+template <class L, int K>
+__device__ __forceinline__ void pair_vjp_clear(SideMoments &mo, SideMoments &mn, const FaceAdj &fa, const float po[4],
+                                               const float pn[4], const float go[12], const float gn[12],
+                                               const FaceRec &fr, float rho0, float ig45, float ig15)
+{
+    constexpr int ex = L::ex[K], ey = L::ey[K], ez = L::ez[K];
+    constexpr float w = L::w(K);
+    const float en = edot<ex, ey, ez>(fr.nx, fr.ny, fr.nz);
+    const float sdt = copysignf(fr.dt, en), s = copysignf(1.0f, en), s3 = copysignf(3.0f, en);
+    const float lgs = w * fmaf(en, edot<ex, ey, ez>(fa.lTx, fa.lTy, fa.lTz), fa.lS0);
+    const float lgd = copysignf(w, en) * edot<ex, ey, ez>(fa.lS1x, fa.lS1y, fa.lS1z);
+    point_vjp<ex, ey, ez>(mo, po, go, sdt, s, s3, lgs + lgd, rho0, ig45, ig15);
+    point_vjp<ex, ey, ez>(mn, pn, gn, -sdt, -s, -s3, lgs - lgd, rho0, ig45, ig15);
+}
+template <class L, int... P>
+__device__ __forceinline__ void all_pair_vjps_clear(std::integer_sequence<int, P...>, SideMoments &mo,
+                                                    SideMoments &mn, const FaceAdj &fa, const float po[4],
+                                                    const float pn[4], const float go[12], const float gn[12],
+                                                    const FaceRec &fr, float rho0, float ig45, float ig15)
+{
+    (pair_vjp_clear<L, 2 * P + 1>(mo, mn, fa, po, pn, go, gn, fr, rho0, ig45, ig15), ...);
+}
+// a side's state (out[0]) and gradient (out[1..3]) adjoint from its moments
+// and the rest point's; d: its centroid's offset from the face
+__device__ __forceinline__ void side_vjp(const SideMoments &m, const float p[4], const float g[12], const float lp0[4],
+                                         float3 d, float dt, float ig, float4 out[4])
+{
+    const float c = -3.0f * ig, cd = c * dt, cdd = cd * dt;
+    const float m0 = c * m.m0, m1[3] = {cd * m.m[0], cd * m.m[1], cd * m.m[2]};
+    const float xx = cdd * m.mm[0], yy = cdd * m.mm[1], zz = cdd * m.mm[2];
+    const float xy = cdd * m.mm[3], xz = cdd * m.mm[4], yz = cdd * m.mm[5];
+    const float hx[3] = {m.hh[0], m.hh[3], m.hh[4]}, hy[3] = {m.hh[3], m.hh[1], m.hh[5]},
+                hz[3] = {m.hh[4], m.hh[5], m.hh[2]};
+    float ls[4], lg[12];
+    ls[0] = m.z0 + 0.5f * lp0[0];
+    lg[0] = -dt * m.z[0]; lg[1] = -dt * m.z[1]; lg[2] = -dt * m.z[2];
+#pragma unroll
+    for (int t = 0; t < 3; t++) {
+        const float gx = g[3 * t + 3], gy = g[3 * t + 4], gz = g[3 * t + 5], u = p[t + 1];
+        ls[t + 1] = m.h[t] + u * m0 - (gx * m1[0] + gy * m1[1] + gz * m1[2]) + 0.5f * lp0[t + 1];
+        lg[3 * t + 3] = (gx * xx + gy * xy + gz * xz) - u * m1[0] - dt * hx[t];
+        lg[3 * t + 4] = (gx * xy + gy * yy + gz * yz) - u * m1[1] - dt * hy[t];
+        lg[3 * t + 5] = (gx * xz + gy * yz + gz * zz) - u * m1[2] - dt * hz[t];
+    }
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        lg[3 * v] -= d.x * ls[v]; lg[3 * v + 1] -= d.y * ls[v]; lg[3 * v + 2] -= d.z * ls[v];
+    }
+    out[0] = make_float4(ls[0], ls[1], ls[2], ls[3]);
+    out[1] = make_float4(lg[0], lg[1], lg[2], lg[3]);
+    out[2] = make_float4(lg[4], lg[5], lg[6], lg[7]);
+    out[3] = make_float4(lg[8], lg[9], lg[10], lg[11]);
+}
+
+// Adjoint of the flux of a face clear of every lattice direction (laid out as
+// face_vjp's)
+template <class L>
+__device__ __forceinline__ void face_vjp_clear(const FluidArgs &a, const FaceLoads &in, const FaceRec &fr, int o,
+                                               float4 out[8])
+{
+    const float sov[4] = {in.so.x, in.so.y, in.so.z, in.so.w}, snv[4] = {in.sn.x, in.sn.y, in.sn.z, in.sn.w};
+    float go[12], gn[12], po[4], pn[4], p0[4], lp0[4];
+    grad_array(in.go, go);
+    grad_array(in.gn, gn);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        po[v] = sov[v] - (fr.d1.x * go[3 * v] + fr.d1.y * go[3 * v + 1] + fr.d1.z * go[3 * v + 2]);
+        pn[v] = snv[v] - (fr.d2.x * gn[3 * v] + fr.d2.y * gn[3 * v + 1] + fr.d2.z * gn[3 * v + 2]);
+        p0[v] = 0.5f * (po[v] + pn[v]);
+    }
+    const float4 lam = make_float4(in.mn.x - in.mo.x, in.mn.y - in.mo.y, in.mn.z - in.mo.z, in.mn.w - in.mo.w);
+    const FaceAdj fj = flux_vjp<L>(a, fr, in.mom, lam, o);
+    rest_vjp<L>(a, fj, p0, lp0);
+    const float ig = a.inv_gamma;
+    SideMoments mo = {}, mn = {};
+    all_pair_vjps_clear<L>(std::make_integer_sequence<int, (L::Q - 1) / 2>{}, mo, mn, fj, po, pn, go, gn, fr, a.rho0,
+                           4.5f * ig, 1.5f * ig);
+    side_vjp(mo, po, go, lp0, fr.d1, fr.dt, ig, out);
+    side_vjp(mn, pn, gn, lp0, fr.d2, fr.dt, ig, out + 4);
+}
+
 // Adjoint of one tile-face's flux (the forward of face_flux in
 // fluid_kernels.hip, strict upwinding), from the face's moments S0, S1 as the
 // forward pass computed them.  out[0] state and out[1..3] gradient
 // adjoint of the owner, out[4..7] the same for the neighbour (zero for a
-// boundary face, whose ghost is a function of the owner).
+// boundary face, whose ghost is a function of the owner).  Boundary faces, and
+// interior faces whose points may come from either side.
 template <class L, bool GHOST>
-__device__ __forceinline__ void face_vjp(const FluidArgs &a, const float4 *__restrict__ st,
-                                         const float4 *__restrict__ grad, const float4 *__restrict__ mu, int tf,
-                                         int o, int nb, float4 out[8])
+__device__ __forceinline__ void face_vjp(const FluidArgs &a, const FaceLoads &in, const FaceRec &fr, int o, int nb,
+                                         float4 out[8])
 {
-    const FaceRec fr = unpack_face(load_face_raw(a, tf));
     const float3 fb = fr.d1, fcv = fr.d2;
     constexpr bool ghost = GHOST;  // boundary faces follow the interior faces in every tile list
     const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
     for (int k = 0; k < 8; k++) out[k] = zero;
-    const float nx = fr.nx, ny = fr.ny, nz = fr.nz, A = fr.A, dt = fr.dt;
-    const float4 so = st[o];
-    const float4 mo = mu[o];
+    const float nx = fr.nx, ny = fr.ny, nz = fr.nz, dt = fr.dt;
+    const float4 so = in.so, mo = in.mo;
     float go[12], gn[12];
-    load_grad(grad, o, go);
+    grad_array(in.go, go);
     const float sov[4] = {so.x, so.y, so.z, so.w};
     float po[4], pn[4], p0[4];
     float4 lam;
     int ty[4] = {0, 0, 0, 0};
     float inv_dmag = 0.0f, dir[3] = {0.0f, 0.0f, 0.0f}, fac[3] = {1.0f, 1.0f, 1.0f};
     if (!ghost) {
-        const float4 sn = st[nb], mn4 = mu[nb];
+        const float4 sn = in.sn, mn4 = in.mn;
         lam = make_float4(mn4.x - mo.x, mn4.y - mo.y, mn4.z - mo.z, mn4.w - mo.w);
-        load_grad(grad, nb, gn);
+        grad_array(in.gn, gn);
         const float snv[4] = {sn.x, sn.y, sn.z, sn.w};
 #pragma unroll
         for (int v = 0; v < 4; v++) {
@@ -260,44 +442,9 @@ __device__ __forceinline__ void face_vjp(const FluidArgs &a, const float4 *__res
 #pragma unroll
     for (int t = 0; t < 12; t++) { Go[t] = go[t] * dt; Gn[t] = gn[t] * dt; }
     const float rho0 = a.rho0, ig = a.inv_gamma;
-    // forward moments S0, S1 of this face, kept by the forward pass
-    const float4 fm = a.face_moments[tf];
-    FaceSums f;
-    f.S0 = fm.x;
-    f.S1x = fm.y;
-    f.S1y = fm.z;
-    f.S1z = fm.w;
-    const float P0 = -1.5f * (p0[1] * p0[1] + p0[2] * p0[2] + p0[3] * p0[3]) * ig;
-    const float rho_f = rho0 + f.S0;
-    const float mnrm = f.S1x * nx + f.S1y * ny + f.S1z * nz;
-    const float vf = a.visc_factor ? a.visc_factor[o] : 1.0f;
-    const float tau = a.visc3_over_gamma * vf / dt;
-    const float c1 = 1.0f - tau;
-    const float irf = 1.0f / rho_f;
-    const float q = mnrm * irf * ig;
-    // reverse of the flux from the moments
-    const float Lx = lam.y, Ly = lam.z, Lz = L::dims == 3 ? lam.w : 0.0f;
-    const float lq = A * c1 * (Lx * f.S1x + Ly * f.S1y + Lz * f.S1z);
-    const float lmn = lam.x * A + lq * ig * irf;
-    const float lrf = -lq * mnrm * ig * irf * irf;
-    FaceAdj fj;
-    fj.lS0 = A * c1 * (Lx * nx + Ly * ny + Lz * nz) * (1.0f / 3.0f) + lrf;
-    fj.lS1x = Lx * A * c1 * q + lmn * nx;
-    fj.lS1y = Ly * A * c1 * q + lmn * ny;
-    fj.lS1z = Lz * A * c1 * q + lmn * nz;
-    fj.lTx = Lx * A * tau;
-    fj.lTy = Ly * A * tau;
-    fj.lTz = Lz * A * tau;
-    // rest point
+    const FaceAdj fj = flux_vjp<L>(a, fr, in.mom, lam, o);
     float lp0[4];
-    {
-        const float w0 = L::w(0);
-        lp0[0] = fj.lS0 * w0 * (1.0f + P0);
-        const float c = fj.lS0 * w0 * (rho0 + p0[0]) * (-3.0f * ig);
-        lp0[1] = c * p0[1];
-        lp0[2] = c * p0[2];
-        lp0[3] = c * p0[3];
-    }
+    rest_vjp<L>(a, fj, p0, lp0);
     float lpo[4] = {0.0f, 0.0f, 0.0f, 0.0f}, lpn[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     float lGo[12], lGn[12];
 #pragma unroll
@@ -361,8 +508,8 @@ __device__ __forceinline__ void face_vjp(const FluidArgs &a, const float4 *__res
     out[3] = make_float4(lgo_[8], lgo_[9], lgo_[10], lgo_[11]);
 }
 
-constexpr int ADJ_THREADS = 512;
-constexpr int ADJ_CHUNK = 512;       // faces per LDS chunk (8 float4 each: 64 KiB), held as 8 planes
+constexpr int ADJ_THREADS = 256;
+constexpr int ADJ_CHUNK = 256;       // faces per LDS chunk (8 float4 each: 32 KiB), held as 8 planes
                                      // of ADJ_CHUNK float4 so that a wavefront's stores are contiguous
 
 __device__ __forceinline__ void add4(float *acc, float4 v)
@@ -370,57 +517,65 @@ __device__ __forceinline__ void add4(float *acc, float4 v)
     acc[0] += v.x; acc[1] += v.y; acc[2] += v.z; acc[3] += v.w;
 }
 
-// ADJ_CELLS: cells per thread (1: tiles of up to 512 cells, 2: up to 1024)
+// Bound by its waits: each chunk's loads, its faces and its sums follow one
+// another behind barriers, and some 180 registers leave two wavefronts a SIMD.
+// Workgroups of 256 threads put two of them on a compute unit, one's faces
+// beside the other's loads and sums.  128x64x64, D3Q19, 8x8x8 tiles: 512
+// threads 111 us, with the moments of face_vjp_clear (37.4 -> 30.9 M vector
+// instructions) 112; 256 threads 87.  Three workgroups in 168 registers take
+// 107 (spills), or 96 with one side of a face after the other; the next
+// chunk's loads issued ahead gain nothing at two.
+// ADJ_CELLS: cells per thread (tiles of up to 256, 512 or 1024 cells)
 template <class L, int ADJ_CELLS>
 __global__ __launch_bounds__(ADJ_THREADS) void k_adj_flux(FluidArgs a, AdjFluidArgs j, const float4 *__restrict__ st,
                                                           const float4 *__restrict__ grad)
 {
     extern __shared__ float4 lds_adj[];
     const TileRec T = a.tiles[xcd_remap(blockIdx.x, gridDim.x)];
-    const int f0 = T.f0, f1 = T.f0 + T.nf, c0 = T.c0, c1 = T.c0 + T.nc, fb = T.f0 + T.nif;
+    const int c0 = T.c0, c1 = T.c0 + T.nc;
+    int *ids = reinterpret_cast<int *>(lds_adj + 8 * ADJ_CHUNK);  // cell id of each slot
+    for (int q = threadIdx.x; q < T.nc + T.nh; q += ADJ_THREADS) ids[q] = slot_cell(a, T, q);
     float acc[ADJ_CELLS][16];
-    uint32_t slot[ADJ_CELLS][6];
+    uint32_t slot[ADJ_CELLS][3];  // two slots each; 0x7fff: none
 #pragma unroll
     for (int u = 0; u < ADJ_CELLS; u++) {
 #pragma unroll
         for (int k = 0; k < 16; k++) acc[u][k] = 0.0f;
-        const int i = c0 + (int)threadIdx.x + u * ADJ_THREADS;
-        if (i < c1) {
-            const uint32_t *sl = reinterpret_cast<const uint32_t *>(a.cell_slots) + 3 * (size_t)(T.pc + i - c0);
-            const uint32_t s01 = sl[0], s23 = sl[1], s45 = sl[2];
-            slot[u][0] = s01 & 0xffffu; slot[u][1] = s01 >> 16;
-            slot[u][2] = s23 & 0xffffu; slot[u][3] = s23 >> 16;
-            slot[u][4] = s45 & 0xffffu; slot[u][5] = s45 >> 16;
-        } else {
+        const int i = (int)threadIdx.x + u * ADJ_THREADS;
+        const uint32_t *sl = reinterpret_cast<const uint32_t *>(a.cell_slots) + 3 * (size_t)(T.pc + i);
 #pragma unroll
-            for (int k = 0; k < 6; k++) slot[u][k] = 0xffffffffu;
-        }
+        for (int k = 0; k < 3; k++) slot[u][k] = i < T.nc ? sl[k] : 0x7fff7fffu;
     }
-    for (int cs = f0; cs < f1; cs += ADJ_CHUNK) {
-        const int ce = cs + ADJ_CHUNK < f1 ? cs + ADJ_CHUNK : f1;
-        for (int f = cs + threadIdx.x; f < ce; f += ADJ_THREADS) {
+    const int last = T.nc + T.nh - 1;
+    __syncthreads();
+    for (int cs = 0; cs < T.nf; cs += ADJ_CHUNK) {
+        const int q = cs + (int)threadIdx.x;
+        if (q < T.nf) {
+            // (a boundary face's neighbour slot is 0xffff: some cell of the tile's, unused)
+            const uint32_t gs = a.face_gslot[T.pf + q];
+            const int oc = ids[gs & 0xffffu];
+            const FaceLoads in = load_face(a, st, grad, j.mu, T.f0 + q, oc, ids[min((int)(gs >> 16), last)]);
+            const FaceRec fr = unpack_face(in.raw);
             float4 o[8];
-            const uint32_t gs = a.face_gslot[T.pf + f - f0];
-            const int oc = slot_cell(a, T, gs & 0xffffu), nb = face_neighbour(a, T, gs, f - f0);
-            if (f < fb) face_vjp<L, false>(a, st, grad, j.mu, f, oc, nb, o);
-            else face_vjp<L, true>(a, st, grad, j.mu, f, oc, nb, o);
+            if (!fr.general) face_vjp_clear<L>(a, in, fr, oc, o);
+            else if (q < T.nif) face_vjp<L, false>(a, in, fr, oc, 0, o);
+            else face_vjp<L, true>(a, in, fr, oc, a.n_cells + a.tile_bc[T.b0 + q - T.nif], o);
 #pragma unroll
-            for (int k = 0; k < 8; k++) lds_adj[k * ADJ_CHUNK + (f - cs)] = o[k];
+            for (int k = 0; k < 8; k++) lds_adj[k * ADJ_CHUNK + threadIdx.x] = o[k];
         }
         __syncthreads();
-        const uint32_t base = (uint32_t)(cs - f0), n = (uint32_t)(ce - cs);
+        const uint32_t base = (uint32_t)cs, n = (uint32_t)min(ADJ_CHUNK, T.nf - cs);
 #pragma unroll
         for (int u = 0; u < ADJ_CELLS; u++)
 #pragma unroll
             for (int k = 0; k < 6; k++) {
-                const uint32_t s = slot[u][k];
-                if (s == 0xffffffffu) continue;
+                const uint32_t s = slot[u][k / 2] >> 16 * (k & 1);
                 const uint32_t r = (s & 0x7fffu) - base;
                 if (r >= n) continue;
                 const int side = (s & 0x8000u) ? 0 : 4;  // bit 15 set: the cell owns the face
                 const float4 *src = lds_adj + side * ADJ_CHUNK + r;
 #pragma unroll
-                for (int q = 0; q < 4; q++) add4(&acc[u][4 * q], src[q * ADJ_CHUNK]);
+                for (int v = 0; v < 4; v++) add4(&acc[u][4 * v], src[v * ADJ_CHUNK]);
             }
         __syncthreads();
     }
@@ -557,15 +712,17 @@ static void launch_adj_flux_l(const FluidArgs &a, const AdjFluidArgs &j, const f
 {
     if (cells_per_thread == 1)
         hipLaunchKernelGGL((k_adj_flux<L, 1>), dim3(a.n_tiles), dim3(ADJ_THREADS), lds, s, a, j, st, grad);
-    else
+    else if (cells_per_thread == 2)
         hipLaunchKernelGGL((k_adj_flux<L, 2>), dim3(a.n_tiles), dim3(ADJ_THREADS), lds, s, a, j, st, grad);
+    else
+        hipLaunchKernelGGL((k_adj_flux<L, 4>), dim3(a.n_tiles), dim3(ADJ_THREADS), lds, s, a, j, st, grad);
 }
 
 hipError_t launch_adj_flux(const FluidArgs &a, const AdjFluidArgs &j, const float4 *st, const float4 *grad,
                            int max_tile_cells, hipStream_t s)
 {
-    const size_t lds = sizeof(float4) * 8 * (size_t)ADJ_CHUNK;
-    const int cpt = max_tile_cells <= ADJ_THREADS ? 1 : 2;
+    const size_t lds = sizeof(float4) * 8 * (size_t)ADJ_CHUNK + sizeof(int) * (size_t)a.max_grad_slots;
+    const int cpt = (max_tile_cells + ADJ_THREADS - 1) / ADJ_THREADS;
     switch (a.lattice) {
     case LBFS_D3Q15: launch_adj_flux_l<D3Q15>(a, j, st, grad, cpt, lds, s); break;
     case LBFS_D3Q19: launch_adj_flux_l<D3Q19>(a, j, st, grad, cpt, lds, s); break;
