@@ -245,36 +245,16 @@ int adjoint_setup(lbfs_ctx *ctx, int n_steps, int every)
     A.n_fpart = (n + 255) / 256;
     if ((rc = adj_alloc(ctx, &A.fpart, 3 * (size_t)A.n_fpart))) return rc;
     if ((rc = adj_alloc(ctx, &A.gforce, 3))) return rc;
-    // reverse stencil rows: for slot k of cell i with neighbour c, the sum of
-    // the weight vectors of c's slots that point back to i; every such slot
-    // of c is claimed by exactly one slot of i (the stencil is symmetric on
-    // face-neighbour meshes; anything else is refused)
+    // reverse stencil rows; a stencil that is not symmetric (none on meshes of
+    // face neighbours) is refused
     {
-        const std::vector<int> &sten = ctx->lay.stencil;
-        const std::vector<float> &gw = ctx->lay.gw;
-        std::vector<float4> rw(6 * (size_t)n, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
-        std::vector<unsigned char> used(6 * (size_t)n, 0);
-        for (int i = 0; i < n; i++)
-            for (int k = 0; k < 6; k++) {
-                const int c = sten[(size_t)k * n + i];
-                if (c < 0) continue;
-                for (int kb = 0; kb < 6; kb++) {
-                    if (used[(size_t)kb * n + c] || sten[(size_t)kb * n + c] != i) continue;
-                    used[(size_t)kb * n + c] = 1;
-                    float4 &w = rw[(size_t)k * n + i];
-                    w.x += gw[(size_t)(3 * kb) * n + c];
-                    w.y += gw[(size_t)(3 * kb + 1) * n + c];
-                    w.z += gw[(size_t)(3 * kb + 2) * n + c];
-                    break;
-                }
-            }
-        for (int i = 0; i < n; i++)
-            for (int k = 0; k < 6; k++)
-                if (sten[(size_t)k * n + i] >= 0 && !used[(size_t)k * n + i])
-                    return ctx->fail(LBFS_E_UNSUPPORTED, "the adjoint needs a symmetric gradient stencil");
-        if ((rc = adj_alloc(ctx, &A.rev_w, rw.size()))) return rc;
-        HIPCHK(hipMemcpyAsync(A.rev_w, rw.data(), sizeof(float4) * rw.size(), hipMemcpyHostToDevice, ctx->stream));
-        HIPCHK(hipStreamSynchronize(ctx->stream));  // (rw is freed at the end of the block)
+        unsigned int *lone, h = 0;
+        if ((rc = adj_alloc(ctx, &A.rev_w, 6 * (size_t)n))) return rc;
+        if ((rc = adj_alloc(ctx, &lone, 1))) return rc;
+        HIPCHK(launch_adj_rev_rows(ctx->args, A.rev_w, lone, ctx->stream));
+        HIPCHK(hipMemcpyAsync(&h, lone, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
+        HIPCHK(hipStreamSynchronize(ctx->stream));
+        if (h) return ctx->fail(LBFS_E_UNSUPPORTED, "the adjoint needs a symmetric gradient stencil");
     }
     if (ctx->have_membranes) {
         const MemArgs &m = ctx->mem;

@@ -28,7 +28,7 @@ struct AdjFluidArgs {
     double *fpart;             // [3 blocks] running per-block sums of the cell-force adjoint
     double *gforce;            // [3] gradient of the uniform body force (sum of fpart)
     const float4 *rev_w;       // [6 n] SoA: for stencil slot k of cell i (neighbour c), the weight
-                               // vector of c's stencil rows that point back to i (x, y, z)
+                               // vector of c's stencil row that points back to i (x, y, z)
     const unsigned long long *acc;  // [3 n] fixed-point adjoint of the interpolated velocity, or null
     unsigned long long *acc_rw;
     const unsigned int *umax;  // float bits of the largest |adjoint node velocity| (fixed-point scale)
@@ -75,6 +75,10 @@ __device__ __forceinline__ double adj_fix_inv_scale(unsigned int m)
     frexpf(x, &e);
     return ldexp(1.0, e - 40);
 }
+
+// rev_w of AdjFluidArgs from the stencil and its weights (set-up); *lone set
+// where a slot has no slot of its neighbour that points back
+hipError_t launch_adj_rev_rows(const FluidArgs &a, float4 *rev_w, unsigned int *lone, hipStream_t s);
 
 hipError_t launch_adj_update(const FluidArgs &a, const AdjFluidArgs &j, const float4 *st, const float4 *res,
                              hipStream_t s);

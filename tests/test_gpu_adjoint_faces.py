@@ -48,3 +48,28 @@ def test_state_adjoint_of_face_classes(lat_a, lat_o, jitter, tile, threads, flag
     # some 10 single-precision sums a step (6e-8 each), of independent sign
     # over the cells; the differences' own error is below 1e-8 of it
     assert abs(ad.sum() - fd) < 1e-5 * np.sqrt(np.sum(ad * ad)), (ad.sum(), fd)
+
+
+@pytest.mark.parametrize("size,periodic", [((2, 7, 2), (1, 0, 1)), ((2, 2, 2), (1, 1, 1)), ((5, 1, 4), (1, 1, 1))])
+def test_state_adjoint_of_repeated_neighbours(size, periodic):
+    """Two layers and one between periodic sides: a cell meets a neighbour, or
+    itself, through two faces."""
+    mesh = abi.HexMesh(*size, periodic=periodic, jitter=0.1, seed=3)
+    st = cases.smooth_state(mesh, seed=6, amp=0.005)
+    rng = np.random.default_rng(8)
+    c = rng.standard_normal((mesh.n_cells, 4))
+    v = 1e-3 * rng.standard_normal((mesh.n_cells, 4))
+    s = abi.Solver(mesh, abi.make_params(lattice=abi.D3Q19, visc=VISC, dt=DT))
+    s.set_state(*st)
+    s.adjoint_forward(STEPS, 3)
+    ad = s.adjoint_backward(lam_state=c)["state0"] * v
+    s.close()
+
+    def loss(eps):
+        o = orc.OracleFluid(mesh, orc.OR_D3Q19, visc=VISC, dt=DT)
+        o.set_state(*(st[k] + eps * v[:, k] for k in range(4)))
+        o.step(STEPS)
+        return float(np.sum(c * np.stack(o.state(), axis=1)))
+
+    fd = (loss(1e-3) - loss(-1e-3)) / 2e-3
+    assert abs(ad.sum() - fd) < 1e-5 * np.sqrt(np.sum(ad * ad)), (ad.sum(), fd)  # (as above)
