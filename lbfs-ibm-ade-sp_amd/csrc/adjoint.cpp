@@ -65,7 +65,7 @@ struct AdjointState {
     hipStream_t rs = nullptr;     // stream of the overlapped replays: one, so that the process's
                                   // streams stay within its hardware queues (four by default) and
                                   // no replay kernel queues behind a reverse kernel
-    hipEvent_t rev[7] = {};       // replay fork and joins, records ready (2), records reversed (2)
+    hipEvent_t rev[4] = {};       // records ready (2), records reversed (2)
     // fluid adjoint
     float4 *lam_st[2] = {nullptr, nullptr};
     float4 *mu = nullptr, *lcf = nullptr, *ls = nullptr, *ls_acc = nullptr, *lam_g = nullptr;
@@ -296,14 +296,19 @@ int adjoint_setup(lbfs_ctx *ctx, int n_steps, int every)
 // `st` (the record's start state), keeping what the reverse step reads; the
 // new state goes to `st_next`.  The kernels and their order are those of
 // lbfs_step.
-// streams and events a replay runs on: the context's own, or those of the
-// overlapped replays
+// streams and events a replay runs on: the context's own (one of them on small
+// meshes, as in the time step), or that of the overlapped replays; no events
+// where the streams are one
 struct Lanes {
     hipStream_t main, side, side2;
     hipEvent_t fork, join, join2;
 };
-Lanes ctx_lanes(lbfs_ctx *ctx) { return {ctx->stream, ctx->side, ctx->side2, ctx->ev_fork, ctx->ev_join, ctx->ev_join2}; }
-Lanes replay_lanes(AdjointState &A) { return {A.rs, A.rs, A.rs, A.rev[0], A.rev[1], A.rev[2]}; }
+Lanes ctx_lanes(lbfs_ctx *ctx)
+{
+    if (ctx->lay.n_cells <= ONE_STREAM_CELLS) return {ctx->stream, ctx->stream, ctx->stream, nullptr, nullptr, nullptr};
+    return {ctx->stream, ctx->side, ctx->side2, ctx->ev_fork, ctx->ev_join, ctx->ev_join2};
+}
+Lanes replay_lanes(AdjointState &A) { return {A.rs, A.rs, A.rs, nullptr, nullptr, nullptr}; }
 
 // the fluid pass of a replayed step, keeping its gradients and face moments:
 // the fused pass where the step uses it (it writes the gradients as well),
@@ -322,8 +327,6 @@ hipError_t replay_fluid(const lbfs_ctx *ctx, FluidArgs a, StepRec &r, const floa
 
 int replay_step(lbfs_ctx *ctx, StepRec &r, const float4 *st, float4 *st_next, const Lanes &q)
 {
-    const hipMemcpyKind k = hipMemcpyDeviceToDevice;
-    const size_t n = (size_t)ctx->lay.n_cells;
     if (!ctx->have_membranes) {
         HIPCHK(replay_fluid(ctx, ctx->args, r, st, st_next, q.main));
         return LBFS_OK;
@@ -333,24 +336,28 @@ int replay_step(lbfs_ctx *ctx, StepRec &r, const float4 *st, float4 *st_next, co
     // node binning; the node kernels write into the record (X^n is advected
     // in r.Xn1; U^n, F^n and the step's globals land in r.U, r.F, r.glob)
     MemArgs m = ctx->mem;
-    const size_t nn = m.n_nodes, nm = m.n_mem;
-    HIPCHK(hipMemcpyAsync(r.Xn1, r.X, sizeof(float4) * nn, k, q.main));
-    HIPCHK(hipMemcpyAsync(r.glob, r.glob_prev, sizeof(double) * 8 * nm, k, q.main));
     m.X = r.Xn1;
+    m.X_from = r.X;
+    m.glob_from = r.glob_prev;
     m.U = r.U;
     m.F = r.F;
     m.glob = r.glob;
     HIPCHK(launch_ibm_interp(m, ctx->ibm, st, q.main));
-    HIPCHK(hipEventRecord(q.fork, q.main));
-    HIPCHK(hipStreamWaitEvent(q.side, q.fork, 0));
+    const bool lanes = q.side != q.main;
+    if (lanes) {
+        HIPCHK(hipEventRecord(q.fork, q.main));
+        HIPCHK(hipStreamWaitEvent(q.side, q.fork, 0));
+        HIPCHK(hipStreamWaitEvent(q.side2, q.fork, 0));
+    }
     HIPCHK(replay_fluid(ctx, ctx->args, r, st, st_next, q.side));
-    HIPCHK(hipEventRecord(q.join, q.side));
-    HIPCHK(hipStreamWaitEvent(q.side2, q.fork, 0));
+    if (lanes) HIPCHK(hipEventRecord(q.join, q.side));
     HIPCHK(launch_mem_forces(m, !spread_gathers_forces(ctx->ibm), q.side2));
-    HIPCHK(hipEventRecord(q.join2, q.side2));
-    HIPCHK(hipStreamWaitEvent(q.main, q.join2, 0));
+    if (lanes) {
+        HIPCHK(hipEventRecord(q.join2, q.side2));
+        HIPCHK(hipStreamWaitEvent(q.main, q.join2, 0));
+    }
     HIPCHK(launch_ibm_spread(m, ctx->ibm, m.n_force_wg > 0, q.main));
-    HIPCHK(hipStreamWaitEvent(q.main, q.join, 0));
+    if (lanes) HIPCHK(hipStreamWaitEvent(q.main, q.join, 0));
     // the step's cell force goes straight into the record (every cell)
     lbfs::ApplyArgs p = ctx->apply_args(st_next, r.cf, 1);
     p.glob = m.glob;
@@ -387,11 +394,17 @@ int reverse_step(lbfs_ctx *ctx, const StepRec &r, bool first, int &cur_l, bool u
         return LBFS_OK;
     }
     // the face adjoint (side stream) beside the coupling adjoint chain; both
-    // read only the update's adjoint, and the gradient transpose waits for both
-    HIPCHK(hipEventRecord(ctx->ev_fork, ctx->stream));
-    HIPCHK(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
-    HIPCHK(launch_adj_flux(a, j, r.st, r.grad, A.max_tile_cells, ctx->side));
-    HIPCHK(hipEventRecord(ctx->ev_join, ctx->side));
+    // read only the update's adjoint, and the gradient transpose waits for
+    // both.  On small meshes the two waits cost more than the overlap gains
+    // (a 12-step gradient on 6144 cells: 1.95 -> 1.47 ms with this and the
+    // replay's copies and same-stream events taken out).
+    const bool fork = ctx->lay.n_cells > ONE_STREAM_CELLS;
+    if (fork) {
+        HIPCHK(hipEventRecord(ctx->ev_fork, ctx->stream));
+        HIPCHK(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
+    }
+    HIPCHK(launch_adj_flux(a, j, r.st, r.grad, A.max_tile_cells, fork ? ctx->side : ctx->stream));
+    if (fork) HIPCHK(hipEventRecord(ctx->ev_join, ctx->side));
     MemArgs m = ctx->mem;
     m.X = r.Xn1; m.U = r.U; m.F = r.F; m.glob = r.glob;
     AdjMemArgs jm{};
@@ -402,7 +415,7 @@ int reverse_step(lbfs_ctx *ctx, const StepRec &r, bool first, int &cur_l, bool u
     jm.mad_lag = first ? 0 : 1;
     jm.echunk = A.echunk; jm.echunk_start = A.echunk_start; jm.epart = A.epart; jm.n_echunks = A.n_echunks;
     HIPCHK(launch_adj_coupling(m, ctx->ibm, jm, ctx->stream));
-    HIPCHK(hipStreamWaitEvent(ctx->stream, ctx->ev_join, 0));
+    if (fork) HIPCHK(hipStreamWaitEvent(ctx->stream, ctx->ev_join, 0));
     HIPCHK(launch_adj_grad(a, j, prev ? &pv : nullptr, ctx->stream));
     cur_l ^= 1;
     return LBFS_OK;
@@ -565,7 +578,7 @@ extern "C" int lbfs_adjoint_backward(lbfs_ctx *ctx, const double *lam_nodes, con
     // runs on the context's: it waits until the reverse of the segment after
     // has released its set, and the reverse of a segment waits for its replay.
     std::vector<StepRec> *sets[2] = {&A.rec, &A.rec2};
-    hipEvent_t *ready = A.rev + 3, *reversed = A.rev + 5;
+    hipEvent_t *ready = A.rev, *reversed = A.rev + 2;
     if (!A.last_in_rec) {
         if (n_seg > 1) {
             HIPCHK(hipEventRecord(ready[1], ctx->stream));  // the seeds above come first

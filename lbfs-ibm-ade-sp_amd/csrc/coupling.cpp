@@ -175,7 +175,7 @@ extern "C" int lbfs_add_membranes(lbfs_ctx *ctx, const lbfs_membrane_desc *mem, 
     if ((rc = cp_alloc<double>(ctx, &ctx->mem_energy, nullptr, 7 * (size_t)count))) return rc;
     m.mem_node_start = dns;
     m.bbox = dbb;
-    m.X = dX; m.U = dU; m.F = dF; m.node_mem = dnm; m.origin = dorig; m.node_origin = dnorig; m.tri = dtri;
+    m.X = dX; m.X_from = dX; m.U = dU; m.F = dF; m.node_mem = dnm; m.origin = dorig; m.node_origin = dnorig; m.tri = dtri;
     m.mem_tri_start = dts; m.mem_edge_start = des0; m.edges = dedg; m.edge_mem = dem;
     m.edge_const = dec; m.edge_area0 = dea; m.edge_state = des; m.edge_force = def;
     std::vector<int2> force_wg;

@@ -33,6 +33,8 @@ struct MemParamDev {
 struct MemArgs {
     int n_mem, n_nodes, n_tri, n_edges;
     float4 *X;                // node position relative to the membrane origin
+    const float4 *X_from;     // positions the interpolation advects into X (X itself in the time step)
+    const double *glob_from;  // globals the interpolation first copies to glob, or null
     float4 *U;                // node velocity (interpolated)
     float4 *F;                // node force
     const int *node_mem;

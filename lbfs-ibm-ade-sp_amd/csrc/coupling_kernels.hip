@@ -150,7 +150,8 @@ __global__ __launch_bounds__(256) void k_ibm_interp(MemArgs m, IbmArgs g, const 
     const int nd = live ? gid / L : m.n_nodes - 1;  // dead lanes shadow a live node for the group sums
     const IbmBlock B = node_block<ONE>(g, nd);
     const float4 o = m.node_origin[nd];
-    float4 xl = m.X[nd];
+    if (INTERP && m.glob_from && gid < 8 * m.n_mem) m.glob[gid] = m.glob_from[gid];
+    float4 xl = m.X_from[nd];
     float *col = g.wnode + 64 * (size_t)nd + r;  // this lane's S weights, L apart
     if constexpr (INTERP) {
         const int4 nb = g.nbase[nd];
