@@ -80,12 +80,14 @@ struct lbfs_ctx {
     lbfs::AdjointState *adj = nullptr;
 
     // hipGraphs of graph_steps(k) consecutive steps (even numbers) starting from
-    // cur == 0, captured when a run first has that many (8 coupled steps hold
-    // some 60 launches, whose capture a first run pays for).  A graph launch costs the
-    // host 16 us and the device a gap of 3-5 us however many steps it holds: per
-    // step of 64x64 cells 8.0 us in graphs of two, 5.7 of 8, 5.2 of 32, and 5.9
-    // launched one by one; of 128x64x64 40.6, 39.1 and 38.9, with its cell (six
-    // launches on two streams) 62.6, 61.8 and 61.8.
+    // cur == 0.  A graph launch costs the host 16 us and the device a gap of 3-5
+    // us however many steps it holds: per step of 64x64 cells 8.0 us in graphs of
+    // two, 5.7 of 8, 5.2 of 32, and 5.9 launched one by one; of 128x64x64 40.6,
+    // 39.1 and 38.9, with its cell (six launches on two streams) 62.6, 61.8 and
+    // 61.8.  Capturing the long graph costs as much as it saves over some 200 to
+    // 600 steps, so a solver takes it from its LONG_GRAPH_AFTER-th step on.
+    static constexpr long long LONG_GRAPH_AFTER = 256;
+    long long steps_enqueued = 0;   // steps of enqueue_steps so far
     int graph_steps(int k) const { return k == 1 ? 2 : (have_membranes ? 8 : 32); }
     int schedule_option = 0;        // LBFS_OPT_STEP_SCHEDULE
     bool fused_ok = false;          // the tiles fit the fused fluid pass's LDS

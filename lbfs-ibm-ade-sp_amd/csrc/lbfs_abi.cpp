@@ -439,7 +439,11 @@ int lbfs_ctx::enqueue_steps(int nsteps)
             if (rc) return rc;
             s++;
         }
-        for (int k = 0; k < 2; k++) {
+        steps_enqueued += nsteps;
+        for (int k = steps_enqueued < LONG_GRAPH_AFTER ? 1 : 0; k < 2; k++) {
+            // (one launch a step: the rest of a run is as fast launched one by
+            // one as in pairs)
+            if (k == 1 && !have_membranes && args.ts_mode != LBFS_TS_MIN) break;
             // graphs of this many steps, falling back to single eager steps
             // where the internal viscosity field is due
             const int gs = graph_steps(k);
@@ -467,9 +471,6 @@ int lbfs_ctx::enqueue_steps(int nsteps)
                 t_step += gs;
                 s += gs;
             }
-            // (one launch a step: the rest of a run is as fast launched one by
-            // one as in pairs)
-            if (!have_membranes && args.ts_mode != LBFS_TS_MIN) break;
         }
     }
     for (; s < nsteps; s++) {
