@@ -179,17 +179,19 @@ public:
         if (e_ != hipSuccess) return ctx->fail(LBFS_E_HIP, "%s: %s", #expr, hipGetErrorString(e_)); \
     } while (0)
 
-// both staging buffers, of `bytes` each (grown if a larger transfer comes)
-int staging(lbfs_ctx *ctx, size_t bytes)
+// the staging buffers of a transfer of `chunks` chunks of up to `bytes` (grown if
+// a larger transfer comes): a single chunk needs one, whose allocation is most
+// of a small mesh's first readback
+int staging(lbfs_ctx *ctx, size_t bytes, size_t chunks)
 {
     Staging &s = ctx->staging;
-    if (s.bytes >= bytes) return LBFS_OK;
-    s.release();
-    for (int k = 0; k < 2; k++) {
-        HIPCHK(hipHostMalloc((void **)&s.buf[k], bytes, hipHostMallocDefault));
-        HIPCHK(hipEventCreateWithFlags(&s.ev[k], hipEventDisableTiming));
+    if (s.bytes < bytes) s.release();
+    const size_t size = std::max(bytes, s.bytes);
+    for (size_t k = 0; k < std::min<size_t>(2, chunks); k++) {
+        if (!s.ev[k]) HIPCHK(hipEventCreateWithFlags(&s.ev[k], hipEventDisableTiming));
+        if (!s.buf[k]) HIPCHK(hipHostMalloc((void **)&s.buf[k], size, hipHostMallocDefault));
     }
-    s.bytes = bytes;
+    s.bytes = size;
     return LBFS_OK;
 }
 
@@ -199,10 +201,10 @@ int stream_out(lbfs_ctx *ctx, size_t n, size_t item, const std::function<hipErro
                const std::function<std::vector<Piece>(int, int, const double *)> &segments)
 {
     const size_t per = std::max<size_t>(1, CHUNK_BYTES / item);
-    int rc = staging(ctx, std::min(n, per) * item);
+    const size_t chunks = (n + per - 1) / per;
+    int rc = staging(ctx, std::min(n, per) * item, chunks);
     if (rc) return rc;
     Staging &s = ctx->staging;
-    const size_t chunks = (n + per - 1) / per;
     CopyTeam team(n * item);
     auto start = [&](size_t k) -> hipError_t {
         const size_t i0 = k * per, m = std::min(per, n - i0);
@@ -273,7 +275,7 @@ int read_nodes(lbfs_ctx *ctx, double *X, double *U, double *F)
 int write_cells(lbfs_ctx *ctx, const double *src, float4 *dst)
 {
     const size_t n = (size_t)ctx->lay.n_cells, per = CHUNK_BYTES / 32, chunks = (n + per - 1) / per;
-    int rc = staging(ctx, std::min(n, per) * 32);
+    int rc = staging(ctx, std::min(n, per) * 32, chunks);
     if (rc) return rc;
     Staging &s = ctx->staging;
     CopyTeam team(n * 32);
