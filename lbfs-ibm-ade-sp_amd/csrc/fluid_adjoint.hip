@@ -521,8 +521,8 @@ __device__ __forceinline__ void add4(float *acc, float4 v)
 // another behind barriers, and some 180 registers leave two wavefronts a SIMD.
 // Workgroups of 256 threads put two of them on a compute unit, one's faces
 // beside the other's loads and sums.  128x64x64, D3Q19, 8x8x8 tiles: 512
-// threads 111 us, with the moments of face_vjp_clear (37.4 -> 30.9 M vector
-// instructions) 112; 256 threads 87.  Three workgroups in 168 registers take
+// threads 111 us, with the moments of face_vjp_clear (37.4 -> 29.6 M vector
+// instructions) 112; 256 threads 85.  Three workgroups in 168 registers take
 // 107 (spills), or 96 with one side of a face after the other; the next
 // chunk's loads issued ahead gain nothing at two.
 // ADJ_CELLS: cells per thread (tiles of up to 256, 512 or 1024 cells)
