@@ -365,7 +365,7 @@ __global__ __launch_bounds__(SPREAD_NT) void k_ibm_spread_tiles(MemArgs m, IbmAr
 {
     constexpr int S = Stencil<K>::S, C = S * S * S, NPW = 64 / C, NW = SPREAD_NT / 64, NS = S * S * S;
     extern __shared__ int4 tile_lds[];  // candidates (bases, forces, ids), then 3 x max_tile_cells sums
-    __shared__ int s_tile[NS], s_pre[NS + 1], s_total, s_nov, s_nk, s_tc[3][S], s_ntc[3];
+    __shared__ int s_tile[NS], s_pre[NS + 1], s_total, s_nov, s_nk[2], s_tc[3][S], s_ntc[3];
     const int T = xcd_remap(blockIdx.x, gridDim.x);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int4 tl = g.tile_lo[T];
@@ -451,8 +451,10 @@ __global__ __launch_bounds__(SPREAD_NT) void k_ibm_spread_tiles(MemArgs m, IbmAr
         }
     }
     const int chunk = keeps == 1 ? SPREAD_NT : SPREAD_NT / keeps;
-    for (int q0 = 0; q0 < tot + nov; q0 += chunk) {
-        if (tid == 0) s_nk = 0;
+    // kept nodes are counted in two counters in turn: a slow wavefront may still
+    // read its chunk's count when another has passed on to the next chunk
+    if (tid == 0) s_nk[0] = 0;
+    for (int q0 = 0, p = 0; q0 < tot + nov; q0 += chunk, p ^= 1) {
         __syncthreads();  // the previous chunk is spread
         const int q = q0 + tid;
         int nd = -1, rx = 0, ry = 0, rz = 0;
@@ -488,7 +490,7 @@ __global__ __launch_bounds__(SPREAD_NT) void k_ibm_spread_tiles(MemArgs m, IbmAr
             // one image each: slots by wavefront
             const unsigned long long kept = __ballot(keep);
             int e0 = 0;
-            if (lane == 0 && kept) e0 = atomicAdd(&s_nk, __popcll(kept));
+            if (lane == 0 && kept) e0 = atomicAdd(&s_nk[p], __popcll(kept));
             e0 = __shfl(e0, 0, 64);
             if (keep)
                 put(e0 + __popcll(kept & ((1ull << lane) - 1ull)), rx < dim[0] ? rx : rx - B.n[0],
@@ -498,10 +500,11 @@ __global__ __launch_bounds__(SPREAD_NT) void k_ibm_spread_tiles(MemArgs m, IbmAr
                 for (int ky = 0, y = ry; ky < img[1]; ky++, y -= B.n[1])
                     for (int kx = 0, x = rx; kx < img[0]; kx++, x -= B.n[0])
                         if (x > -S && x < dim[0] && y > -S && y < dim[1] && z > -S && z < dim[2])
-                            put(atomicAdd(&s_nk, 1), x, y, z);
+                            put(atomicAdd(&s_nk[p], 1), x, y, z);
         }
         __syncthreads();
-        const int nk = s_nk;
+        const int nk = s_nk[p];
+        if (tid == 0) s_nk[p ^ 1] = 0;  // (every wavefront has read it, before this chunk)
         int off[3];
         lane_offset(S, lane % C, off);
         const int loff = off[0] + dim[0] * (off[1] + dim[1] * off[2]);
