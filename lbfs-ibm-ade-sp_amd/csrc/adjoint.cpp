@@ -106,7 +106,11 @@ template <class T>
 int adj_alloc(lbfs_ctx *ctx, T **dst, size_t n)
 {
     void *p = nullptr;
-    HIPCHK(hipMalloc(&p, (n > 0 ? n : 1) * sizeof(T)));
+    const hipError_t e = hipMalloc(&p, (n > 0 ? n : 1) * sizeof(T));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // (the next launch's check would report it again)
+        return ctx->fail(LBFS_E_HIP, "adjoint buffers: %s", hipGetErrorString(e));
+    }
     ctx->adj->allocs.push_back(p);
     HIPCHK(hipMemsetAsync(p, 0, (n > 0 ? n : 1) * sizeof(T), ctx->stream));  // ordered before the kernels
     *dst = (T *)p;
@@ -207,17 +211,11 @@ int alloc_records(lbfs_ctx *ctx, std::vector<StepRec> &recs, int every)
     return LBFS_OK;
 }
 
-int adjoint_setup(lbfs_ctx *ctx, int n_steps, int every)
+// the buffers of a new shape, ctx->adj->n_steps steps in segments of every
+int adjoint_buffers(lbfs_ctx *ctx)
 {
-    if (ctx->adj && ctx->adj->n_steps == n_steps && ctx->adj->every == every) {
-        ctx->adj->recorded = false;  // same shape: the buffers are reused
-        return LBFS_OK;
-    }
-    adjoint_release(ctx);
-    ctx->adj = new AdjointState();
     AdjointState &A = *ctx->adj;
-    A.n_steps = n_steps;
-    A.every = every;
+    const int n_steps = A.n_steps, every = A.every;
     for (int t = 0; t < ctx->lay.n_tiles; t++)
         A.max_tile_cells = std::max(A.max_tile_cells, ctx->lay.tile_cell_start[t + 1] - ctx->lay.tile_cell_start[t]);
     const int n = ctx->lay.n_cells;
@@ -290,6 +288,22 @@ int adjoint_setup(lbfs_ctx *ctx, int n_steps, int every)
     // the buffers were cleared on the context's stream
     HIPCHK(hipStreamSynchronize(ctx->stream));
     return LBFS_OK;
+}
+
+int adjoint_setup(lbfs_ctx *ctx, int n_steps, int every)
+{
+    if (ctx->adj && ctx->adj->n_steps == n_steps && ctx->adj->every == every) {
+        ctx->adj->recorded = false;  // same shape: the buffers are reused
+        return LBFS_OK;
+    }
+    adjoint_release(ctx);
+    ctx->adj = new AdjointState();
+    ctx->adj->n_steps = n_steps;
+    ctx->adj->every = every;
+    // (a failed set-up leaves no state that a later call could take for whole)
+    const int rc = adjoint_buffers(ctx);
+    if (rc) adjoint_release(ctx);
+    return rc;
 }
 
 // One step of a segment replay, from the live state with its fluid state in

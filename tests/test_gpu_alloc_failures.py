@@ -1,0 +1,131 @@
+"""Calls during which an allocation fails, forced from the host: a child process
+loads a library that stands before the runtime's allocation entry points and
+turns chosen calls into ones that the runtime refuses (an impossible size)."""
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+SHIM = r"""
+#include <dlfcn.h>
+#include <stddef.h>
+static long left = -1, calls = 0;
+static int keep = 0;
+extern "C" void shim_malloc(long after, int stay) { left = after; keep = stay; }
+extern "C" long shim_calls() { return calls; }
+extern "C" int hipMalloc(void **p, size_t n)
+{
+    static int (*real)(void **, size_t) = (int (*)(void **, size_t))dlsym(RTLD_NEXT, "hipMalloc");
+    calls++;
+    if (left == 0) {
+        if (!keep) left = -1;
+        n = (size_t)1 << 60;
+    } else if (left > 0) {
+        left--;
+    }
+    return real(p, n);
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    d = tmp_path_factory.mktemp("shim")
+    src, lib = d / "shim.cpp", d / "libshim.so"
+    src.write_text(SHIM)
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", str(src), "-o", str(lib), "-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib",
+                    "-Wl,--no-as-needed", "-lamdhip64", "-ldl"], check=True)
+    return str(lib)
+
+
+def child(shim, name):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), shim, name], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+
+
+@pytest.mark.gpu
+def test_failed_adjoint_setup_is_not_taken_for_whole(shim):
+    child(shim, "adjoint_setup")
+
+
+# ---------------------------------------------------------------------------
+# in the child
+# ---------------------------------------------------------------------------
+class Failures:
+    def __init__(self, path):
+        self.lib = C.CDLL(path, mode=C.RTLD_GLOBAL)
+        self.lib.shim_calls.restype = C.c_long
+        self.lib.shim_malloc.argtypes = [C.c_long, C.c_int]
+
+    def calls(self):
+        return self.lib.shim_calls()
+
+    def after(self, n, keep=False):
+        """Fail the (n + 1)-th allocation from now on, and with keep all that follow."""
+        self.lib.shim_malloc(n, 1 if keep else 0)
+
+    def off(self):
+        self.lib.shim_malloc(-1, 0)
+
+
+def small_solver():
+    import cases
+    from lbfs_amd import abi
+    mesh = cases.channel_mesh(24, 16, 16, seed=8)
+    s = abi.Solver(mesh, abi.make_params(visc=1.0 / 6.0, dt=0.25, body_force=(2e-5, 0.0, 0.0)))
+    s.set_state(*cases.smooth_state(mesh, seed=8, amp=0.005))
+    x, t = abi.rbc(4, 8.0, center=(12.0, 8.0, 8.0))
+    s.add_membranes([abi.Membrane(x, t, **dict(abi.RBC_PARAMS, volume_ratio=0.95))])
+    return s
+
+
+def refused(call, *args):
+    from lbfs_amd import abi
+    try:
+        call(*args)
+    except abi.LbfsError:
+        return True
+    return False
+
+
+def adjoint_setup(fail):
+    """A gradient whose set-up failed fails again while memory is short, and
+    succeeds in full afterwards."""
+    rng = np.random.default_rng(3)
+
+    def gradient(s):
+        s.adjoint_forward(9, 4)
+        lam = rng0.standard_normal((s.n_mem_nodes, 3))
+        g = s.adjoint_backward(lam_nodes=lam, lam_state=rng0.standard_normal((s.n, 4)))
+        return [s.membrane_nodes()[0], g["body_force"], g["moduli"], g["state0"], g["nodes0"]]
+
+    s = small_solver()
+    assert fail.calls() > 0  # the allocations do pass through the library
+    c0 = fail.calls()
+    rng0 = np.random.default_rng(3)
+    want = gradient(s)
+    n = fail.calls() - c0
+    s.close()
+    for k in sorted(set([0, 1, n - 1] + list(rng.integers(0, n, 8)))):
+        print("set-up of %d allocations, failing at %d" % (n, k), flush=True)
+        s = small_solver()
+        fail.after(int(k), keep=True)
+        assert refused(s.adjoint_forward, 9, 4)
+        assert refused(s.adjoint_forward, 9, 4)
+        fail.off()
+        assert refused(s.adjoint_rewind)
+        rng0 = np.random.default_rng(3)
+        got = gradient(s)
+        for a, b in zip(want, got):
+            assert np.all(np.isfinite(a)) and np.array_equal(a, b)
+        s.close()
+
+
+if __name__ == "__main__":
+    sys.path[:0] = [HERE, os.path.dirname(HERE), os.path.join(os.path.dirname(HERE), "lbfs-ibm-ade-sp_amd")]
+    globals()[sys.argv[2]](Failures(sys.argv[1]))
