@@ -176,8 +176,10 @@ __device__ __forceinline__ void pair_step(FaceSums &f, const float po[4], const 
 // neighbour side, so each point is one contraction and one multiply-add per
 // variable where the selection of pair_step evaluates both sides for both
 // points.  g / w = drho + 3/2 (rho / gamma) (eu (3 eu + 2 s gamma) - u.u) is the
-// equilibrium deviation of eq_point; the lattice weight and the signs ride in
-// the factors of the sums: about 45 operations a diagonal pair where pair_step
+// equilibrium deviation of eq_point (u.u summed by itself: its squares taken from
+// the larger first term one by one are each rounded at that term's size, 8 % more
+// error in a face's flux); the lattice weight and the signs ride in the factors
+// of the sums: about 45 operations a diagonal pair where pair_step
 // takes 63.  128x64x64 channel, D3Q19, 8x8x8 tiles: face pass 34.8 -> 30.6 us,
 // fused pass 45.9 -> 42.9 us (both were vector-bound, now memory).  pair_step
 // stays for the faces whose points may come from either side.
@@ -197,12 +199,8 @@ __device__ __forceinline__ void pair_fast(FaceSums &f, const float po[4], const 
         qn[v] = fmaf(sdt, edot<ex, ey, ez>(gn[3 * v], gn[3 * v + 1], gn[3 * v + 2]), pn[v]);
     }
     const float euo = edot<ex, ey, ez>(qo[1], qo[2], qo[3]), eun = edot<ex, ey, ez>(qn[1], qn[2], qn[3]);
-    float Bo = euo * fmaf(3.0f, euo, sgam), Bn = eun * fmaf(3.0f, eun, -sgam);
-#pragma unroll
-    for (int t = 1; t < 4; t++) {
-        Bo = fmaf(-qo[t], qo[t], Bo);
-        Bn = fmaf(-qn[t], qn[t], Bn);
-    }
+    const float Bo = fmaf(euo, fmaf(3.0f, euo, sgam), -dot3(qo[1], qo[2], qo[3], qo[1], qo[2], qo[3]));
+    const float Bn = fmaf(eun, fmaf(3.0f, eun, -sgam), -dot3(qn[1], qn[2], qn[3], qn[1], qn[2], qn[3]));
     const float g_o = fmaf(fmaf(ig15, qo[0], rho15), Bo, qo[0]), g_n = fmaf(fmaf(ig15, qn[0], rho15), Bn, qn[0]);
     const float gs = g_o + g_n, gd = g_o - g_n;
     f.S0 = fmaf(w, gs, f.S0);

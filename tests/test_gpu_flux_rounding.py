@@ -1,0 +1,116 @@
+"""Rounding error of the face fluxes, against the same formula in FP64 from the
+same single-precision inputs (records, states and gradients), for every
+lattice: no larger than that of the general reconstruction evaluated in single
+precision, with the multiply-adds the kernels write out."""
+import numpy as np
+import pytest
+
+import cases
+from lbfs_amd import abi
+
+# one direction of each opposite pair, and the weight of 0, 1, 2, 3 nonzero components
+LATTICES = {
+    abi.D3Q15: ([(1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 1, 1), (1, 1, -1), (1, -1, 1), (-1, 1, 1)],
+                (2 / 9, 1 / 9, None, 1 / 72)),
+    abi.D3Q19: ([(1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 1, 0), (1, -1, 0), (1, 0, 1), (1, 0, -1), (0, 1, 1), (0, 1, -1)],
+                (1 / 3, 1 / 18, 1 / 36)),
+    abi.D2Q9: ([(1, 0, 0), (0, 1, 0), (1, 1, 0), (1, -1, 0)], (4 / 9, 1 / 9, 1 / 36)),
+}
+
+
+def fma(a, b, c):
+    """a b + c rounded once to the operands' type."""
+    r = np.float64(a) * np.float64(b) + np.float64(c)
+    return r.astype(np.result_type(a, b, c))
+
+
+def dot3(a, b):
+    return fma(a[0], b[0], fma(a[1], b[1], a[2] * b[2]))
+
+
+def along(e, v):
+    s = None
+    for c, x in zip(e, v):
+        if c:
+            s = (x if c > 0 else -x) if s is None else (s + x if c > 0 else s - x)
+    return s
+
+
+def face_flux(lattice, T, rec, dt, d1, d2, so, sn, go, gn, visc):
+    """Fluxes [4] of faces from records, states [4] and gradients [4][3] of both
+    sides, all in type T (gamma = 1, rho0 = 1)."""
+    dirs, weights = LATTICES[lattice]
+    rec, dt, d1, d2, so, sn, go, gn = (np.asarray(a).astype(T) for a in (rec, dt, d1, d2, so, sn, go, gn))
+    A = np.sqrt(dot3(rec, rec))
+    n = rec * (T(1) / A)
+    po = np.array([so[v] - dot3(d1, go[v]) for v in range(4)])
+    pn = np.array([sn[v] - dot3(d2, gn[v]) for v in range(4)])
+    p0 = T(0.5) * (po + pn)
+
+    def equilibrium(p, eu, w):
+        P = fma(eu, fma(T(4.5), eu, T(3)), T(-1.5) * dot3(p[1:], p[1:]))
+        return T(w) * fma(T(1) + p[0], P, p[0])
+
+    S0 = equilibrium(p0, np.zeros_like(dt), weights[0])
+    S1, M = [np.zeros_like(dt) for _ in range(3)], [np.zeros_like(dt) for _ in range(3)]
+    go, gn = go * dt, gn * dt
+    for e in dirs:
+        w = weights[sum(abs(c) for c in e)]
+        en = along(e, n)
+        q = [np.array([np.where(s * en < 0, pn[v] - s * along(e, gn[v]), po[v] - s * along(e, go[v])) for v in range(4)])
+             for s in (T(1), T(-1))]
+        g = [equilibrium(p, s * along(e, p[1:]), w) for p, s in zip(q, (T(1), T(-1)))]
+        gs, gd = g[0] + g[1], g[0] - g[1]
+        S0 = S0 + gs
+        for t in range(3):
+            if e[t]:
+                S1[t] = S1[t] + T(e[t]) * gd
+                M[t] = fma(T(e[t]) * en, gs, M[t])
+    tau = T(3 * visc) * (T(1) / dt)
+    mn = dot3(S1, n)
+    third, q = S0 * T(1 / 3), mn * (T(1) / (T(1) + S0))
+    out = [mn * A] + [A * fma(T(1) - tau, fma(S1[t], q, third * n[t]), tau * M[t]) for t in range(3)]
+    if lattice == abi.D2Q9:
+        out[3] = np.zeros_like(mn)
+    return np.array(out)
+
+
+def inputs(mesh, visc, state, grad):
+    """Records and both sides' states and gradients of the interior faces."""
+    g = mesh.geometry(visc=visc)
+    ni, f32 = mesh.n_internal, np.float32
+    o, nb = np.array(mesh.owner[:ni]), np.array(mesh.neighbour[:ni])
+    area, normal = g["area"][:ni], g["normal"].reshape(-1, 3)[:ni]
+    fc, cc = g["face_centroid"].reshape(-1, 3)[:ni], g["centroid"].reshape(-1, 3)
+    shift = np.array(mesh.face_shift).reshape(-1, 3)[:ni]
+    st = np.array([state[0] - 1.0, *state[1:]]).astype(f32)
+    gr = grad.reshape(-1, 4, 3).astype(f32).transpose(1, 2, 0)
+    return (f32(normal.T * area), f32(g["face_dt"][:ni]), f32((cc[o] - fc).T), f32((cc[nb] + shift - fc).T),
+            st[:, o], st[:, nb], gr[:, :, o], gr[:, :, nb])
+
+
+def case(lattice, amp):
+    n = (40, 36, 1) if lattice == abi.D2Q9 else (18, 14, 12)
+    mesh = abi.HexMesh(*n, periodic=(1, 1, 1), jitter=0.1, seed=3)
+    return mesh, 1.0 / 6.0, cases.smooth_state(mesh, seed=4, amp=amp, drho=0.1 * amp)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lattice", sorted(LATTICES))
+@pytest.mark.parametrize("amp", [0.004, 0.01, 0.05])
+def test_flux_error_no_larger_than_general_reconstruction(lattice, amp):
+    mesh, visc, state = case(lattice, amp)
+    s = abi.Solver(mesh, abi.make_params(lattice=lattice, visc=visc, dt=0.25))
+    s.set_state(*state)
+    x = inputs(mesh, visc, s.get_state(), s.gradients())
+    got = s.face_flux().reshape(-1, 4)[: mesh.n_internal].T.copy()
+    s.close()
+    g = mesh.geometry(visc=visc)
+    ni = mesh.n_internal
+    got[1:4] -= (g["normal"].reshape(-1, 3)[:ni] * g["area"][:ni, None]).T / 3.0 * \
+        np.array([1, 1, 0 if lattice == abi.D2Q9 else 1])[:, None]  # the rest pressure
+    exact = face_flux(lattice, np.float64, *x, visc)
+    single = face_flux(lattice, np.float32, *x, visc)
+    rows = slice(1, 3) if lattice == abi.D2Q9 else slice(1, 4)
+    rms = [np.sqrt(np.mean((f - exact)[rows] ** 2)) for f in (got, single)]
+    assert rms[0] <= rms[1], rms
