@@ -276,14 +276,13 @@ __device__ __forceinline__ void tile_update(const FluidArgs &a, const float4 *ld
             r0 = fmaf(sg, fl.x, r0); r1 = fmaf(sg, fl.y, r1); r2 = fmaf(sg, fl.z, r2); r3 = fmaf(sg, fl.w, r3);
         }
         const float iv = a.inv_vol[i];
-        r0 *= iv; r1 *= iv; r2 *= iv; r3 *= iv;
-        if (res_out) res_out[i] = make_float4(r0, r1, r2, r3);
+        if (res_out) res_out[i] = make_float4(r0 * iv, r1 * iv, r2 * iv, r3 * iv);
         if (!do_update) continue;
         float fx = a.body_force[0], fy = a.body_force[1], fz = a.body_force[2];
         if (a.cell_force) {
             fx += cfv[0]; fy += cfv[1]; fz += cfv[2];
         }
-        r1 += fx; r2 += fy; r3 += fz;
+        r0 *= iv; r1 = fmaf(r1, iv, fx); r2 = fmaf(r2, iv, fy); r3 = fmaf(r3, iv, fz);
         float dt = a.dt;
         if (a.ts_mode == LBFS_TS_LOCAL) {
             const float2 c = a.cfl_coef[i];

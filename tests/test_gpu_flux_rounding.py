@@ -124,16 +124,36 @@ def test_flux_error_no_larger_than_general_reconstruction(lattice, amp):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("lattice", sorted(LATTICES))
-def test_pressure_error_no_larger_than_with_exact_roots(lattice):
+@pytest.mark.parametrize("amp", [0.004, 0.01, 0.05])
+def test_flux_error_of_orthogonal_cells(lattice, amp):
+    """Faces with directions in their plane, of the general reconstruction
+    itself: below the formula's, whose sums over a pair round both weighted
+    points (in emulation 0.963 to 0.977 of it)."""
+    n = (40, 36, 1) if lattice == abi.D2Q9 else (18, 14, 12)
+    mesh = abi.HexMesh(*n, periodic=(1, 1, 1), jitter=0.0, seed=3)
+    visc = 1.0 / 6.0
+    s = abi.Solver(mesh, abi.make_params(lattice=lattice, visc=visc, dt=0.25))
+    s.set_state(*cases.smooth_state(mesh, seed=4, amp=amp, drho=0.1 * amp))
+    x = inputs(mesh, visc, s.get_state(), s.gradients())
+    rms = errors(s, mesh, lattice, visc, x)
+    s.close()
+    assert rms[0] <= 0.99 * rms[1], rms
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lattice", sorted(LATTICES))
+@pytest.mark.parametrize("visc,room", [(1.0 / 60.0, 1.03), (1.0, 1.02)])
+def test_pressure_error_no_larger_than_with_exact_roots(lattice, visc, room):
     """A gas at rest, whose flux is its pressure times the area vector: the
     error of normal and area together is that of a rounded square root and a
-    rounded division.  (3 %: the kernels' reciprocals and their order of sums.)"""
+    rounded division, and (visc 1, where the second moments carry most) the
+    moments take the rounded normal as it is: weights rounded into it give 1.03
+    to 1.07.  (The room is for the kernels' reciprocals and order of sums.)"""
     mesh, _, _ = case(lattice, 0.0)
-    visc = 1.0 / 60.0
     s = abi.Solver(mesh, abi.make_params(lattice=lattice, visc=visc, dt=0.25))
     n = mesh.n_cells
     s.set_state(np.full(n, 1.05), *(np.zeros(n) for _ in range(3)))
     x = inputs(mesh, visc, s.get_state(), s.gradients())
     rms = errors(s, mesh, lattice, visc, x)
     s.close()
-    assert rms[0] <= 1.03 * rms[1], rms
+    assert rms[0] <= room * rms[1], rms
