@@ -106,11 +106,8 @@ template <class T>
 int adj_alloc(lbfs_ctx *ctx, T **dst, size_t n)
 {
     void *p = nullptr;
-    const hipError_t e = hipMalloc(&p, (n > 0 ? n : 1) * sizeof(T));
-    if (e != hipSuccess) {
-        (void)hipGetLastError();  // (the next launch's check would report it again)
-        return ctx->fail(LBFS_E_HIP, "adjoint buffers: %s", hipGetErrorString(e));
-    }
+    const hipError_t e = ctx->device_alloc(&p, (n > 0 ? n : 1) * sizeof(T));
+    if (e != hipSuccess) return ctx->fail(LBFS_E_HIP, "adjoint buffers: %s", hipGetErrorString(e));
     ctx->adj->allocs.push_back(p);
     HIPCHK(hipMemsetAsync(p, 0, (n > 0 ? n : 1) * sizeof(T), ctx->stream));  // ordered before the kernels
     *dst = (T *)p;

@@ -53,6 +53,12 @@ struct lbfs_ctx {
     int *cell_inv = nullptr;        // [n] internal id of each caller cell
     lbfs::Staging staging;          // pinned buffers of the host transfers
     std::vector<void *> allocs;
+    float *tile_w = nullptr;        // weight rows of the fused pass (FluidArgs::tile_w)
+    // Device memory; where it is short, the fused pass's weight rows (126 B a cell
+    // with 8x8x8 tiles) are given back and the steps run the two passes, which need
+    // none of them and give the same bits.
+    hipError_t device_alloc(void **p, size_t bytes);
+    void release_tile_weights();
 
     // membranes and IBM coupling (lbfs_add_membranes)
     bool have_membranes = false;
@@ -90,7 +96,7 @@ struct lbfs_ctx {
     long long steps_enqueued = 0;   // steps of enqueue_steps so far
     int graph_steps(int k) const { return k == 1 ? 2 : (have_membranes ? 8 : 32); }
     int schedule_option = 0;        // LBFS_OPT_STEP_SCHEDULE
-    bool fused_ok = false;          // the tiles fit the fused fluid pass's LDS
+    bool fused_ok = false;          // the tiles fit the fused fluid pass's LDS, and its weight rows memory
     bool fused = false;             // LBFS_OPT_FUSED_FLUID: whole steps run the fused fluid pass
     bool use_graph = true;
     hipGraphExec_t graph_exec[2] = {nullptr, nullptr};

@@ -23,7 +23,7 @@ template <class T>
 static int cp_alloc(lbfs_ctx *ctx, T **dst, const T *src, size_t n)
 {
     void *p = nullptr;
-    HIPCHK(hipMalloc(&p, (n > 0 ? n : 1) * sizeof(T) + 16));
+    HIPCHK(ctx->device_alloc(&p, (n > 0 ? n : 1) * sizeof(T) + 16));
     ctx->coupling_allocs.push_back(p);
     if (src && n) HIPCHK(hipMemcpy(p, src, n * sizeof(T), hipMemcpyHostToDevice));
     else HIPCHK(hipMemsetAsync(p, 0, (n > 0 ? n : 1) * sizeof(T), ctx->stream));  // ordered before the kernels

@@ -35,11 +35,36 @@ int lbfs_ctx::fail(int code, const char *fmt, ...)
     return code;
 }
 
+hipError_t lbfs_ctx::device_alloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    for (int k = 0; k < 2 && e != hipSuccess; k++) {
+        (void)hipGetLastError();  // (the next launch's check would report it again)
+        if (e != hipErrorOutOfMemory || !tile_w) break;
+        release_tile_weights();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
+void lbfs_ctx::release_tile_weights()
+{
+    if (!tile_w) return;
+    // the steps under way read them
+    (void)hipStreamSynchronize(stream);
+    if (side) (void)hipStreamSynchronize(side);
+    drop_graph();
+    (void)hipFree(tile_w);
+    tile_w = nullptr;
+    args.tile_w = nullptr;
+    fused_ok = fused = false;
+}
+
 template <class T>
 static int dev_upload(lbfs_ctx *ctx, T **dst, const T *src, size_t n)
 {
     void *p = nullptr;
-    HIPCHK(hipMalloc(&p, n * sizeof(T) + 16));
+    HIPCHK(ctx->device_alloc(&p, n * sizeof(T) + 16));
     ctx->allocs.push_back(p);
     if (src) HIPCHK(hipMemcpy(p, src, n * sizeof(T), hipMemcpyHostToDevice));
     *dst = (T *)p;
@@ -132,9 +157,6 @@ static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params
         a.max_tile_cells = std::max(a.max_tile_cells, d.tile_cell_start[t + 1] - d.tile_cell_start[t]);
     a.max_grad_slots = d.max_grad_slots;
     a.max_slots = d.max_slots;
-    // (larger tiles run the two passes)
-    ctx->fused_ok = d.fused_fits;
-    ctx->fused = ctx->fused_ok;
     a.lattice = p.lattice;
     a.flags = p.flags;
     a.rho0 = (float)p.rho0;
@@ -214,12 +236,6 @@ static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params
     a.stencil = stencil; a.gw = gw; a.inv_vol = inv_vol;
     a.tile_cell_start = tcs;
     a.fA = fA; a.fB = fB; a.fC = fC;
-    if (ctx->fused_ok) {
-        float *tw;
-        if ((rc = dev_upload<float>(ctx, &tw, nullptr, 18 * (size_t)d.n_slots))) return rc;
-        HIPCHK(launch_tile_weights(a, tw, ctx->stream));
-        a.tile_w = tw;
-    }
     a.bc_type = bct; a.bc_val = bcv;
     a.visc_factor = nullptr;
     // cell force density: body force + closure term, IBM forces are added on top
@@ -273,6 +289,20 @@ static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params
     HIPCHK(hipMemsetAsync(ctx->st[0], 0, sizeof(float4) * n, ctx->stream));
     HIPCHK(hipMemsetAsync(ctx->st[1], 0, sizeof(float4) * n, ctx->stream));
     ctx->cur = 0;
+    // the fused pass's weight rows last, from what memory is left (larger tiles,
+    // and meshes whose rows do not fit, run the two passes)
+    if (d.fused_fits) {
+        void *tw = nullptr;
+        const hipError_t e = ctx->device_alloc(&tw, 18 * sizeof(float) * (size_t)d.n_slots);
+        if (e != hipSuccess && e != hipErrorOutOfMemory)
+            return ctx->fail(LBFS_E_HIP, "weight rows of the tiles: %s", hipGetErrorString(e));
+        if (e == hipSuccess) {
+            ctx->tile_w = (float *)tw;
+            a.tile_w = ctx->tile_w;
+            HIPCHK(launch_tile_weights(a, ctx->tile_w, ctx->stream));
+        }
+    }
+    ctx->fused_ok = ctx->fused = ctx->tile_w != nullptr;
     return LBFS_OK;
 }
 
@@ -339,6 +369,7 @@ extern "C" int lbfs_destroy(lbfs_ctx *ctx)
     ctx->release_extensions();
     for (void *p : ctx->allocs) hipFree(p);
     ctx->allocs.clear();
+    if (ctx->tile_w) (void)hipFree(ctx->tile_w);
     ctx->staging.release();
     if (ctx->side) (void)hipStreamSynchronize(ctx->side);
     if (ctx->side2) (void)hipStreamSynchronize(ctx->side2);
@@ -502,7 +533,9 @@ extern "C" int lbfs_set_option(lbfs_ctx *ctx, int option, int value)
     if (option == LBFS_OPT_FUSED_FLUID) {
         if (value < 0 || value > 1) return ctx->fail(LBFS_E_INVALID_ARG, "LBFS_OPT_FUSED_FLUID takes 0 or 1");
         if (value && !ctx->fused_ok)
-            return ctx->fail(LBFS_E_UNSUPPORTED, "the tiles are too large for the fused fluid pass");
+            return ctx->fail(LBFS_E_UNSUPPORTED, ctx->lay.fused_fits
+                                                     ? "the fused fluid pass's weight rows do not fit the device's memory"
+                                                     : "the tiles are too large for the fused fluid pass");
         ctx->fused = value != 0;
         ctx->drop_graph();
         return LBFS_OK;

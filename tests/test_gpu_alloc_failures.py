@@ -53,6 +53,11 @@ def test_failed_adjoint_setup_is_not_taken_for_whole(shim):
     child(shim, "adjoint_setup")
 
 
+@pytest.mark.gpu
+def test_without_memory_for_the_fused_pass(shim):
+    child(shim, "weight_rows")
+
+
 # ---------------------------------------------------------------------------
 # in the child
 # ---------------------------------------------------------------------------
@@ -123,6 +128,70 @@ def adjoint_setup(fail):
         got = gradient(s)
         for a, b in zip(want, got):
             assert np.all(np.isfinite(a)) and np.array_equal(a, b)
+        s.close()
+
+
+def weight_rows(fail):
+    """A solver whose fused pass's weight rows find no memory runs the two passes,
+    and gives the rows back where a later allocation needs them: the same bits."""
+    import cases
+    from lbfs_amd import abi
+    mesh = cases.channel_mesh(24, 16, 16, seed=8)
+    x, t = abi.rbc(4, 8.0, center=(12.0, 8.0, 8.0))
+
+    def create():
+        return abi.Solver(mesh, abi.make_params(visc=1.0 / 6.0, dt=0.25, body_force=(2e-5, 0.0, 0.0)))
+
+    def run(s, membranes_fail=None, gradient_fail=None):
+        rng = np.random.default_rng(3)
+        s.set_state(*cases.smooth_state(mesh, seed=8, amp=0.005))
+        s.step(5)
+        if membranes_fail is not None:
+            fail.after(membranes_fail)
+        c = fail.calls()
+        s.add_membranes([abi.Membrane(x, t, **dict(abi.RBC_PARAMS, volume_ratio=0.95))])
+        c_mem = fail.calls() - c
+        s.step(5)
+        if gradient_fail is not None:
+            fail.after(gradient_fail)
+        c = fail.calls()
+        s.adjoint_forward(9, 4)
+        c_adj = fail.calls() - c
+        g = s.adjoint_backward(lam_nodes=rng.standard_normal((s.n_mem_nodes, 3)),
+                               lam_state=rng.standard_normal((s.n, 4)))
+        out = list(s.get_state()) + list(s.membrane_nodes()) + [g[k] for k in sorted(g)]
+        return out, c_mem, c_adj
+
+    def equal(a, b):
+        return all(np.all(np.isfinite(p)) and np.array_equal(p, q) for p, q in zip(a, b))
+
+    c = fail.calls()
+    s = create()
+    n = fail.calls() - c
+    s.set_fused(True)
+    want, n_mem, n_adj = run(s)
+    s.close()
+    created = []
+    for k in range(n):
+        print("creation of %d allocations, failing at %d" % (n, k), flush=True)
+        fail.after(k)
+        try:
+            s = create()
+        except abi.LbfsError:
+            fail.off()
+            continue
+        fail.off()
+        created.append(k)
+        assert refused(s.set_fused, True)
+        assert equal(want, run(s)[0])
+        s.close()
+    assert created == [n - 1]
+    for kw in [dict(membranes_fail=k) for k in (0, n_mem // 2, n_mem - 1)] + \
+              [dict(gradient_fail=k) for k in (0, n_adj // 2, n_adj - 1)]:
+        print(kw, flush=True)
+        s = create()
+        assert equal(want, run(s, **kw)[0])
+        assert refused(s.set_fused, True)
         s.close()
 
 
