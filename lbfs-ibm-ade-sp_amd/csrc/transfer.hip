@@ -179,31 +179,93 @@ public:
         if (e_ != hipSuccess) return ctx->fail(LBFS_E_HIP, "%s: %s", #expr, hipGetErrorString(e_)); \
     } while (0)
 
-// the staging buffers of a transfer of `chunks` chunks of up to `bytes` (grown if
-// a larger transfer comes): a single chunk needs one, whose allocation is most
-// of a small mesh's first readback
-int staging(lbfs_ctx *ctx, size_t bytes, size_t chunks)
+// Readies the staging buffers of a transfer of `chunks` chunks of up to `bytes`
+// (grown if a larger transfer comes): a single chunk needs one, whose allocation
+// is most of a small mesh's first readback.  False where pinned memory cannot be
+// had; the transfer then goes through pageable memory.
+bool staging(lbfs_ctx *ctx, size_t bytes, size_t chunks)
 {
     Staging &s = ctx->staging;
     if (s.bytes < bytes) s.release();
     const size_t size = std::max(bytes, s.bytes);
     for (size_t k = 0; k < std::min<size_t>(2, chunks); k++) {
-        if (!s.ev[k]) HIPCHK(hipEventCreateWithFlags(&s.ev[k], hipEventDisableTiming));
-        if (!s.buf[k]) HIPCHK(hipHostMalloc((void **)&s.buf[k], size, hipHostMallocDefault));
+        hipError_t e = hipSuccess;
+        if (!s.ev[k]) e = hipEventCreateWithFlags(&s.ev[k], hipEventDisableTiming);
+        if (e == hipSuccess && !s.buf[k]) e = hipHostMalloc((void **)&s.buf[k], size, hipHostMallocDefault);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();  // (the next launch's check would report it again)
+            s.release();
+            return false;
+        }
     }
     s.bytes = size;
+    return true;
+}
+
+// the device's records in pageable memory
+int pageable(lbfs_ctx *ctx, const float4 *src, size_t n, std::vector<float4> &h)
+{
+    h.resize(n);
+    HIPCHK(hipMemcpyAsync(h.data(), src, sizeof(float4) * n, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return LBFS_OK;
+}
+
+int read_cells_pageable(lbfs_ctx *ctx, const float4 *src, double add0, const CellArrays &out)
+{
+    std::vector<float4> h;
+    const int rc = pageable(ctx, src, (size_t)ctx->lay.n_cells, h);
+    if (rc) return rc;
+    for (int i = 0; i < ctx->lay.n_cells; i++) {
+        const size_t c = (size_t)ctx->lay.perm[i];
+        const double v[4] = {add0 + (double)h[i].x, (double)h[i].y, (double)h[i].z, (double)h[i].w};
+        for (int t = 0; t < 4; t++) (out.aos ? out.aos[4 * c + t] : out.soa[t][c]) = v[t];
+    }
+    return LBFS_OK;
+}
+
+int write_cells_pageable(lbfs_ctx *ctx, const double *src, float4 *dst)
+{
+    const size_t n = (size_t)ctx->lay.n_cells;
+    std::vector<float4> h(n);
+    for (size_t i = 0; i < n; i++) {
+        const double *v = src + 4 * (size_t)ctx->lay.perm[i];
+        h[i] = make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
+    }
+    HIPCHK(hipMemcpyAsync(dst, h.data(), sizeof(float4) * n, hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return LBFS_OK;
+}
+
+int read_nodes_pageable(lbfs_ctx *ctx, double *const out[3])
+{
+    const MemArgs &m = ctx->mem;
+    const float4 *const src[3] = {m.X, m.U, m.F};
+    std::vector<float4> h, o;
+    for (int q = 0; q < 3; q++) {
+        if (!out[q]) continue;
+        int rc = pageable(ctx, src[q], (size_t)m.n_nodes, h);
+        if (!rc && q == 0) rc = pageable(ctx, m.node_origin, (size_t)m.n_nodes, o);
+        if (rc) return rc;
+        for (int n = 0; n < m.n_nodes; n++) {
+            const double v[3] = {(double)h[n].x, (double)h[n].y, (double)h[n].z};
+            const double c[3] = {q ? 0.0 : (double)o[n].x, q ? 0.0 : (double)o[n].y, q ? 0.0 : (double)o[n].z};
+            for (int t = 0; t < 3; t++) out[q][3 * (size_t)n + t] = q ? v[t] : c[t] + v[t];
+        }
+    }
     return LBFS_OK;
 }
 
 // n items of `item` bytes out: launch(i0, m, buf) enqueues the kernel that
-// fills buf, segments(i0, m, buf) lists where its parts go
+// fills buf, segments(i0, m, buf) lists where its parts go; pageable() does the
+// whole transfer without pinned memory
 int stream_out(lbfs_ctx *ctx, size_t n, size_t item, const std::function<hipError_t(int, int, double *)> &launch,
-               const std::function<std::vector<Piece>(int, int, const double *)> &segments)
+               const std::function<std::vector<Piece>(int, int, const double *)> &segments,
+               const std::function<int()> &pageable)
 {
     const size_t per = std::max<size_t>(1, CHUNK_BYTES / item);
     const size_t chunks = (n + per - 1) / per;
-    int rc = staging(ctx, std::min(n, per) * item, chunks);
-    if (rc) return rc;
+    if (!staging(ctx, std::min(n, per) * item, chunks)) return pageable();
     Staging &s = ctx->staging;
     CopyTeam team(n * item);
     auto start = [&](size_t k) -> hipError_t {
@@ -240,7 +302,8 @@ int read_cells(lbfs_ctx *ctx, const float4 *src, double add0, const CellArrays &
                 for (int t = 0; t < 4; t++) p.push_back({out.soa[t] + c0, buf + (size_t)t * m, 8 * (size_t)m});
             }
             return p;
-        });
+        },
+        [&] { return read_cells_pageable(ctx, src, add0, out); });
 }
 
 int read_nodes(lbfs_ctx *ctx, double *X, double *U, double *F)
@@ -269,14 +332,14 @@ int read_nodes(lbfs_ctx *ctx, double *X, double *U, double *F)
             for (int q = 0; q < rows; q++)
                 p.push_back({dst[q] + 3 * (size_t)n0, buf + (size_t)q * 3 * count, 24 * (size_t)count});
             return p;
-        });
+        },
+        [&] { return read_nodes_pageable(ctx, arr); });
 }
 
 int write_cells(lbfs_ctx *ctx, const double *src, float4 *dst)
 {
     const size_t n = (size_t)ctx->lay.n_cells, per = CHUNK_BYTES / 32, chunks = (n + per - 1) / per;
-    int rc = staging(ctx, std::min(n, per) * 32, chunks);
-    if (rc) return rc;
+    if (!staging(ctx, std::min(n, per) * 32, chunks)) return write_cells_pageable(ctx, src, dst);
     Staging &s = ctx->staging;
     CopyTeam team(n * 32);
     for (size_t k = 0; k < chunks; k++) {

@@ -15,7 +15,18 @@ SHIM = r"""
 #include <dlfcn.h>
 #include <stddef.h>
 static long left = -1, calls = 0;
-static int keep = 0;
+static int keep = 0, no_pinned = 0;
+extern "C" void shim_no_pinned(int on) { no_pinned = on; }
+extern "C" int hipHostMalloc(void **p, size_t n, unsigned flags)
+{
+    static int (*real)(void **, size_t, unsigned) = (int (*)(void **, size_t, unsigned))dlsym(RTLD_NEXT, "hipHostMalloc");
+    if (no_pinned) {
+        no_pinned++;
+        n = (size_t)1 << 60;
+    }
+    return real(p, n, flags);
+}
+extern "C" int shim_pinned_refused() { return no_pinned - 1; }
 extern "C" void shim_malloc(long after, int stay) { left = after; keep = stay; }
 extern "C" long shim_calls() { return calls; }
 extern "C" int hipMalloc(void **p, size_t n)
@@ -56,6 +67,11 @@ def test_failed_adjoint_setup_is_not_taken_for_whole(shim):
 @pytest.mark.gpu
 def test_without_memory_for_the_fused_pass(shim):
     child(shim, "weight_rows")
+
+
+@pytest.mark.gpu
+def test_transfers_without_pinned_memory(shim):
+    child(shim, "pinned")
 
 
 # ---------------------------------------------------------------------------
@@ -193,6 +209,47 @@ def weight_rows(fail):
         assert equal(want, run(s, **kw)[0])
         assert refused(s.set_fused, True)
         s.close()
+
+
+def pinned(fail):
+    """Readbacks and adjoint seeds without pinned memory: the same values, on a
+    small solver and on one whose arrays move in three staged chunks."""
+    import cases
+    from lbfs_amd import abi
+    rng = np.random.default_rng(5)
+    lam_nodes = lam_state = None
+    mesh = abi.HexMesh(96, 80, 72, periodic=(1, 0, 0), jitter=0.1, seed=2)
+    large_state, large_seed = cases.smooth_state(mesh, seed=1), rng.standard_normal((mesh.n_cells, 4))
+
+    def run_large():
+        s = abi.Solver(mesh, abi.make_params(visc=1.0 / 6.0, dt=0.25))
+        s.set_state(*large_state)
+        s.adjoint_forward(1, 1)
+        g = s.adjoint_backward(lam_state=large_seed)
+        out = [g["state0"], g["body_force"]] + list(s.get_state())
+        s.close()
+        return out
+
+    def run():
+        nonlocal lam_nodes, lam_state
+        s = small_solver()
+        s.step(3)
+        out = list(s.get_state()) + list(s.membrane_nodes())
+        s.adjoint_forward(5, 3)
+        if lam_nodes is None:
+            lam_nodes, lam_state = rng.standard_normal((s.n_mem_nodes, 3)), rng.standard_normal((s.n, 4))
+        g = s.adjoint_backward(lam_nodes=lam_nodes, lam_state=lam_state)
+        s.step(2)
+        out += [g[k] for k in sorted(g)] + list(s.get_state())
+        s.close()
+        return out
+
+    want = run() + run_large()
+    fail.lib.shim_no_pinned(1)
+    got = run() + run_large()
+    assert fail.lib.shim_pinned_refused() > 0
+    for a, b in zip(want, got):
+        assert np.all(np.isfinite(a)) and np.array_equal(a, b)
 
 
 if __name__ == "__main__":
