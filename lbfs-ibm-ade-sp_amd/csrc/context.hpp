@@ -137,9 +137,12 @@ struct lbfs_ctx {
         std::function<int()> run;
         double model_bytes;
     };
-    // fused: the fluid passes as the one fused launch "fluid" (the step's own
-    // launches); otherwise "gradients" and "flux_update" (the stage API)
-    std::vector<Stage> step_stages(bool with_visc = false, bool fused = false);
+    // fused: the fluid passes as the one fused launch "fluid"; otherwise
+    // "gradients" and "flux_update".  one_force_pass: the membrane forces as the
+    // one launch "mem_forces" where the step takes it; otherwise "mem_volume",
+    // "mem_edges" and "mem_nodes".  (The stage API splits both; whole steps and
+    // their timing take the step's own launches.)
+    std::vector<Stage> step_stages(bool with_visc = false, bool fused = false, bool one_force_pass = false);
     // the internal viscosity field is rebuilt at t = 1 (mod 10000) (Solver_gpu.cu:884-889)
     bool visc_due(long long t) const { return visc_factor && (t % 10000) == 1; }
     int run_stages(bool with_visc);

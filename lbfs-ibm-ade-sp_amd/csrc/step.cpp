@@ -16,7 +16,7 @@ using namespace lbfs;
         if (e_ != hipSuccess) return ctx->fail(LBFS_E_HIP, "%s: %s", #expr, hipGetErrorString(e_)); \
     } while (0)
 
-std::vector<lbfs_ctx::Stage> lbfs_ctx::step_stages(bool with_visc, bool fused_fluid)
+std::vector<lbfs_ctx::Stage> lbfs_ctx::step_stages(bool with_visc, bool fused_fluid, bool one_force_pass)
 {
     std::vector<Stage> s;
     lbfs_ctx *ctx = this;
@@ -38,23 +38,32 @@ std::vector<lbfs_ctx::Stage> lbfs_ctx::step_stages(bool with_visc, bool fused_fl
                      608.0 * nn + 32.0 * touched});
         // volume and area sums: triangle 16 + nodes 48 per triangle; edge
         // forces: nodes 96 + indices 24 + constants 24 + state 16 + forces
-        // written 64 per edge
-        s.push_back({"mem_volume", [ctx]() -> int {
-                         HIPCHK(launch_mem_volume(ctx->mem, ctx->stream));
-                         return LBFS_OK;
-                     },
-                     64.0 * nt});
-        s.push_back({"mem_edges", [ctx]() -> int {
-                         HIPCHK(launch_mem_edges(ctx->mem, ctx->stream));
-                         return LBFS_OK;
-                     },
-                     224.0 * ne});
-        // node forces: per edge its four force slots 64 and their incidence
-        // ids 16; per node the incidence range 4 and the force written 16 (in
-        // the spreading when it gathers them itself)
+        // written 64 per edge; node forces: per edge its four force slots 64
+        // and their incidence ids 16; per node the incidence range 4 and the
+        // force written 16 (in the spreading when it gathers them itself).  One
+        // launch: the same without the force slots
         const double node_force_bytes = 80.0 * ne + 20.0 * nn;
-        const bool gather_forces = spread_gathers_forces(ibm);
-        if (!gather_forces)
+        const bool one_pass = one_force_pass && mem.n_force_wg > 0;
+        const bool gather_forces = !one_pass && spread_gathers_forces(ibm);
+        if (one_pass) {
+            s.push_back({"mem_forces", [ctx]() -> int {
+                             HIPCHK(launch_mem_forces(ctx->mem, true, ctx->stream));
+                             return LBFS_OK;
+                         },
+                         64.0 * nt + 176.0 * ne + 20.0 * nn});
+        } else {
+            s.push_back({"mem_volume", [ctx]() -> int {
+                             HIPCHK(launch_mem_volume(ctx->mem, ctx->stream));
+                             return LBFS_OK;
+                         },
+                         64.0 * nt});
+            s.push_back({"mem_edges", [ctx]() -> int {
+                             HIPCHK(launch_mem_edges(ctx->mem, ctx->stream));
+                             return LBFS_OK;
+                         },
+                         224.0 * ne});
+        }
+        if (!one_pass && !gather_forces)
             s.push_back({"mem_nodes", [ctx]() -> int {
                              HIPCHK(launch_mem_nodes(ctx->mem, ctx->stream));
                              return LBFS_OK;
@@ -71,8 +80,8 @@ std::vector<lbfs_ctx::Stage> lbfs_ctx::step_stages(bool with_visc, bool fused_fl
         // touched cell the force density written 12 (tile gathering) or the
         // fixed-point sums read and written 48 (per-node and bin scattering)
         const double cell_bytes = ibm.binned == IBM_SPREAD_GATHER ? 12.0 : 48.0;
-        s.push_back({"ibm_spread", [ctx]() -> int {
-                         HIPCHK(launch_ibm_spread(ctx->mem, ctx->ibm, false, ctx->stream));
+        s.push_back({"ibm_spread", [ctx, one_pass]() -> int {
+                         HIPCHK(launch_ibm_spread(ctx->mem, ctx->ibm, one_pass, ctx->stream));
                          return LBFS_OK;
                      },
                      288.0 * nn + cell_bytes * touched + (gather_forces ? node_force_bytes : 0.0)});
@@ -154,7 +163,7 @@ int lbfs_ctx::run_stages(bool with_visc)
     if (!have_membranes || !side || with_visc) {
         // (the internal viscosity field feeds the face pass: in the steps
         // that rebuild it, everything runs in order on one stream)
-        for (auto &st : step_stages(with_visc, fz)) {
+        for (auto &st : step_stages(with_visc, fz, true)) {
             int rc = st.run();
             if (rc) return rc;
         }
@@ -277,13 +286,13 @@ extern "C" int lbfs_time_steps(lbfs_ctx *ctx, int nsteps, double *ms_total)
 extern "C" int lbfs_time_kernels(lbfs_ctx *ctx, int nsteps, int max_count, const char **names, double *ms, int *count)
 {
     if (!ctx || nsteps <= 0 || !ms || !count || max_count <= 0) return LBFS_E_INVALID_ARG;
-    // whole steps, one stage at a time with an event between stages (the
-    // stage list of a step that does not rebuild the internal viscosity
-    // field; such steps are refused so the schedule stays that of lbfs_step)
+    // whole steps, one launch of lbfs_step at a time with an event between
+    // launches (the list of a step that does not rebuild the internal viscosity
+    // field; such steps are refused)
     for (int s = 0; s < nsteps; s++)
         if (ctx->visc_due(ctx->t_step + s))
             return ctx->fail(LBFS_E_STATE, "a timed step would rebuild the internal viscosity field");
-    std::vector<lbfs_ctx::Stage> stages = ctx->step_stages(false, ctx->fused);
+    std::vector<lbfs_ctx::Stage> stages = ctx->step_stages(false, ctx->fused, true);
     const int ns = (int)stages.size();
     EventSet E;
     HIPCHK(E.create((size_t)nsteps * (ns + 1)));
@@ -345,7 +354,7 @@ extern "C" int lbfs_time_stage(lbfs_ctx *ctx, const char *name, int n, double *m
 extern "C" int lbfs_model_bytes(lbfs_ctx *ctx, int max_count, double *bytes, int *count)
 {
     if (!ctx || !bytes || !count || max_count <= 0) return LBFS_E_INVALID_ARG;
-    std::vector<lbfs_ctx::Stage> stages = ctx->step_stages(false, ctx->fused);
+    std::vector<lbfs_ctx::Stage> stages = ctx->step_stages(false, ctx->fused, true);
     *count = (int)stages.size() < max_count ? (int)stages.size() : max_count;
     for (int k = 0; k < *count; k++) bytes[k] = stages[k].model_bytes;
     return LBFS_OK;

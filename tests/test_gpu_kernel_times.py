@@ -1,0 +1,35 @@
+"""The timed kernels are those a step launches, and timed steps are whole steps."""
+import numpy as np
+import pytest
+
+import cases
+from lbfs_amd import abi
+
+pytestmark = pytest.mark.gpu
+
+
+# 162 nodes: membrane forces in one launch; 1442 nodes (2880 triangles): in separate passes, the
+# bin scattering (mode 2) gathering the node forces itself
+@pytest.mark.parametrize("freq,mode,forces", [
+    (4, 0, ["mem_forces"]), (4, 1, ["mem_forces"]), (4, 2, ["mem_forces"]),
+    (12, 1, ["mem_volume", "mem_edges", "mem_nodes"]), (12, 2, ["mem_volume", "mem_edges"]),
+])
+def test_timed_kernels_are_the_steps(freq, mode, forces):
+    mesh = cases.channel_mesh(24, 16, 16, seed=14)
+    x, t = abi.rbc(freq, 8.0, center=(12.0, 8.0, 8.0))
+    outs = []
+    for timed in (True, False):
+        s = abi.Solver(mesh, abi.make_params(visc=1.0 / 6.0, dt=0.25, body_force=(2e-5, 0.0, 0.0)))
+        s.set_state(*cases.smooth_state(mesh, seed=14, amp=0.005))
+        s.set_ibm_binned(mode)
+        s.add_membranes([abi.Membrane(x, t, **dict(abi.RBC_PARAMS, volume_ratio=0.95))])
+        if timed:
+            names = list(s.time_kernels(6))
+            assert names == ["ibm_interp"] + forces + ["ibm_spread", "fluid", "ibm_apply"]
+            assert len(s.model_bytes()) == len(names)
+        else:
+            s.step(6)
+        outs.append(list(s.get_state()) + list(s.membrane_nodes()) + [s.membrane_globals()])
+        s.close()
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
