@@ -81,16 +81,25 @@ extern "C" const char *lbfs_last_error(const lbfs_ctx *ctx)
 
 // The tile and workgroup size a caller leaves open.  A tile costs its halo's
 // gradients and its border faces again (8x8x8: 1.75 gradients and 3.4 faces a
-// cell, 8x4x4: 2.25 and 3.6, 4x4x4: 2.5 and 3.75), a small mesh the time of one
-// workgroup, so 8x8x8 tiles of 512 threads (two workgroups a compute unit) are
-// taken from 1000 tiles on, about two rounds of the chip: measured per plain
-// D3Q19 step 128x64x64 (1024 tiles) 38.3 us against 43.1 with 8x4x4, 192x96x96
-// 147 against 165, but 96x64x48 (576) 29.5 against 28.9 and 45x22x22 (54) 12.5
-// against 8.7.  Below 200 tiles of 8x4x4 the 4x4x4 ones are as fast or faster:
-// 24x16x16 (48) 7.4 against 9.5 us, 45x22x22 (216) 8.6 against 8.7, 70x33x29
-// (648) 14.1 against 11.7.  One layer of cells keeps 8x8 tiles of 256 threads
-// (64x64: 5.3 us, 16x16 9.5), and meshes without a logical structure runs of
-// 256 cells.
+// cell, 8x4x4: 2.25 and 3.6, 4x4x4: 2.5 and 3.75) and a membrane's tile spreading
+// looks through the nodes of 2.6 (8x4x4: 4.2) times its cells, while a small mesh
+// costs the time of one workgroup.  us a D3Q19 step with 8x8x8 tiles of 512
+// threads (two workgroups a compute unit) and with 8x4x4: plain, beside a
+// suspension of 0.2 nodes a cell, and of 0.025:
+//   64x48x48 (288 tiles of 8x8x8) 20.1 and 18.4, 103 and 104, 50 and 54
+//   72x56x48 (378)                21.0 and 22.5, 103 and 105, 52 and 58
+//   80x64x48 (480)                22.4 and 26.5, 117 and 121, 52 and 60
+//   96x64x48 (576)                29.6 and 29.5, 188 and 174, 59 and 74
+//   96x64x64 (768)                31.8 and 34.8, 203 and 223, 72 and 92
+//   120x64x64 (960)               37.6 and 40.5, 231 and 259, 82 and 107
+//   128x64x64 (1024)              38.3 and 43.1
+// Tiles only partly filled (the 8x8x8 ones of 73x57x49 to 71 %) make that 28.6
+// and 24.0, 105 and 109, 53 and 63; of 97x65x49 (74 %) 33.5 and 31.8, 181 and
+// 191, 66 and 82; of 68x60x52 (82 %) 21.3 and 23.5, 144 and 127, 54 and 59.
+// Below 200 tiles of 8x4x4 the 4x4x4 ones are as fast or faster: 24x16x16 (48)
+// 7.4 against 9.5 us, 45x22x22 (216) 8.6 against 8.7, 70x33x29 (648) 14.1 against
+// 11.7.  One layer of cells keeps 8x8 tiles of 256 threads (64x64: 5.3 us, 16x16
+// 9.5), and meshes without a logical structure runs of 256 cells.
 static void default_tile(const std::vector<HostBlock> &blocks, int tile[3], int &threads)
 {
     if (blocks.empty()) return;
@@ -102,7 +111,10 @@ static void default_tile(const std::vector<HostBlock> &blocks, int tile[3], int 
     };
     for (const HostBlock &b : blocks)
         if (b.n[0] == 1 || b.n[1] == 1 || b.n[2] == 1) return;
-    const bool large = tiles(8, 8, 8) >= 1000;
+    long long cells = 0;
+    for (const HostBlock &b : blocks) cells += (long long)b.n[0] * b.n[1] * b.n[2];
+    const long long cubes = tiles(8, 8, 8);
+    const bool large = cells >= 300000 || (cubes >= 350 && cells >= 400 * cubes);
     tile[0] = large || tiles(8, 4, 4) >= 200 ? 8 : 4;
     tile[1] = tile[2] = large ? 8 : 4;
     threads = large ? 512 : 256;
