@@ -24,7 +24,8 @@ void adjoint_release(lbfs_ctx *ctx);
 // overlap gains there.  One stream against two, a cell of 642 nodes: 9600 cells
 // 38.6 and 47.4 us a step, 41k 38.9 and 44.7, 77k 40.1 and 43.7, 147k 47.5 and
 // 46.4, 251k 55.5 and 50.2; of 2562 nodes 73 and 83, 58 and 65, 53 and 58, 59 and
-// 60, 71 and 66.
+// 60, 71 and 66; suspensions of 0.2 nodes a cell 32k 78.6 and 85.5, 58k 99.6 and
+// 101.7, 123k 107.3 and 108.2, of 0.025 34.7 and 40.8, 39.3 and 42.8, 51.6 and 54.3.
 constexpr int ONE_STREAM_CELLS = 128 * 1024;
 
 struct lbfs_ctx {

@@ -10,9 +10,12 @@ returns the fastest candidate.
 """
 from . import abi
 
-# candidate (tile x, tile y, tile z, workgroup threads)
+# candidate (tile x, tile y, tile z, workgroup threads); the solver's own choices by
+# mesh size (8x8x8 with 512 threads, 8x8x4, 8x4x4, 4x4x4) are among them
 CANDIDATES = (
     (8, 8, 4, 256),
+    (8, 4, 4, 256),
+    (4, 4, 4, 256),
     (8, 4, 8, 256),
     (8, 8, 8, 256),
     (8, 8, 8, 512),
