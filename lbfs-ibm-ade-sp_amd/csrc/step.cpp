@@ -93,37 +93,35 @@ std::vector<lbfs_ctx::Stage> lbfs_ctx::step_stages(bool with_visc, bool fused_fl
                          return LBFS_OK;
                      },
                      24.0 * n});
-    // pass G: state 16 + stencil 24 + RHS 72 + LS matrix 36 + gradients written 48 (B per cell)
+    // gradient pass: state 16 + stencil 24 + weights 72 + gradients written 48 (B per cell)
     if (!fused)
         s.push_back({"gradients", [ctx]() -> int {
                          HIPCHK(launch_gradients(ctx->args, ctx->st[ctx->cur], ctx->grad, ctx->stream));
                          return LBFS_OK;
                      },
-                     196.0 * n});
+                     160.0 * n});
     if (have_membranes) {
         // The face pass updates the cell with the static force (it does not
         // need the spread force, so it runs beside the coupling chain); the
         // apply pass then adds the spread force density in the tiles the
-        // spreading wrote into.  Face pass as below; apply: force density 12
+        // spreading wrote into.  Fluid passes as below; apply: force density 12
         // + static force 12 + state read and written 32 + force written 12
         // per touched cell (about 8 per node)
         const double touched = std::min(n, 8.0 * (double)mem.n_nodes);
         if (fused)
-            // the fused pass: both passes' bytes less the gradients written
-            // and read back (they stay in LDS) and the second read of the state
             s.push_back({"fluid", [ctx]() -> int {
                              HIPCHK(launch_fluid_fused(ctx->args, ctx->st[ctx->cur], ctx->st[ctx->cur ^ 1],
                                                        ctx->res_out(), 1, ctx->stream));
                              return LBFS_OK;
                          },
-                         192.0 * n + 40.0 * nf});
+                         120.0 * n + 40.0 * nf});
         else
             s.push_back({"flux_update", [ctx]() -> int {
                              HIPCHK(launch_flux_update(ctx->args, ctx->st[ctx->cur], ctx->grad, ctx->st[ctx->cur ^ 1],
                                                        ctx->res_out(), 1, ctx->stream));
                              return LBFS_OK;
                          },
-                         108.0 * n + 40.0 * nf});
+                         96.0 * n + 40.0 * nf});
         s.push_back({"ibm_apply", [ctx]() -> int {
                          HIPCHK(launch_ibm_apply(ctx->ibm, ctx->apply_args(ctx->st[ctx->cur ^ 1], ctx->cell_force, 0),
                                                  ctx->stream));
@@ -133,10 +131,11 @@ std::vector<lbfs_ctx::Stage> lbfs_ctx::step_stages(bool with_visc, bool fused_fl
                      68.0 * touched});
         return s;
     }
-    // pass F: state 16 + gradients 48 + volume/centroid 16 + force 12 + state written 16 per cell,
-    // plus owner/nb 8, normal 12, face centroid 12, area 4, dt 4 per face; the
-    // fused pass moves G + F less the gradients written and read back (they
-    // stay in LDS) and the second read of the state: 192 per cell
+    // face pass: state 16 + gradients 48 + inverse volume 4 + force 12 + state
+    // written 16 per cell, and the record of each face once (area vector and step
+    // 16, the two centroid offsets 24); the fused pass reads the weights 72 in
+    // place of the gradients.  (What tiles read again, halo cells and border
+    // faces, and the slot patterns shared through the caches are not counted.)
     if (fused)
         s.push_back({"fluid", [ctx]() -> int {
                          HIPCHK(launch_fluid_fused(ctx->args, ctx->st[ctx->cur], ctx->st[ctx->cur ^ 1], ctx->res_out(),
@@ -144,7 +143,7 @@ std::vector<lbfs_ctx::Stage> lbfs_ctx::step_stages(bool with_visc, bool fused_fl
                          ctx->cur ^= 1;
                          return LBFS_OK;
                      },
-                     192.0 * n + 40.0 * nf});
+                     120.0 * n + 40.0 * nf});
     else
         s.push_back({"flux_update", [ctx]() -> int {
                          HIPCHK(launch_flux_update(ctx->args, ctx->st[ctx->cur], ctx->grad, ctx->st[ctx->cur ^ 1],
@@ -152,7 +151,7 @@ std::vector<lbfs_ctx::Stage> lbfs_ctx::step_stages(bool with_visc, bool fused_fl
                          ctx->cur ^= 1;
                          return LBFS_OK;
                      },
-                     108.0 * n + 40.0 * nf});
+                     96.0 * n + 40.0 * nf});
     return s;
 }
 

@@ -33,3 +33,15 @@ def test_timed_kernels_are_the_steps(freq, mode, forces):
         s.close()
     for a, b in zip(*outs):
         assert np.array_equal(a, b)
+
+
+def test_model_bytes_of_the_fluid_passes():
+    """What each pass must move once: per cell the state in and out, inverse
+    volume, force and weights (72) or gradients (48), per face its record (40)."""
+    mesh = cases.channel_mesh(24, 16, 16, seed=14)
+    s = abi.Solver(mesh, abi.make_params(visc=1.0 / 6.0, dt=0.25))
+    n, faces = mesh.n_cells, mesh.n_faces
+    assert list(s.model_bytes()) == [(16 + 72 + 4 + 12 + 16) * n + 40 * faces]
+    s.set_fused(False)
+    assert list(s.model_bytes()) == [(16 + 24 + 72 + 48) * n, (16 + 48 + 4 + 12 + 16) * n + 40 * faces]
+    s.close()
