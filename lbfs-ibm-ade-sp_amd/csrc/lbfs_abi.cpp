@@ -151,8 +151,10 @@ static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params
         default_tile(ctx->blocks, tile, threads);
     }
     if (p.block_threads) threads = p.block_threads;
+    // (the reconstruction of clear faces takes 2 gamma, the general one 1 / gamma)
+    const bool general = !std::isfinite((float)(2.0 * p.gamma));
     rc = build_layout(m, ctx->geo, lhs, rhs, p.rho0, p.body_force, p.lattice, (p.flags & LBFS_FLAG_UPWIND_BAND) != 0,
-                      tile, ctx->blocks, ctx->lay, err);
+                      general, tile, ctx->blocks, ctx->lay, err);
     if (rc) return ctx->fail(rc, "layout: %s", err.c_str());
     const DeviceLayout &d = ctx->lay;
     const int n = d.n_cells, nbc = d.n_bc;

@@ -435,7 +435,7 @@ static double min_direction_component(int lattice, const double n[3])
 
 int build_layout(const lbfs_mesh_desc &m, const Geometry &g, const std::vector<double> &lhs,
                  const std::vector<double> &rhs, double rho0, const double body_force[3], int lattice, bool band,
-                 const int tile[3], const std::vector<HostBlock> &blocks, DeviceLayout &d, std::string &err)
+                 bool general, const int tile[3], const std::vector<HostBlock> &blocks, DeviceLayout &d, std::string &err)
 {
     const int nc = g.n_cells;
     const int dims = lattice == LBFS_D2Q9 ? 2 : 3;
@@ -497,12 +497,14 @@ int build_layout(const lbfs_mesh_desc &m, const Geometry &g, const std::vector<d
     const int nt = d.n_tiles;
     // 0: every lattice direction clearly on one side of the face; 1: one lies
     // within rounding of the face's plane or of the tie band around it (normals
-    // are held in float: e.n is off by at most 3 ulps of 1); 2: boundary face
+    // are held in float: e.n is off by at most 3 ulps of 1), or the caller wants
+    // the general reconstruction throughout; 2: boundary face
     std::vector<unsigned char> fclass(g.n_faces);
     parallel_for(g.n_faces, [&](int f0, int f1) {
         for (int f = f0; f < f1; f++) {
             const double tol = 1e-6 + (band ? 0.001 * g.fdt[f] * (1.0 + 1e-6) : 0.0);
-            fclass[f] = f >= g.n_int ? 2 : (min_direction_component(lattice, &g.normal[3 * (size_t)f]) > tol ? 0 : 1);
+            const bool clear = !general && min_direction_component(lattice, &g.normal[3 * (size_t)f]) > tol;
+            fclass[f] = f >= g.n_int ? 2 : (clear ? 0 : 1);
         }
     }, 8192);
     // What a tile's lists hold, in buffers of the worker that made them: its

@@ -111,6 +111,6 @@ struct DeviceLayout {
 };
 int build_layout(const lbfs_mesh_desc &m, const Geometry &g, const std::vector<double> &lhs,
                  const std::vector<double> &rhs, double rho0, const double body_force[3], int lattice, bool band,
-                 const int tile[3], const std::vector<HostBlock> &blocks, DeviceLayout &d, std::string &err);
+                 bool general, const int tile[3], const std::vector<HostBlock> &blocks, DeviceLayout &d, std::string &err);
 
 }  // namespace lbfs
