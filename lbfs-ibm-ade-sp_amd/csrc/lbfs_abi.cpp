@@ -120,6 +120,17 @@ static void default_tile(const std::vector<HostBlock> &blocks, int tile[3], int 
     threads = large ? 512 : 256;
 }
 
+// Tiles that leave most of a workgroup idle, or whose halo holds more than three
+// times their cells, run the two passes where the mesh has many of them: us a step
+// fused and in two passes, 128x64x64 in tiles of 4x2x2 150 and 116, 3x3x3 105 and
+// 84, 64x1x1 96 and 63, but 8x8x1 59 and 62, 16x2x2 57 and 59; 64x48x48 2x2x2 77
+// and 61, 4x4x2 (4608 tiles) both 27; 24x16x16 2x2x1 (1536) 13.0 and 10.7, 2x2x2
+// (768) 8.1 and 9.8, 64x1x1 (256) 7.2 and 8.9.
+static bool small_tiles(const DeviceLayout &d)
+{
+    return d.n_tiles >= 1500 && (d.n_cells < 64ll * d.n_tiles || d.n_slots > 4ll * d.n_cells);
+}
+
 static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params &p)
 {
     std::string err;
@@ -316,7 +327,8 @@ static int fluid_setup(lbfs_ctx *ctx, const lbfs_mesh_desc &m, const lbfs_params
             HIPCHK(launch_tile_weights(a, ctx->tile_w, ctx->stream));
         }
     }
-    ctx->fused_ok = ctx->fused = ctx->tile_w != nullptr;
+    ctx->fused_ok = ctx->tile_w != nullptr;
+    ctx->fused = ctx->fused_ok && !small_tiles(d);
     return LBFS_OK;
 }
 

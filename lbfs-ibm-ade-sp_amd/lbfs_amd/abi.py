@@ -688,7 +688,8 @@ class Solver:
 
     def set_fused(self, on):
         """Whole steps with the fused fluid pass (1, the default where the
-        tiles fit) or the two passes (0); the same bits either way."""
+        tiles fit and are not many small ones) or the two passes (0); the same
+        bits either way."""
         check(load().lbfs_set_option(self.ctx, OPT_FUSED_FLUID, 1 if on else 0), self.ctx)
 
     def set_ibm_binned(self, mode):

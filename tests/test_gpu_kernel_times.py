@@ -45,3 +45,22 @@ def test_model_bytes_of_the_fluid_passes():
     s.set_fused(False)
     assert list(s.model_bytes()) == [(16 + 24 + 72 + 48) * n, (16 + 48 + 4 + 12 + 16) * n + 40 * faces]
     s.close()
+
+
+@pytest.mark.parametrize("tile,fused", [((0, 0, 0), True), ((2, 2, 2), False), ((4, 4, 4), True), ((32, 1, 1), True)])
+def test_default_fluid_pass(tile, fused):
+    """Many small tiles (2304 of 2x2x2) run the two passes, others the fused one;
+    either can be asked for."""
+    mesh = cases.channel_mesh(32, 24, 24, seed=14)
+    st = cases.smooth_state(mesh, seed=14, amp=0.005)
+    s = abi.Solver(mesh, abi.make_params(visc=1.0 / 6.0, dt=0.25, tile=tile))
+    names = (["gradients", "flux_update"], ["fluid"])
+    assert list(s.time_kernels(1)) == names[fused]
+    outs = []
+    for on in (False, True):
+        s.set_fused(on)
+        s.set_state(*st)
+        assert list(s.time_kernels(2)) == names[on]
+        outs.append(np.concatenate(s.get_state()))
+    s.close()
+    assert np.array_equal(*outs)
