@@ -508,10 +508,6 @@ __device__ __forceinline__ void face_vjp(const FluidArgs &a, const FaceLoads &in
     out[3] = make_float4(lgo_[8], lgo_[9], lgo_[10], lgo_[11]);
 }
 
-constexpr int ADJ_THREADS = 256;
-constexpr int ADJ_CHUNK = 256;       // faces per LDS chunk (8 float4 each: 32 KiB), held as 8 planes
-                                     // of ADJ_CHUNK float4 so that a wavefront's stores are contiguous
-
 __device__ __forceinline__ void add4(float *acc, float4 v)
 {
     acc[0] += v.x; acc[1] += v.y; acc[2] += v.z; acc[3] += v.w;
@@ -524,31 +520,34 @@ __device__ __forceinline__ void add4(float *acc, float4 v)
 // threads 111 us, with the moments of face_vjp_clear (37.4 -> 29.6 M vector
 // instructions) 112; 256 threads 85.  Three workgroups in 168 registers take
 // 107 (spills), or 96 with one side of a face after the other; the next
-// chunk's loads issued ahead gain nothing at two.
-// ADJ_CELLS: cells per thread (tiles of up to 256, 512 or 1024 cells)
-template <class L, int ADJ_CELLS>
-__global__ __launch_bounds__(ADJ_THREADS) void k_adj_flux(FluidArgs a, AdjFluidArgs j, const float4 *__restrict__ st,
-                                                          const float4 *__restrict__ grad)
+// chunk's loads issued ahead gain nothing at two.  Tiles of more than 512 cells
+// keep 512 threads of two cells: four cells' sums a thread spill (20 steps of
+// 64x48x48 on 16x8x8 tiles reversed in 2.16 ms, 2.43 with 256 threads).
+// NT: threads, and the faces per LDS chunk (8 float4 each), held as 8 planes of NT
+// float4 so that a wavefront's stores are contiguous; ADJ_CELLS: cells per thread
+template <class L, int NT, int ADJ_CELLS>
+__global__ __launch_bounds__(NT) void k_adj_flux(FluidArgs a, AdjFluidArgs j, const float4 *__restrict__ st,
+                                                 const float4 *__restrict__ grad)
 {
     extern __shared__ float4 lds_adj[];
     const TileRec T = a.tiles[xcd_remap(blockIdx.x, gridDim.x)];
     const int c0 = T.c0, c1 = T.c0 + T.nc;
-    int *ids = reinterpret_cast<int *>(lds_adj + 8 * ADJ_CHUNK);  // cell id of each slot
-    for (int q = threadIdx.x; q < T.nc + T.nh; q += ADJ_THREADS) ids[q] = slot_cell(a, T, q);
+    int *ids = reinterpret_cast<int *>(lds_adj + 8 * NT);  // cell id of each slot
+    for (int q = threadIdx.x; q < T.nc + T.nh; q += NT) ids[q] = slot_cell(a, T, q);
     float acc[ADJ_CELLS][16];
     uint32_t slot[ADJ_CELLS][3];  // two slots each; 0x7fff: none
 #pragma unroll
     for (int u = 0; u < ADJ_CELLS; u++) {
 #pragma unroll
         for (int k = 0; k < 16; k++) acc[u][k] = 0.0f;
-        const int i = (int)threadIdx.x + u * ADJ_THREADS;
+        const int i = (int)threadIdx.x + u * NT;
         const uint32_t *sl = reinterpret_cast<const uint32_t *>(a.cell_slots) + 3 * (size_t)(T.pc + i);
 #pragma unroll
         for (int k = 0; k < 3; k++) slot[u][k] = i < T.nc ? sl[k] : 0x7fff7fffu;
     }
     const int last = T.nc + T.nh - 1;
     __syncthreads();
-    for (int cs = 0; cs < T.nf; cs += ADJ_CHUNK) {
+    for (int cs = 0; cs < T.nf; cs += NT) {
         const int q = cs + (int)threadIdx.x;
         if (q < T.nf) {
             // (a boundary face's neighbour slot is 0xffff: some cell of the tile's, unused)
@@ -561,10 +560,10 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_flux(FluidArgs a, AdjFluidA
             else if (q < T.nif) face_vjp<L, false>(a, in, fr, oc, 0, o);
             else face_vjp<L, true>(a, in, fr, oc, a.n_cells + a.tile_bc[T.b0 + q - T.nif], o);
 #pragma unroll
-            for (int k = 0; k < 8; k++) lds_adj[k * ADJ_CHUNK + threadIdx.x] = o[k];
+            for (int k = 0; k < 8; k++) lds_adj[k * NT + threadIdx.x] = o[k];
         }
         __syncthreads();
-        const uint32_t base = (uint32_t)cs, n = (uint32_t)min(ADJ_CHUNK, T.nf - cs);
+        const uint32_t base = (uint32_t)cs, n = (uint32_t)min(NT, T.nf - cs);
 #pragma unroll
         for (int u = 0; u < ADJ_CELLS; u++)
 #pragma unroll
@@ -573,15 +572,15 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_flux(FluidArgs a, AdjFluidA
                 const uint32_t r = (s & 0x7fffu) - base;
                 if (r >= n) continue;
                 const int side = (s & 0x8000u) ? 0 : 4;  // bit 15 set: the cell owns the face
-                const float4 *src = lds_adj + side * ADJ_CHUNK + r;
+                const float4 *src = lds_adj + side * NT + r;
 #pragma unroll
-                for (int v = 0; v < 4; v++) add4(&acc[u][4 * v], src[v * ADJ_CHUNK]);
+                for (int v = 0; v < 4; v++) add4(&acc[u][4 * v], src[v * NT]);
             }
         __syncthreads();
     }
 #pragma unroll
     for (int u = 0; u < ADJ_CELLS; u++) {
-        const int i = c0 + (int)threadIdx.x + u * ADJ_THREADS;
+        const int i = c0 + (int)threadIdx.x + u * NT;
         if (i >= c1) continue;
         const float4 l = j.ls[i];
         j.ls_acc[i] = make_float4(l.x + acc[u][0], l.y + acc[u][1], l.z + acc[u][2], l.w + acc[u][3]);
@@ -747,27 +746,29 @@ hipError_t launch_adj_force_sum(const AdjFluidArgs &j, hipStream_t s)
     return hipGetLastError();
 }
 
+template <class L, int NT, int ADJ_CELLS>
+static void launch_adj_flux_as(const FluidArgs &a, const AdjFluidArgs &j, const float4 *st, const float4 *grad, hipStream_t s)
+{
+    const size_t lds = sizeof(float4) * 8 * NT + sizeof(int) * (size_t)a.max_grad_slots;
+    hipLaunchKernelGGL((k_adj_flux<L, NT, ADJ_CELLS>), dim3(a.n_tiles), dim3(NT), lds, s, a, j, st, grad);
+}
+
 template <class L>
 static void launch_adj_flux_l(const FluidArgs &a, const AdjFluidArgs &j, const float4 *st, const float4 *grad,
-                              int cells_per_thread, size_t lds, hipStream_t s)
+                              int max_tile_cells, hipStream_t s)
 {
-    if (cells_per_thread == 1)
-        hipLaunchKernelGGL((k_adj_flux<L, 1>), dim3(a.n_tiles), dim3(ADJ_THREADS), lds, s, a, j, st, grad);
-    else if (cells_per_thread == 2)
-        hipLaunchKernelGGL((k_adj_flux<L, 2>), dim3(a.n_tiles), dim3(ADJ_THREADS), lds, s, a, j, st, grad);
-    else
-        hipLaunchKernelGGL((k_adj_flux<L, 4>), dim3(a.n_tiles), dim3(ADJ_THREADS), lds, s, a, j, st, grad);
+    if (max_tile_cells <= 256) launch_adj_flux_as<L, 256, 1>(a, j, st, grad, s);
+    else if (max_tile_cells <= 512) launch_adj_flux_as<L, 256, 2>(a, j, st, grad, s);
+    else launch_adj_flux_as<L, 512, 2>(a, j, st, grad, s);
 }
 
 hipError_t launch_adj_flux(const FluidArgs &a, const AdjFluidArgs &j, const float4 *st, const float4 *grad,
                            int max_tile_cells, hipStream_t s)
 {
-    const size_t lds = sizeof(float4) * 8 * (size_t)ADJ_CHUNK + sizeof(int) * (size_t)a.max_grad_slots;
-    const int cpt = (max_tile_cells + ADJ_THREADS - 1) / ADJ_THREADS;
     switch (a.lattice) {
-    case LBFS_D3Q15: launch_adj_flux_l<D3Q15>(a, j, st, grad, cpt, lds, s); break;
-    case LBFS_D3Q19: launch_adj_flux_l<D3Q19>(a, j, st, grad, cpt, lds, s); break;
-    case LBFS_D2Q9: launch_adj_flux_l<D2Q9>(a, j, st, grad, cpt, lds, s); break;
+    case LBFS_D3Q15: launch_adj_flux_l<D3Q15>(a, j, st, grad, max_tile_cells, s); break;
+    case LBFS_D3Q19: launch_adj_flux_l<D3Q19>(a, j, st, grad, max_tile_cells, s); break;
+    case LBFS_D2Q9: launch_adj_flux_l<D2Q9>(a, j, st, grad, max_tile_cells, s); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
