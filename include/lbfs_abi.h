@@ -392,7 +392,9 @@ int lbfs_case_read(const char *path, lbfs_case *out);
 /* ---- measurement (no counterpart in the reference; used by bench.py) ----
  * HIP events recorded on the context's stream.  lbfs_time_steps: wall time of
  * nsteps whole steps.  lbfs_time_kernels: average duration per launch of each
- * kernel of the step, names[i] / ms[i] for i < *count (at most max_count). */
+ * kernel of the step, names[i] / ms[i] for i < *count (at most max_count).  Named
+ * as the stages above, but for the launches that whole steps join: "fluid" (the
+ * fused fluid pass) and "mem_forces" (the membrane forces of small membranes). */
 int lbfs_time_steps(lbfs_ctx *ctx, int nsteps, double *ms_total);
 int lbfs_time_kernels(lbfs_ctx *ctx, int nsteps, int max_count, const char **names, double *ms, int *count);
 /* average duration of one fluid pass ("gradients" or "flux_update") over n

@@ -334,13 +334,13 @@ __global__ __launch_bounds__(NT) void k_flux_update(FluidArgs a, const float4 *_
 // not read, and written (the tile's own cells) only when a.grad_out is set.
 //
 // Bound by memory: at 256x128x128 the same loads without the face arithmetic
-// take 0.97 of its time, 333 us for the 330 B a cell it moves (4.1 TB/s; a
+// take 0.97 of its time, 335 us for the 330 B a cell it moves (4.1 TB/s; a
 // device copy on the same card 5.1).  What it reads is laid out for it: cells
 // by slots of shared patterns rather than ids (faces 40 B, no stencil), the
 // weights of a tile and its halo as whole rows, each thread's next face on its
 // way while the present one is reconstructed.  D3Q19, 8x8x8 tiles, with face
 // ids, stencil ids and gathered weights before: 128x64x64 42.9 -> 38.3 us,
-// 256x128x128 428 -> 333 us.
+// 256x128x128 428 -> 335 us.
 template <class L, bool BAND, int NT>
 __global__ __launch_bounds__(NT) void k_fluid_fused(FluidArgs a, const float4 *__restrict__ st,
                                                      float4 *__restrict__ st_out, float4 *__restrict__ res_out,
@@ -383,7 +383,8 @@ __global__ __launch_bounds__(NT) void k_fluid_fused(FluidArgs a, const float4 *_
             g[2] = o[2];
         }
     }
-    // a boundary face's neighbour slot is 0xffff: its state is the owner's, unused
+    // a boundary face's neighbour slot is 0xffff: it loads the last gradient slot's
+    // state, unused
     const int last = ns - 1;
     float4 so = st[ids[gs & 0xffffu]], sn = st[ids[min((int)(gs >> 16), last)]];
     __syncthreads();
