@@ -113,6 +113,15 @@ __device__ __forceinline__ double lagrange4(const IbmArgs &g, const IbmBlock &B,
     return v;
 }
 
+// The index of a grid coordinate.  One beyond an integer (a run that has blown up;
+// the conversion saturates) stays far enough from its ends for a stencil's
+// offsets: past the largest integer an index would wrap to one below zero, which
+// only the first of the range's two checks, done on the offset alone, refuses.
+__device__ __forceinline__ int grid_index(float v)
+{
+    return min(max((int)v, -(1 << 30)), 1 << 30);
+}
+
 __device__ __forceinline__ void node_base(const IbmArgs &g, const IbmBlock &B, const float P[3], float xr[3], int base[3])
 {
 #pragma unroll
@@ -121,7 +130,7 @@ __device__ __forceinline__ void node_base(const IbmArgs &g, const IbmBlock &B, c
         if (g.kernel == LBFS_IBM_LAGRANGE4)
             base[a] = closest_vertex(g.axis + B.ax_off[a], B.n[a] + 1, (double)P[a]) - 2;
         else
-            base[a] = g.kernel == LBFS_IBM_LINEAR2 ? (int)roundf(xr[a]) - 1 : (int)floorf(xr[a] - 1.5f);
+            base[a] = g.kernel == LBFS_IBM_LINEAR2 ? grid_index(roundf(xr[a])) - 1 : grid_index(floorf(xr[a] - 1.5f));
     }
 }
 
